@@ -235,6 +235,17 @@ __device__ __forceinline__ void s8x4_to_h(uint32_t v, uint32_t& lo, uint32_t& hi
     bytes_to_h(v ^ 0x80808080u, kHm1152, lo, hi);
 }
 
+// Four signed int8 codes -> their fp16 values / 16 (two dwords): (1024 + c +
+// 128) / 16 - 72, one rounding, exact.
+__device__ __forceinline__ void s8x4_to_h16(uint32_t v, uint32_t& lo, uint32_t& hi)
+{
+    uint32_t a, b;
+    bytes_to_h1024(v ^ 0x80808080u, a, b);
+    const h2_t sc = {(_Float16)0.0625f, (_Float16)0.0625f}, off = {(_Float16)-72.0f, (_Float16)-72.0f};
+    lo = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2_t, a), sc, off));
+    hi = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2_t, b), sc, off));
+}
+
 // NW wavefronts per workgroup share the staged activation blocks of 4 MR
 // rows and own 16 weight columns each; a chunk is CH blocks (one LDS barrier
 // per chunk), and PF chunks of weights and activation blocks are in flight.
@@ -491,6 +502,337 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same products for prompts with enough (row, column) tiles to fill the
+// chip: a wavefront owns 4 MR rows x 16 NG columns, so each activation
+// operand, accumulator start and row delta it reads from LDS serves NG
+// weight operands, and each converted weight operand MR row groups.
+//
+// What bounds it: the vector unit.  Per block a wavefront issues 9 fp32
+// operations per 64 (row, column) pairs (the reference's rounding steps, none
+// of which can go) beside 11 per weight operand; with one column group (NG =
+// 1, k_gemm_qh) the LDS reads were the limit instead: per block and row group
+// 18 LDS cycles (two 16-byte reads and a dword per lane) on a unit that four
+// SIMDs share, against 9 + 11 / MR vector operations of 4 cycles each on one.
+//
+// The weights are read in their own layout, 16 bytes per lane: lane (column,
+// g) of a 16 x 4 arrangement reads block b0 + g of its column, and a 4 x 4
+// transpose over the four 16-lane rows (two lane swaps per pair of registers)
+// hands every lane its AVX lane's codes of the four blocks; or (CL) from the
+// chunk-major copy, where they lie in that order already.
+//
+// Codes enter raw, as fp16 1024 + byte (one v_perm_b32 per two), and the
+// accumulators start at what that adds.  Q8: the byte is w + 128, so the
+// products sum to sum (1152 + w) x and the start is -1152 sum x.  Q4: the
+// low nibbles enter as 1024 + n against x, the high ones in place as 1024 +
+// 16 n against x / 16 (exact in fp16), giving (64 + n) x; the start is -1031
+// sum x over the low ones and -71 sum x over the high ones, which leaves sum
+// (n - 7) x.  Every value on the way is an integer below 2^22.
+//
+// ODT: F32 stores the dot products (out_pitch floats per row); Q8 stores them
+// as write_row_from_float does (out_pitch bytes per row), a block of 32
+// columns being two column groups of one wavefront.
+__device__ __forceinline__ void lane_rows_transpose4(uint32_t (&r)[4])
+{
+    // r[b] of lane row g <- r[g] of lane row b
+    auto swap32 = [](uint32_t& a, uint32_t& b) {
+        const auto t = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = t[0];
+        b = t[1];
+    };
+    auto swap16 = [](uint32_t& a, uint32_t& b) {
+        const auto t = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = t[0];
+        b = t[1];
+    };
+    swap32(r[0], r[2]);
+    swap32(r[1], r[3]);
+    swap16(r[0], r[1]);
+    swap16(r[2], r[3]);
+}
+
+template <int WT, int MR, int NG, int NW, bool CL, int WPE, int ODT>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) void k_gemm_qw(
+        const uint8_t* __restrict__ x, int x_pitch, int n_rows, const uint32_t* __restrict__ wq,
+        const uint16_t* __restrict__ wd, void* __restrict__ out, int out_pitch, int N, int nb)
+{
+    constexpr int WV = WT == Q4 ? 1 : 2;  // code dwords of one lane of a weight block
+    constexpr int WD = WT == Q4 ? 4 : 8;  // code dwords per weight block
+    constexpr int CH = 4;                 // blocks per chunk
+    constexpr int PF = 2;                 // chunks in flight
+    constexpr int kRows = 4 * MR, kThreads = 64 * NW;
+    static_assert(ODT != Q8 || NG % 2 == 0, "a Q8 output block is two column groups");
+    __shared__ __align__(16) uint4 xa[2][CH][MR][64];                   // expanded operands (see k_gemm_qh)
+    __shared__ __align__(16) float xd[2][CH][4][MR];                    // deltas of rows 4m + g as [g][m]
+    __shared__ __align__(16) float xc[2][CH][kRows][4];  // accumulator starts
+    static_assert(MR >= 2, "the row deltas of two blocks are held in turn");
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int lc = lane & 15, lg = lane >> 4;
+    const int r0 = blockIdx.y * kRows;
+    const int c0 = (blockIdx.x * NW + wv) * 16 * NG;
+    const int nch = nb / CH;
+
+    for (int e = tid; e < 2 * CH * MR * 64; e += kThreads)
+        if (((e & 15) & 3) != ((e >> 4) & 3)) (&xa[0][0][0][0])[e] = make_uint4(0, 0, 0, 0);
+
+    // staging tasks: one AVX lane k of one (row, block) of the chunk
+    constexpr int kTasks = 4 * kRows * CH;
+    constexpr int TPT = (kTasks + kThreads - 1) / kThreads;
+    static_assert(kThreads % 4 == 0, "a thread's tasks share their lane");
+    const uint32_t psel = tid & 1 ? 0x07060302u : 0x05040100u;  // byte pairs of lanes k odd / even
+    struct XLane {
+        uint32_t d[4];
+        uint16_t d16;
+    };
+    // 32-bit offsets from buffer resources: a chunk's position is the scalar
+    // offset, so no address is formed per load
+    const auto xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (unsigned)((size_t)n_rows * x_pitch), kBufferFlags);
+    int t_row[TPT], t_blk[TPT], t_k[TPT], t_off[TPT], t_dof[TPT];
+#pragma unroll
+    for (int i = 0; i < TPT; i++) {
+        const int t = min(tid + i * kThreads, kTasks - 1);
+        t_k[i] = t & 3;
+        t_row[i] = (t >> 2) % kRows;
+        t_blk[i] = (t >> 2) / kRows;
+        const int base = min(r0 + t_row[i], n_rows - 1) * x_pitch;
+        t_off[i] = base + t_blk[i] * 32 + (t_k[i] >> 1) * 4;
+        t_dof[i] = base + nb * 32 + t_blk[i] * 2;
+    }
+    auto x_load = [&](int ch, XLane (&q)[TPT]) {
+        const int b0 = min(ch, nch - 1) * CH;
+#pragma unroll
+        for (int i = 0; i < TPT; i++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) q[i].d[v] = __builtin_amdgcn_raw_buffer_load_b32(xres, t_off[i] + 8 * v, b0 * 32, 0);
+            q[i].d16 = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(xres, t_dof[i], b0 * 2, 0);
+        }
+    };
+    auto stage = [&](const XLane (&q)[TPT], int buf) {
+#pragma unroll
+        for (int i = 0; i < TPT; i++) {
+            if (tid + i * kThreads >= kTasks) break;  // uniform per wave: kTasks is a multiple of 64
+            const int k = t_k[i], r = t_row[i], j = t_blk[i];
+            const uint32_t a = __builtin_amdgcn_perm(q[i].d[1], q[i].d[0], psel);  // pick_pair of lane k
+            const uint32_t bq = __builtin_amdgcn_perm(q[i].d[3], q[i].d[2], psel);
+            const int sa = __builtin_amdgcn_sdot4((int)a, 0x01010101, 0, false);
+            const int sb = __builtin_amdgcn_sdot4((int)bq, 0x01010101, 0, false);
+            uint4 hv;
+            if constexpr (WT == Q4) {
+                s8x4_to_h16(a, hv.x, hv.y);
+                xc[buf][j][r][k] = (float)(-71 * sa - 1031 * sb);
+            } else {
+                s8x4_to_h(a, hv.x, hv.y);
+                xc[buf][j][r][k] = (float)(-1152 * (sa + sb));
+            }
+            s8x4_to_h(bq, hv.z, hv.w);
+            xa[buf][j][r >> 2][(r & 3) * 4 + k + 16 * k] = hv;
+            if (k == 0) xd[buf][j][r & 3][r >> 2] = h2f(q[i].d16);
+        }
+    };
+
+    // this thread's weight columns (columns past the end repeat the last)
+    const size_t wbytes = (size_t)N * nb * WD * 4;
+    const auto wres = __builtin_amdgcn_make_buffer_rsrc((void*)wq, 0, (unsigned)wbytes, kBufferFlags);
+    const auto dres = __builtin_amdgcn_make_buffer_rsrc((void*)wd, 0, (unsigned)((size_t)N * nb * 2), kBufferFlags);
+    int w_off[NG], d_off[NG];
+#pragma unroll
+    for (int n = 0; n < NG; n++) {
+        const int col = min(c0 + 16 * n + lc, N - 1);
+        w_off[n] = CL ? (col * 4 + lg) * 16 * WV : (col * nb + lg) * WD * 4;
+        d_off[n] = CL ? col * 8 : col * nb * 2;
+    }
+    typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t U2 __attribute__((ext_vector_type(2)));
+    struct WChunk {
+        uint32_t c[NG][WV][4];  // CL: block b's lane-lg codes; plain: block lg's codes, before the transpose
+        uint32_t d[NG][2];      // the four blocks' deltas
+    };
+    auto w_load = [&](int ch, WChunk& w) {
+        const int cc = min(ch, nch - 1);
+        const int ws = CL ? cc * N * 64 * WV : cc * CH * WD * 4, ds = CL ? cc * N * 8 : cc * CH * 2;
+#pragma unroll
+        for (int n = 0; n < NG; n++) {
+#pragma unroll
+            for (int q = 0; q < WV; q++) {
+                const U4 t = __builtin_amdgcn_raw_buffer_load_b128(wres, w_off[n] + 16 * q, ws, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) w.c[n][q][e] = t[e];
+            }
+            const U2 d = __builtin_amdgcn_raw_buffer_load_b64(dres, d_off[n], ds, 0);
+            w.d[n][0] = d[0];
+            w.d[n][1] = d[1];
+        }
+    };
+    // one lane's code dwords of block b, after the transpose (plain) or as
+    // the copy has them
+    auto w_order = [&](WChunk& w) {
+        if constexpr (CL) {
+            if constexpr (WV == 2)
+#pragma unroll
+                for (int n = 0; n < NG; n++) {
+                    // [block][2 dwords] in order -> [dword][block]
+                    uint32_t a[8];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) a[e] = w.c[n][e >> 2][e & 3];
+#pragma unroll
+                    for (int b = 0; b < 4; b++) {
+                        w.c[n][0][b] = a[2 * b];
+                        w.c[n][1][b] = a[2 * b + 1];
+                    }
+                }
+        } else {
+#pragma unroll
+            for (int n = 0; n < NG; n++) {
+                if constexpr (WV == 1) {
+                    lane_rows_transpose4(w.c[n][0]);
+                } else {
+                    // dwords 2k, 2k + 1 of a block belong to lane k
+                    uint32_t lo[4] = {w.c[n][0][0], w.c[n][0][2], w.c[n][1][0], w.c[n][1][2]};
+                    uint32_t hi[4] = {w.c[n][0][1], w.c[n][0][3], w.c[n][1][1], w.c[n][1][3]};
+                    lane_rows_transpose4(lo);
+                    lane_rows_transpose4(hi);
+#pragma unroll
+                    for (int b = 0; b < 4; b++) {
+                        w.c[n][0][b] = lo[b];
+                        w.c[n][1][b] = hi[b];
+                    }
+                }
+            }
+        }
+    };
+    auto b_operand = [&](const WChunk& w, int n, int j, h8_t& Bh, float& dw) {
+        uint4 B;
+        if constexpr (WT == Q4) {
+            // high nibbles in place: 1024 + 16 n
+            const uint32_t P = w.c[n][0][j];
+            bytes_to_h1024(P & 0xF0F0F0F0u, B.x, B.y);
+            bytes_to_h1024(P & 0x0F0F0F0Fu, B.z, B.w);
+        } else {
+            bytes_to_h1024(w.c[n][0][j] ^ 0x80808080u, B.x, B.y);
+            bytes_to_h1024(w.c[n][WV - 1][j] ^ 0x80808080u, B.z, B.w);
+        }
+        Bh = __builtin_bit_cast(h8_t, B);
+        dw = h2f((uint16_t)(w.d[n][j >> 1] >> (16 * (j & 1))));
+    };
+
+    float acc[MR][NG][4];
+#pragma unroll
+    for (int m = 0; m < MR; m++)
+#pragma unroll
+        for (int n = 0; n < NG; n++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) acc[m][n][k] = 0.0f;
+
+    // weights and activation blocks in a ring of PF chunks, as k_gemm_qh
+    WChunk wr[PF];
+    XLane xq[PF][TPT];
+#pragma unroll
+    for (int p = 0; p < PF; p++) {
+        w_load(p, wr[p]);
+        x_load(p, xq[p]);
+    }
+    stage(xq[0], 0);
+    lds_barrier();
+    auto chunk = [&](int ch, auto pc) {
+            constexpr int p = decltype(pc)::value, buf = p;
+            w_order(wr[p]);
+            // steps s = (block j, row group m) in turn: step s's products are
+            // issued, then step s - 1's are folded, with step s + 1's LDS
+            // reads in flight; the fences keep that order (and the registers
+            // a deeper interleaving would take)
+            auto a_read = [&](int s, uint4& A, f4_t& ci) {
+                A = xa[buf][s / MR][s % MR][lane];
+                ci = *reinterpret_cast<const f4_t*>(&xc[buf][s / MR][4 * (s % MR) + lg][0]);
+            };
+            uint4 A[2];
+            f4_t ci[2], L[2][NG];
+            h8_t Bh[NG];
+            float dw[2][NG], dx[2][MR];
+            a_read(0, A[0], ci[0]);
+#pragma unroll
+            for (int m = 0; m < MR; m++) dx[0][m] = xd[buf][0][lg][m];
+            auto fold = [&](int s) {
+                const int j = s / MR, m = s % MR;
+#pragma unroll
+                for (int n = 0; n < NG; n++) {
+                    const float dd = dx[j & 1][m] * dw[j & 1][n];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        acc[m][n][k] = acc[m][n][k] + L[s & 1][n][k] * dd;
+                        asm volatile("" : "+v"(acc[m][n][k]));  // the add stays in this step
+                    }
+                }
+            };
+#pragma unroll
+            for (int s = 0; s < CH * MR; s++) {
+                const int j = s / MR, m = s % MR;
+                if (m == 0) {
+#pragma unroll
+                    for (int n = 0; n < NG; n++) {
+#pragma unroll
+                        for (int q = 0; q < WV; q++) asm volatile("" : "+v"(wr[p].c[n][q][j]));  // convert here, not earlier
+                        b_operand(wr[p], n, j, Bh[n], dw[j & 1][n]);
+                    }
+                }
+                if (s + 1 < CH * MR) a_read(s + 1, A[(s + 1) & 1], ci[(s + 1) & 1]);
+                if (m == MR - 1 && j + 1 < CH) {
+#pragma unroll
+                    for (int mm = 0; mm < MR; mm++) dx[(j + 1) & 1][mm] = xd[buf][j + 1][lg][mm];
+                }
+#pragma unroll
+                for (int n = 0; n < NG; n++)
+                    L[s & 1][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, A[s & 1]), Bh[n],
+                                                                        ci[s & 1], 0, 0, 0);
+                if (s > 0) fold(s - 1);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            fold(CH * MR - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            w_load(ch + PF, wr[p]);
+            x_load(ch + PF, xq[p]);
+            stage(xq[p ^ 1], buf ^ 1);  // past the end: the last chunk again, never read
+            lds_barrier();
+    };
+    int ch = 0;
+    for (; ch + 1 < nch; ch += 2) {
+        chunk(ch, std::integral_constant<int, 0>{});
+        chunk(ch + 1, std::integral_constant<int, 1>{});
+    }
+    if (ch < nch) chunk(ch, std::integral_constant<int, 0>{});
+#pragma unroll
+    for (int m = 0; m < MR; m++) {
+        const int row = r0 + 4 * m + lg;
+        const bool row_ok = row < n_rows;
+        float v[NG];
+#pragma unroll
+        for (int n = 0; n < NG; n++) v[n] = (acc[m][n][0] + acc[m][n][1]) + (acc[m][n][2] + acc[m][n][3]);
+        if constexpr (ODT == F32) {
+            float* o = reinterpret_cast<float*>(out) + (size_t)row * out_pitch;
+#pragma unroll
+            for (int n = 0; n < NG; n++)
+                if (row_ok && c0 + 16 * n + lc < N) o[c0 + 16 * n + lc] = v[n];
+        } else {
+            uint8_t* o = reinterpret_cast<uint8_t*>(out) + (size_t)row * out_pitch;
+#pragma unroll
+            for (int n = 0; n < NG; n += 2) {
+                // q8_quant_lane over the block's 16 lanes x 2 columns
+                const int ca = c0 + 16 * n + lc, cb2 = ca + 16;
+                float a = fmaxf(ca < N ? fabsf(v[n]) : 0.0f, cb2 < N ? fabsf(v[n + 1]) : 0.0f);
+                a = quad_max(a);
+                a = fmaxf(a, dpp_f<0x141>(a));  // row_half_mirror
+                a = fmaxf(a, dpp_f<0x140>(a));  // row_mirror
+                const float delta = a / 127.0f;
+                const float scale = delta != 0.0f ? 1.0f / delta : 0.0f;
+                if (row_ok && ca < N) o[ca] = (uint8_t)(int8_t)roundf(v[n] * scale);
+                if (row_ok && cb2 < N) o[cb2] = (uint8_t)(int8_t)roundf(v[n + 1] * scale);
+                if (row_ok && lc == 0 && ca < N)
+                    reinterpret_cast<uint16_t*>(o + act_delta_offset(N))[ca >> 5] = f2h(delta);
+            }
+        }
+    }
+}
+
 // The chunk-major copy of a Q4 / Q8 weight [N, K] (K % 128 == 0) that the
 // prefill matmul reads: codes [K/128][N][4 lanes][4 blocks][WV dwords] --
 // for each group of four blocks, each row's lane-k code dwords of the four
@@ -560,8 +902,92 @@ int chunk_layout_launch(const nc_tensor* w, void* codes, void* deltas, hipStream
 // load per thread and chunk; at 512 rows the staging was the largest part
 // (28%) while one wavefront of four did it, so every thread now stages one
 // AVX lane of one (row, block).
-constexpr int kGemmWideRows = 256;
+// k_gemm_qw (MR, NG, NW) against k_gemm_qh, the same cold-cache timing (us
+// over the chunk-major copy / the weight's own layout; Q4, Q8 in brackets):
+//   512 rows x 11520 x 2304:  (4, 2, 4) 175 / 193 [199 / 210], k_gemm_qh 258
+//       / (k_gemm_q) 312 [305 / 310]; 6912 x 2304: 103 / 111 [115 / 124]
+//       against 152 / 214 [182 / 212]; 2304 x 5760: 106 / 115 [112 / 123]
+//       against 134 / 195 [161 / 194]
+//   201 rows x 5632 x 2048:  42 / 47 [47 / 54] against 55 / 77 [63 / 75]
+//   128 rows x 6144 x 2048:  (2, 2, 4) 30, (4, 2, 4) 32 / 36 [36 / 38]
+//       against 39 / 51 [42 / 50]
+//   201 rows x 2048 x 5632 (208 and 416 workgroups of 16 and 8 rows):
+//       (2, 2, 4) 53 / 60 [61 / 71], (4, 2, 4) 61 / 64 [67 / 72], k_gemm_qh
+//       66 / 76 [65 / 79]
+//   64 rows x 2048 x 5632 (64 and 128 workgroups): (2, 2, 4) 43 / 44,
+//       k_gemm_qh 28 / 41: too few workgroups, every one a serial chain over
+//       the blocks, so the smaller tiles win.
+// At 512 x 11520 x 2304 the (4, 2, 4) launch issues a vector instruction in
+// 87% of the SIMDs' slots (counters); holding LDS operands two steps ahead
+// or taking the d_x d_w products from the matrix cores changed nothing.
+//
+// The rule follows the workgroups a shape would have: 16 rows per workgroup
+// from kWide16 of them (Q8's weight operands cost more to form, so it shares
+// them over 16 rows earlier), else 8 rows from kWide8, else k_gemm_qh.
+template <int WT>
+constexpr int kWide16 = WT == Q4 ? 448 : 320;
+constexpr int kWide8 = 256;
+
+static int wide_groups(int N, int n_rows, int rows) { return ((N + 127) / 128) * ((n_rows + rows - 1) / rows); }
+
+// Rows per workgroup of k_gemm_qw for this product, 0 when it is not taken:
+// its chunks are four blocks, its loads 16 (codes) and 8 (deltas) bytes, and
+// its offsets 32 bits.
+static int gemm_wide_rows(int x_pitch, int n_rows, const nc_tensor* w)
+{
+    const int N = w->rows, nb = w->cols / 32;
+    const size_t lim = (size_t)1 << 31;
+    if (w->cols % 128 || ((uintptr_t)w->data & 15) || ((uintptr_t)w->deltas & 7)) return 0;
+    if ((size_t)N * nb * (w->dtype == NC_Q4 ? 16 : 32) >= lim || (size_t)n_rows * x_pitch >= lim) return 0;
+    if (wide_groups(N, n_rows, 16) >= (w->dtype == NC_Q4 ? kWide16<Q4> : kWide16<Q8>)) return 16;
+    return wide_groups(N, n_rows, 8) >= kWide8 ? 8 : 0;
+}
+
+template <int ODT>
+static int gemm_wide(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, bool cl, int rows, void* out,
+                     int out_pitch, hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop)
+{
+    const int N = w->rows, nb = w->cols / 32;
+    auto go = [&](auto kern) {
+        const dim3 grid((N + 127) / 128, (n_rows + rows - 1) / rows);
+        if (ev_start)
+            hipExtLaunchKernelGGL(kern, grid, dim3(256), 0, st, ev_start, ev_stop, 0, x, x_pitch, n_rows,
+                                  (const uint32_t*)w->data, (const uint16_t*)w->deltas, out, out_pitch, N, nb);
+        else
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x, x_pitch, n_rows, (const uint32_t*)w->data,
+                               (const uint16_t*)w->deltas, out, out_pitch, N, nb);
+    };
+    auto by_layout = [&](auto wt, auto c) {
+        constexpr int WT = decltype(wt)::value;
+        constexpr bool CL = decltype(c)::value;
+        if (rows == 16) go(k_gemm_qw<WT, 4, 2, 4, CL, 3, ODT>);
+        else go(k_gemm_qw<WT, 2, 2, 4, CL, 4, ODT>);
+    };
+    auto by_type = [&](auto wt) {
+        if (cl) by_layout(wt, std::true_type{});
+        else by_layout(wt, std::false_type{});
+    };
+    if (w->dtype == NC_Q4) by_type(std::integral_constant<int, Q4>{});
+    else by_type(std::integral_constant<int, Q8>{});
+    return launch_status("k_gemm_qw");
+}
+
+bool gemm_q_act_supported(int x_pitch, int n_rows, const nc_tensor* w)
+{
+    return (w->dtype == NC_Q4 || w->dtype == NC_Q8) && n_rows >= kGemmMinRows && gemm_wide_rows(x_pitch, n_rows, w) != 0;
+}
+
+int gemm_q_act(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, uint8_t* out, int out_pitch,
+               hipStream_t st)
+{
+    if (!gemm_q_act_supported(x_pitch, n_rows, w))
+        return fail(NC_ERR_ARG, "gemm to Q8 rows: [%d x %d] weights, %d rows", w->rows, w->cols, n_rows);
+    return gemm_wide<Q8>(x, x_pitch, n_rows, w, false, gemm_wide_rows(x_pitch, n_rows, w), out, out_pitch, st, nullptr,
+                         nullptr);
+}
+
 constexpr int kGemmTallCols = 8192;
+constexpr int kGemmWideRows = 256;
 constexpr int kGemmShortRows = 80;  // prompts up to this many rows take the short-prompt shapes
 
 int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, float* out, int out_pitch,
@@ -571,6 +997,11 @@ int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, fl
     if (w->cols % 32 || w->cols <= 0 || w->rows <= 0 || n_rows <= 0)
         return fail(NC_ERR_ARG, "gemm: [%d x %d] weights, %d rows", w->rows, w->cols, n_rows);
     const int N = w->rows, nb = w->cols / 32;
+    if (wc && (wc->dtype != w->dtype || wc->rows != N || wc->cols != w->cols || !chunk_layout_supported(wc)))
+        return fail(NC_ERR_ARG, "gemm: chunk copy [%d x %d] of a [%d x %d] weight", wc->rows, wc->cols, N, w->cols);
+    if (const int rows = gemm_wide_rows(x_pitch, n_rows, wc ? wc : w))
+        return gemm_wide<F32>(x, x_pitch, n_rows, wc ? wc : w, wc != nullptr, rows, out, out_pitch, st, ev_start,
+                              ev_stop);
     auto go = [&](auto kern, int mr, int ng, int nw, const nc_tensor* wt = nullptr) {
         if (!wt) wt = w;
         const dim3 grid((N + 16 * ng * nw - 1) / (16 * ng * nw), (n_rows + 4 * mr - 1) / (4 * mr));
@@ -583,21 +1014,15 @@ int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, fl
     };
     const bool wide = n_rows >= kGemmWideRows, tall = N >= kGemmTallCols;
     // the chunk-major copy, when the caller has one (shapes measured with
-    // cold caches, as a prefill meets its weights)
+    // cold caches, as a prefill meets its weights): few tiles, or a product
+    // past k_gemm_qw's offsets
     if (wc) {
-        if (wc->dtype != w->dtype || wc->rows != N || wc->cols != w->cols || !chunk_layout_supported(wc))
-            return fail(NC_ERR_ARG, "gemm: chunk copy [%d x %d] of a [%d x %d] weight", wc->rows, wc->cols, N, w->cols);
         auto goc = [&](auto kern, int mr, int nw) { go(kern, mr, 1, nw, wc); };
         auto by_type_c = [&](auto wt) {
             constexpr int WT = decltype(wt)::value;
             // chunks of 8 blocks need nb % 8 == 0 (the copy itself is in
-            // 4-block chunks).  Long Q4 prompts: 8 rows per workgroup, one
-            // chunk in flight, five wavefronts per SIMD (84 VGPRs); medium
-            // ones (81-255 rows): 8 rows, two chunks in flight, four
-            // wavefronts (120 VGPRs).
-            if (wide && WT == Q4) goc(k_gemm_qh<WT, 2, 4, 4, 1, true, 5>, 2, 4);
-            else if (n_rows > kGemmShortRows && WT == Q4) goc(k_gemm_qh<WT, 2, 4, 4, 2, true, 4>, 2, 4);
-            else if (wide || tall || n_rows > kGemmShortRows || nb % 8)
+            // 4-block chunks)
+            if (tall || n_rows > kGemmShortRows || nb % 8)
                 goc(k_gemm_qh<WT, 4, 4, 4, 2, true, WT == Q4 ? 3 : 1>, 4, 4);
             else goc(k_gemm_qh<WT, 2, 4, 8, 2, true>, 2, 4);
         };
@@ -612,8 +1037,7 @@ int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, fl
     auto goh = [&](auto kern, int mr, int nw) { go(kern, mr, 1, nw); };
     auto by_type = [&](auto wt) {
         constexpr int WT = decltype(wt)::value;
-        if (wide && tall) go(k_gemm_q<WT, 2, 2, 8, 3>, 8, 2, 2);
-        else if (qh4 && (wide || tall || n_rows > kGemmShortRows || !qh8)) goh(k_gemm_qh<WT, 4, 4, 4, 2, false>, 4, 4);
+        if (qh4 && (wide || tall || n_rows > kGemmShortRows || !qh8)) goh(k_gemm_qh<WT, 4, 4, 4, 2, false>, 4, 4);
         else if (qh8 && n_rows <= 16) goh(k_gemm_qh<WT, 2, 2, 8, 3, false>, 2, 2);
         else if (qh8 && (N <= 2048 || nb >= 128)) goh(k_gemm_qh<WT, 2, 4, 8, 2, false>, 2, 4);
         else if (qh8) goh(k_gemm_qh<WT, 4, 4, 4, 2, false>, 4, 4);

@@ -46,6 +46,12 @@ int dmv_f16_nrm_launch(int kind, const uint8_t* a, int a_pitch, const float* bra
 int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, float* out, int out_pitch,
                hipStream_t st, hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr,
                const nc_tensor* wc = nullptr);
+// The same product stored as Q8 activation rows (write_row_from_float of the
+// dots) by the launch itself; for the products whose launch can
+// (gemm_q_act_supported).
+bool gemm_q_act_supported(int x_pitch, int n_rows, const nc_tensor* w);
+int gemm_q_act(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, uint8_t* out, int out_pitch,
+               hipStream_t st);
 // The chunk-major copy of a Q4 / Q8 weight with K % 128 == 0 (codes and
 // deltas the same sizes as the weight's own) that gemm_q_raw reads.
 bool chunk_layout_supported(const nc_tensor* w);

@@ -900,58 +900,75 @@ int noalloc_scratch_setup(int dev)
 
 }  // namespace nc
 
+namespace {
+
+bool overlap(const void* a, size_t na, const void* b, size_t nb)
+{
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a && b && x < y + nb && y < x + na;
+}
+
+// Whether the launch that computes x [rows] times w can store out's
+// activation rows itself: the rules of gemm_q_act, and no output byte that
+// the product still reads (a staged product has read everything before it
+// writes).
+bool stores_rows(const nc_tensor* x, const uint8_t* xr, const nc_tensor* w, const nc_tensor* out, const uint8_t* orow,
+                 int rows)
+{
+    if (out->dtype != NC_Q8 || x->dtype != NC_Q8 || x->cols <= 0 || !gemm_q_act_supported(x->pitch, rows, w)) return false;
+    const size_t on = (size_t)rows * out->pitch;
+    size_t cb, db;
+    if (nc_weight_bytes(w->dtype, w->rows, w->cols, &cb, &db)) return false;
+    return !overlap(orow, on, xr, (size_t)rows * x->pitch) && !overlap(orow, on, w->data, cb) &&
+           !overlap(orow, on, w->deltas, db);
+}
+
+// nc_matmul_2d with the staging of an activation-dtype output given by
+// stage(bytes, &ptr).
+template <class Stage>
+int matmul_2d(const char* name, const nc_tensor* x, const nc_tensor* w, nc_tensor* out, int start, int n_ctx,
+              void* stream, Stage&& stage)
+{
+    NC_CHECK_ARG(x && w && out && x->data && w->data && out->data, "%s: null tensor", name);
+    NC_CHECK_ARG(x->cols == w->cols, "%s: x has %d columns, w has %d", name, x->cols, w->cols);
+    NC_CHECK_ARG(out->cols == w->rows, "%s: out has %d columns, w has %d rows", name, out->cols, w->rows);
+    NC_CHECK_ARG(start >= 0 && start <= n_ctx && n_ctx <= x->rows && n_ctx <= out->rows, "%s: rows [%d, %d)", name,
+                 start, n_ctx);
+    const int rows = n_ctx - start;
+    if (rows == 0) return NC_OK;
+    hipStream_t st = stream_of(stream);
+    const uint8_t* xr = (const uint8_t*)x->data + (size_t)start * x->pitch;
+    uint8_t* orow = (uint8_t*)out->data + (size_t)start * out->pitch;
+    if (out->dtype == NC_F32) {
+        NC_CHECK_ARG(out->pitch % 4 == 0, "%s: fp32 pitch %d", name, out->pitch);
+        return matvec_raw(xr, x->dtype, x->pitch, rows, w, (float*)orow, out->pitch / 4, st);
+    }
+    float* sp = nullptr;
+    int s = stage((size_t)rows * w->rows * 4, rows, &sp);
+    if (s) return s;
+    if (stores_rows(x, xr, w, out, orow, rows)) return gemm_q_act(xr, x->pitch, rows, w, orow, out->pitch, st);
+    if ((s = matvec_raw(xr, x->dtype, x->pitch, rows, w, sp, w->rows, st))) return s;
+    return write_rows(sp, w->rows, orow, out->pitch, out->dtype, w->rows, rows, st);
+}
+
+}  // namespace
+
 // The same as nc_matmul_2d, with an activation-dtype output staged in the
 // device's fixed array instead of library-allocated memory: no allocation
 // anywhere on this path.
 extern "C" int nc_matmul_2d_noalloc(const nc_tensor* x, const nc_tensor* w, nc_tensor* out, int start, int n_ctx,
                                     void* stream)
 {
-    NC_CHECK_ARG(x && w && out && x->data && w->data && out->data, "matmul_2d_noalloc: null tensor");
-    NC_CHECK_ARG(x->cols == w->cols, "matmul_2d_noalloc: x has %d columns, w has %d", x->cols, w->cols);
-    NC_CHECK_ARG(out->cols == w->rows, "matmul_2d_noalloc: out has %d columns, w has %d rows", out->cols, w->rows);
-    NC_CHECK_ARG(start >= 0 && start <= n_ctx && n_ctx <= x->rows && n_ctx <= out->rows,
-                 "matmul_2d_noalloc: rows [%d, %d)", start, n_ctx);
-    const int rows = n_ctx - start;
-    if (rows == 0) return NC_OK;
-    hipStream_t st = stream_of(stream);
-    const uint8_t* xr = (const uint8_t*)x->data + (size_t)start * x->pitch;
-    if (out->dtype == NC_F32) {
-        NC_CHECK_ARG(out->pitch % 4 == 0, "matmul_2d_noalloc: fp32 pitch %d", out->pitch);
-        return matvec_raw(xr, x->dtype, x->pitch, rows, w, (float*)((uint8_t*)out->data + (size_t)start * out->pitch),
-                          out->pitch / 4, st);
-    }
-    const size_t need = (size_t)rows * w->rows * 4;
-    NC_CHECK_ARG(need <= kNoAllocStageBytes,
-                 "matmul_2d_noalloc: %d rows x %d outputs need %zu staging bytes, more than the %zu-byte array", rows,
-                 w->rows, need, kNoAllocStageBytes);
-    float* stage = nullptr;
-    int s = scratch_for_current(&stage);
-    if (s) return s;
-    if ((s = matvec_raw(xr, x->dtype, x->pitch, rows, w, stage, w->rows, st))) return s;
-    return write_rows(stage, w->rows, (uint8_t*)out->data + (size_t)start * out->pitch, out->pitch, out->dtype, w->rows,
-                      rows, st);
+    return matmul_2d("matmul_2d_noalloc", x, w, out, start, n_ctx, stream, [&](size_t need, int rows, float** p) {
+        NC_CHECK_ARG(need <= kNoAllocStageBytes,
+                     "matmul_2d_noalloc: %d rows x %d outputs need %zu staging bytes, more than the %zu-byte array",
+                     rows, w->rows, need, kNoAllocStageBytes);
+        return scratch_for_current(p);
+    });
 }
 
 extern "C" int nc_matmul_2d(const nc_tensor* x, const nc_tensor* w, nc_tensor* out, int start, int n_ctx, void* stream)
 {
-    NC_CHECK_ARG(x && w && out && x->data && w->data && out->data, "matmul_2d: null tensor");
-    NC_CHECK_ARG(x->cols == w->cols, "matmul_2d: x has %d columns, w has %d", x->cols, w->cols);
-    NC_CHECK_ARG(out->cols == w->rows, "matmul_2d: out has %d columns, w has %d rows", out->cols, w->rows);
-    NC_CHECK_ARG(start >= 0 && start <= n_ctx && n_ctx <= x->rows && n_ctx <= out->rows, "matmul_2d: rows [%d, %d)",
-                 start, n_ctx);
-    const int rows = n_ctx - start;
-    if (rows == 0) return NC_OK;
-    hipStream_t st = stream_of(stream);
-    const uint8_t* xr = (const uint8_t*)x->data + (size_t)start * x->pitch;
-    if (out->dtype == NC_F32) {
-        NC_CHECK_ARG(out->pitch % 4 == 0, "matmul_2d: fp32 pitch %d", out->pitch);
-        return matvec_raw(xr, x->dtype, x->pitch, rows, w, (float*)((uint8_t*)out->data + (size_t)start * out->pitch),
-                          out->pitch / 4, st);
-    }
-    float* stage;
-    int s = stage_buffer((size_t)rows * w->rows * 4, &stage);
-    if (s) return s;
-    if ((s = matvec_raw(xr, x->dtype, x->pitch, rows, w, stage, w->rows, st))) return s;
-    return write_rows(stage, w->rows, (uint8_t*)out->data + (size_t)start * out->pitch, out->pitch, out->dtype, w->rows,
-                      rows, st);
+    return matmul_2d("matmul_2d", x, w, out, start, n_ctx, stream,
+                     [&](size_t need, int, float** p) { return stage_buffer(need, p); });
 }

@@ -113,6 +113,46 @@ def test_matmul_act_out(gpu, oracle, xdt, wdt, K, N):
     assert_same(out.ref(), want, "matmul act out")
 
 
+WIDE_CASES = [
+    # (w dtype, K, N, rows, start): the prefill matmul's launches that share
+    # activation operands over 32 columns, 16 rows per workgroup (Q4 from 448
+    # workgroups, Q8 from 320) and 8 (from 256): one, an odd and an even number
+    # of four-block chunks, rows and columns past a tile, a partial last block
+    (Q4, 128, 1010, 903, 3),
+    (Q4, 384, 4100, 225, 0),
+    (Q8, 640, 2050, 310, 0),
+    (Q4, 256, 1010, 260, 0),
+    (Q8, 384, 3000, 85, 0),
+]
+
+
+@pytest.mark.parametrize("wdt,K,N,rows,start", WIDE_CASES)
+@pytest.mark.parametrize("odt", [F32, Q8])
+def test_matmul_wide(gpu, oracle, wdt, K, N, rows, start, odt):
+    rng = np.random.default_rng(K + N)
+    x = rand_act(oracle, rng, Q8, rows, K)
+    w = rand_weight(oracle, rng, wdt, N, K)
+    want = np.zeros((rows, N), np.float32) if odt == F32 else np.zeros((rows, OL.row_bytes(Q8, N)), np.uint8)
+    oracle.matmul(OL.ptr(x), Q8, OL.ptr(w), wdt, OL.ptr(want), odt, K, N, start, rows, None)
+    dx, dw, out = DevAct(x, Q8, rows, K), DevWeight(w, wdt, N, K), DevAct.empty(odt, rows, N)
+    gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), start, rows, None), "matmul")
+    got = out.ref() if odt == Q8 else out.ref().view(np.float32)
+    assert_same(got[start:], want[start:], f"matmul Q{8 if wdt == Q8 else 4} K={K} N={N} out {odt}")
+
+
+def test_matmul_in_place(gpu, oracle):
+    """Output rows over the input rows: the product is read whole first."""
+    rng = np.random.default_rng(17)
+    d, rows = 1024, 900
+    x = rand_act(oracle, rng, Q8, rows, d)
+    w = rand_weight(oracle, rng, Q4, d, d)
+    want = np.zeros((rows, OL.row_bytes(Q8, d)), np.uint8)
+    oracle.matmul(OL.ptr(x), Q8, OL.ptr(w), Q4, OL.ptr(want), Q8, d, d, 0, rows, None)
+    dx, dw = DevAct(x, Q8, rows, d), DevWeight(w, Q4, d, d)
+    gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(dx.t), 0, rows, None), "matmul")
+    assert_same(dx.ref(), want, "matmul in place")
+
+
 @pytest.mark.parametrize("dt", [Q8, F16])
 @pytest.mark.parametrize("d,scale", [(2048, 1.0), (2304, 30.0), (256, 0.01)])
 def test_rms_norm(gpu, oracle, dt, d, scale):
