@@ -22,10 +22,11 @@
 // Weights are held in registers across activation rows, so prefill reads
 // every weight once per launch.
 //
-// F16 kernel: thread = (row, lane j); each thread reads 16-byte runs of its
-// own lane (the weight layout interleaves 64-column groups over 8-row
-// groups, so a wavefront reads 1 KiB contiguous) and folds its chain in
-// order; the eight lanes of a row meet through wavefront shuffles.
+// F16 kernels: several rows on the matrix cores (k_mfma_f16); one row with
+// thread = (row, lane j): each thread reads 16-byte runs of its own lane (the
+// weight layout interleaves 64-column groups over 8-row groups, so a
+// wavefront reads 1 KiB contiguous) and folds its chain in order; the eight
+// lanes of a row meet through wavefront shuffles.
 #include <hip/hip_ext.h>
 
 #include <type_traits>
@@ -102,257 +103,191 @@ __global__ __launch_bounds__(kMvThreads) void k_matvec_q(const uint8_t* __restri
     }
 }
 
-// F16: 8 rows x 8 lanes per wavefront, 32 rows per workgroup.
-__global__ __launch_bounds__(kMvThreads) void k_matvec_f16(const uint8_t* __restrict__ x, int x_pitch, int n_xrows,
-                                                          const uint16_t* __restrict__ w, float* __restrict__ out,
-                                                          int out_pitch, int N, int K)
+// F16, prefill, on the matrix cores.  v_mfma_f32_16x16x1_4b_f32 multiplies
+// four independent pairs of 16-vectors (one K step each) and adds them to
+// four 16 x 16 fp32 accumulators: one fused multiply-add per entry, which on
+// exact fp16 products is the reference's multiply then add.  So its four
+// blocks hold four lane chains j of a 16 x 16 tile (rows of x times rows of
+// w), two of them (j = 0..3, 4..7) all eight, and the K steps m of the
+// 64-column groups run in the reference's order; the eight chains of an
+// output end up in one thread, which sums them left to right.
+//
+// What bounds it: the matrix cores' fp32 rate, 128 multiply-adds per clock
+// and CU (134 TFLOP/s measured with nothing else in the loop), twice the
+// vector unit's without packed math; for few tiles, the chain of K steps one
+// wavefront runs (32 cycles each and half).  x is staged widened to fp32 in
+// the operand order [group][lane j][m / 4][row]; the weights come straight
+// from their layout, one 16-byte load per lane giving eight K steps, and are
+// widened beside the products.
+// Measured (us, cold caches; before: register-tiled vector kernel):
+//   1500 rows x 2048 x 2048     259 -> 134 (94 TFLOP/s)
+//   128 rows x 11264 x 2048     126 -> 67, 5632 x 2048 72 -> 39
+//   64 rows x 2560 x 2048       32 -> 17, 2048 x 5632 73 -> 39
+//   2 rows x 5632 x 2048        21 -> 16 (before: one row at a time)
+//
+// RN row tiles and CN column tiles of 16 per wavefront (four wavefronts side
+// by side in columns); GC groups staged at a time, PF (GC or GC / 2) groups
+// of weights in flight; ODT F32 or F16 rows out (out_pitch in floats or
+// bytes).
+typedef float f16x_t __attribute__((ext_vector_type(16)));
+
+template <int RN, int CN, int GC, int PF, int ODT>
+__global__ __launch_bounds__(256) void k_mfma_f16(const uint8_t* __restrict__ x, int x_pitch, int n_rows,
+                                                  const uint16_t* __restrict__ w, void* __restrict__ out, int out_pitch,
+                                                  int N, int K)
 {
-    extern __shared__ __align__(16) float xsf[];  // [K/64][8 lanes][8]
-    const int tid = threadIdx.x;
-    const int j = tid & 7;
-    const int row = blockIdx.x * 32 + (tid >> 3);
-    const int G = K / 64;
-    const int npad = (N + 7) & ~7;
-    const uint4* wrow = reinterpret_cast<const uint4*>(w) + (size_t)row * 8 + j;  // group 0
-    const size_t gstride = (size_t)npad * 8;                                        // uint4s per group
-
-    for (int p = 0; p < n_xrows; p++) {
-        const uint16_t* xr = reinterpret_cast<const uint16_t*>(x + (size_t)p * x_pitch);
-        for (int e = tid; e < K; e += kMvThreads) {
-            const int g = e >> 6, m = (e >> 3) & 7, jj = e & 7;
-            xsf[(g * 8 + jj) * 8 + m] = h2f(xr[e]);
-        }
-        __syncthreads();
-        float acc = 0.0f;
-        if (row < N) {
-            for (int g = 0; g < G; g++) {
-                const uint4 u = wrow[(size_t)g * gstride];
-                const float4 xa = *reinterpret_cast<const float4*>(xsf + (g * 8 + j) * 8);
-                const float4 xb = *reinterpret_cast<const float4*>(xsf + (g * 8 + j) * 8 + 4);
-                const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
-                const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-                for (int m = 0; m < 8; m++) {
-                    const uint16_t h = (uint16_t)(m & 1 ? wv[m >> 1] >> 16 : wv[m >> 1] & 0xFFFFu);
-                    acc = __builtin_fmaf(xv[m], h2f(h), acc);  // exact product: same as mul then add
-                }
-            }
-        }
-        const int base = tid & ~7;
-        float s = __shfl(acc, base);
-#pragma unroll
-        for (int l = 1; l < 8; l++) s = s + __shfl(acc, base + l);
-        if (j == 0 && row < N) out[(size_t)p * out_pitch + row] = s;
-        __syncthreads();
-    }
-}
-
-// F16, many activation rows (prefill): a 256-thread workgroup owns 32
-// weight rows (thread (row, lane j) as in k_matvec_f16) and runs the
-// activation rows kF16TileRows at a time, so each weight is read once per
-// tile instead of once per row.  Every (activation row, weight row, lane)
-// chain folds its lane's products over the 64-column groups in order, as the
-// reference's 8-lane fp32 dot does; the activation tile is staged in LDS
-// kF16TileGroups groups at a time.
-constexpr int kF16TileRows = 16;
-constexpr int kF16TileGroups = 8;  // 512 columns per stage
-
-__global__ __launch_bounds__(kMvThreads) void k_matvec_f16_tile(const uint8_t* __restrict__ x, int x_pitch,
-                                                               int n_xrows, const uint16_t* __restrict__ w,
-                                                               float* __restrict__ out, int out_pitch, int N, int K)
-{
-    // xs[p][gl][j][m] = x[p0 + p][64 (g0 + gl) + 8 m + j]
-    __shared__ __align__(16) float xs[kF16TileRows][kF16TileGroups][8][8];
-    const int tid = threadIdx.x;
-    const int j = tid & 7;
-    const int row = blockIdx.x * 32 + (tid >> 3);
-    const int G = K / 64;
-    const int npad = (N + 7) & ~7;
-    const int rowc = row < N ? row : N - 1;  // rows past N read a valid row and store nothing
-    const uint4* wrow = reinterpret_cast<const uint4*>(w) + (size_t)rowc * 8 + j;  // group 0
-    const size_t gstride = (size_t)npad * 8;                                         // uint4s per group
-
-    for (int p0 = 0; p0 < n_xrows; p0 += kF16TileRows) {
-        const int np = min(kF16TileRows, n_xrows - p0);
-        float acc[kF16TileRows];
-#pragma unroll
-        for (int p = 0; p < kF16TileRows; p++) acc[p] = 0.0f;
-        for (int g0 = 0; g0 < G; g0 += kF16TileGroups) {
-            const int ng = min(kF16TileGroups, G - g0);
-            // this stage's weights first, then the activation tile
-            uint4 wv4[kF16TileGroups];
-#pragma unroll
-            for (int gl = 0; gl < kF16TileGroups; gl++) wv4[gl] = wrow[(size_t)(g0 + (gl < ng ? gl : 0)) * gstride];
-            __syncthreads();  // the previous stage's tile is no longer read
-            // 8-value chunks: chunk c of row p covers columns 64 g0 + 8 c .. + 7
-            for (int q = tid; q < kF16TileRows * kF16TileGroups * 8; q += kMvThreads) {
-                const int p = q / (kF16TileGroups * 8), c = q % (kF16TileGroups * 8);
-                const int gl = c >> 3, m = c & 7;
-                float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                if (p < np && gl < ng) {
-                    const uint4 u = *reinterpret_cast<const uint4*>(x + (size_t)(p0 + p) * x_pitch +
-                                                                   ((size_t)(g0 + gl) * 64 + 8 * m) * 2);
-                    const uint32_t h[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-                    for (int t = 0; t < 8; t++) v[t] = h2f((uint16_t)(t & 1 ? h[t >> 1] >> 16 : h[t >> 1] & 0xFFFFu));
-                }
-#pragma unroll
-                for (int t = 0; t < 8; t++) xs[p][gl][t][m] = v[t];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int gl = 0; gl < kF16TileGroups; gl++) {
-                if (gl >= ng) break;
-                const uint32_t wq[4] = {wv4[gl].x, wv4[gl].y, wv4[gl].z, wv4[gl].w};
-                float wf[8];
-#pragma unroll
-                for (int m = 0; m < 8; m++) wf[m] = h2f((uint16_t)(m & 1 ? wq[m >> 1] >> 16 : wq[m >> 1] & 0xFFFFu));
-#pragma unroll
-                for (int p = 0; p < kF16TileRows; p++) {
-                    const float4 xa = *reinterpret_cast<const float4*>(&xs[p][gl][j][0]);
-                    const float4 xb = *reinterpret_cast<const float4*>(&xs[p][gl][j][4]);
-                    const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-                    for (int m = 0; m < 8; m++) acc[p] = __builtin_fmaf(xv[m], wf[m], acc[p]);  // exact product
-                }
-            }
-        }
-        // lanes 0..7 of each row summed left to right
-        const int base = tid & ~7;
-#pragma unroll
-        for (int p = 0; p < kF16TileRows; p++) {
-            float sum = __shfl(acc[p], base);
-#pragma unroll
-            for (int l = 1; l < 8; l++) sum = sum + __shfl(acc[p], base + l);
-            if (j == 0 && row < N && p < np) out[(size_t)(p0 + p) * out_pitch + row] = sum;
-        }
-    }
-}
-
-// F16, prefill (several activation rows): the lane chains of
-// k_matvec_f16_row with register tiles.  A 256-thread workgroup owns 32 R
-// weight rows and P activation rows; thread (row group rr, lane j) runs lane
-// j's chain for its R weight rows and the P activation rows (R x P chains),
-// over the 64-column groups in order.  Per chunk of GC groups it holds the
-// R weight rows' lane-j values in registers (the next chunk's requested
-// before this one is folded) and reads the P rows' lane-j values of each
-// group from LDS (fp32, staged per chunk, double-buffered): R P 8 fused
-// multiply-adds per 2 P LDS reads.  The products of two fp16 values are
-// exact in fp32, so each fused multiply-add is the reference's multiply
-// then add.  Workgroups of one weight block sit on one XCD when the grid's
-// x extent is a multiple of 8.
-template <int R, int P, int GC>
-__global__ __launch_bounds__(256) void k_mm_f16(const uint8_t* __restrict__ x, int x_pitch, int n_xrows,
-                                              const uint16_t* __restrict__ w, float* __restrict__ out, int out_pitch,
-                                              int N, int K)
-{
-    static_assert(P * GC * 8 <= 256, "one staged chunk per thread at most");
-    __shared__ __align__(16) float xs[2][P][GC][8][8];  // [buffer][row][group][lane j][m]
-    const int tid = threadIdx.x, j = tid & 7, rr = tid >> 3;
+    static_assert(GC % PF == 0, "a group's weight slot is fixed");
+    constexpr int kRows = 16 * RN, TPT = kRows * GC * 4 / 256;
+    static_assert(kRows * GC * 4 % 256 == 0, "staging tasks spread evenly");
+    __shared__ __align__(16) float4 xs[2][GC][8][2][kRows];  // [buffer][group][lane j][m / 4][row]
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int lc = lane & 15, lb = lane >> 4;
+    const int r0 = blockIdx.y * kRows;
+    const int c0 = (blockIdx.x * 4 + wv) * 16 * CN;
     const int G = K / 64, nck = (G + GC - 1) / GC;
     const size_t gstride = (size_t)((N + 7) & ~7) * 8;  // uint4s per group
-    const int wr0 = (int)blockIdx.x * (32 * R) + rr * R;
-    const int p0 = (int)blockIdx.y * P;
-    const uint4* wrow[R];
+    const uint4* wcol[CN];  // lane j = lb of this thread's columns; j + 4 follows 4 uint4s on
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int rowc = min(wr0 + r, N - 1);  // rows past N read a valid row and store nothing
-        wrow[r] = reinterpret_cast<const uint4*>(w) + (size_t)rowc * 8 + j;
+    for (int n = 0; n < CN; n++)
+        wcol[n] = reinterpret_cast<const uint4*>(w) + (size_t)min(c0 + 16 * n + lc, N - 1) * 8 + lb;
+
+    // staging: a task is two 8-value runs m = 2p, 2p + 1 of one (row, group),
+    // widened into the operand order
+    uint4 xq[TPT][2];
+    int t_row[TPT], t_g[TPT], t_p[TPT];
+#pragma unroll
+    for (int i = 0; i < TPT; i++) {
+        const int t = tid + i * 256;
+        t_row[i] = t % kRows;
+        t_g[i] = t / kRows % GC;
+        t_p[i] = t / (kRows * GC);
     }
-    // staging: thread q < P GC 8 converts the 8 values of (row q / (8 GC),
-    // group (q / 8) % GC, m = q % 8) of a chunk
-    auto stage = [&](int ck, int buf) {
-        if (tid < P * GC * 8) {
-            const int p = tid / (GC * 8), gl = (tid >> 3) % GC, m = tid & 7;
-            const int g = ck * GC + gl;
-            float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            if (p0 + p < n_xrows && g < G) {
-                const uint4 u =
-                    *reinterpret_cast<const uint4*>(x + (size_t)(p0 + p) * x_pitch + ((size_t)g * 64 + 8 * m) * 2);
-                const uint32_t h[4] = {u.x, u.y, u.z, u.w};
+    auto x_load = [&](int ck) {
 #pragma unroll
-                for (int t = 0; t < 8; t++) v[t] = h2f((uint16_t)(t & 1 ? h[t >> 1] >> 16 : h[t >> 1] & 0xFFFFu));
-            }
-#pragma unroll
-            for (int t = 0; t < 8; t++) xs[buf][p][gl][t][m] = v[t];
+        for (int i = 0; i < TPT; i++) {
+            const int g = min(ck * GC + t_g[i], G - 1);
+            const uint4* xrow = reinterpret_cast<const uint4*>(x + (size_t)min(r0 + t_row[i], n_rows - 1) * x_pitch);
+            xq[i][0] = xrow[g * 8 + 2 * t_p[i]];
+            xq[i][1] = xrow[g * 8 + 2 * t_p[i] + 1];
         }
     };
-    auto wload = [&](int ck, uint4 (&dst)[GC][R]) {
+    auto stage = [&](int buf) {
 #pragma unroll
-        for (int gl = 0; gl < GC; gl++) {
-            const int g = min(ck * GC + gl, G - 1);
+        for (int i = 0; i < TPT; i++) {
+            const uint32_t a[4] = {xq[i][0].x, xq[i][0].y, xq[i][0].z, xq[i][0].w};
+            const uint32_t b[4] = {xq[i][1].x, xq[i][1].y, xq[i][1].z, xq[i][1].w};
 #pragma unroll
-            for (int r = 0; r < R; r++) dst[gl][r] = load_stream(wrow[r] + (size_t)g * gstride);
-        }
-    };
-    float acc[R][P];
-#pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-        for (int p = 0; p < P; p++) acc[r][p] = 0.0f;
-    auto fold = [&](int ck, int buf, const uint4 (&wv)[GC][R]) {
-#pragma unroll
-        for (int gl = 0; gl < GC; gl++) {
-            if (ck * GC + gl >= G) break;  // uniform
-            float wf[R][8];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const uint32_t q[4] = {wv[gl][r].x, wv[gl][r].y, wv[gl][r].z, wv[gl][r].w};
-#pragma unroll
-                for (int m = 0; m < 8; m++) wf[r][m] = h2f((uint16_t)(m & 1 ? q[m >> 1] >> 16 : q[m >> 1] & 0xFFFFu));
-            }
-#pragma unroll
-            for (int p = 0; p < P; p++) {
-                const float4 xa = *reinterpret_cast<const float4*>(&xs[buf][p][gl][j][0]);
-                const float4 xb = *reinterpret_cast<const float4*>(&xs[buf][p][gl][j][4]);
-                const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-                for (int m = 0; m < 8; m++)
-#pragma unroll
-                    for (int r = 0; r < R; r++) acc[r][p] = __builtin_fmaf(xv[m], wf[r][m], acc[r][p]);
+            for (int j = 0; j < 8; j++) {
+                const uint32_t va = j & 1 ? a[j >> 1] >> 16 : a[j >> 1] & 0xFFFFu;
+                const uint32_t vb = j & 1 ? b[j >> 1] >> 16 : b[j >> 1] & 0xFFFFu;
+                reinterpret_cast<float2*>(&xs[buf][t_g[i]][j][t_p[i] >> 1][t_row[i]])[t_p[i] & 1] =
+                    make_float2(h2f((uint16_t)va), h2f((uint16_t)vb));
             }
         }
     };
-    uint4 wa[GC][R], wb[GC][R];
-    wload(0, wa);
-    stage(0, 0);
+    // the weights of the next PF groups, each group's slot refilled once its
+    // products are issued
+    uint4 wq[PF][CN][2];
+    auto w_load = [&](int g, uint4 (&q)[CN][2]) {
+        const size_t o = (size_t)min(g, G - 1) * gstride;
+#pragma unroll
+        for (int n = 0; n < CN; n++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) q[n][h] = wcol[n][o + 4 * h];
+    };
+    f16x_t acc[RN][CN][2];
+#pragma unroll
+    for (int r = 0; r < RN; r++)
+#pragma unroll
+        for (int n = 0; n < CN; n++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[r][n][h][e] = 0.0f;
+    // the weight operands of two K steps in fp32, converted while the
+    // products of the two before them are issued (a conversion into a
+    // register that a product in flight still reads would wait for it)
+    auto convert = [&](const uint4 (&q)[CN][2], int mp, float (&b)[CN][2][2]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int n = 0; n < CN; n++) {
+                const uint4& u = q[n][h];
+                const uint32_t d = mp == 0 ? u.x : mp == 1 ? u.y : mp == 2 ? u.z : u.w;
+                b[n][h][0] = h2f((uint16_t)(d & 0xFFFFu));
+                b[n][h][1] = h2f((uint16_t)(d >> 16));
+            }
+    };
+    auto group = [&](int buf, int gl, const uint4 (&q)[CN][2]) {
+        float4 xa[RN][2][2];  // [row tile][lane half][m / 4]
+#pragma unroll
+        for (int mh = 0; mh < 2; mh++)
+#pragma unroll
+            for (int r = 0; r < RN; r++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) xa[r][h][mh] = xs[buf][gl][4 * h + lb][mh][16 * r + lc];
+        float b[2][CN][2][2];
+        convert(q, 0, b[0]);
+#pragma unroll
+        for (int mp = 0; mp < 4; mp++) {
+            if (mp < 3) convert(q, mp + 1, b[(mp + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int r = 0; r < RN; r++) {
+                        const float4 v = xa[r][h][mp >> 1];
+                        const float a = mp & 1 ? (t ? v.w : v.z) : (t ? v.y : v.x);
+#pragma unroll
+                        for (int n = 0; n < CN; n++)
+                            acc[r][n][h] = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b[mp & 1][n][h][t], acc[r][n][h], 0, 0, 0);
+                    }
+        }
+    };
+    x_load(0);
+#pragma unroll
+    for (int p = 0; p < PF; p++) w_load(p, wq[p]);
+    stage(0);
+    x_load(min(1, nck - 1));
     __syncthreads();
-    // chunks in pairs, so the two weight sets keep compile-time names
-    for (int ck = 0; ck < nck; ck += 2) {
-        if (ck + 1 < nck) {
-            wload(ck + 1, wb);
-            stage(ck + 1, 1);
+    for (int ck = 0; ck < nck; ck++) {
+        const int buf = ck & 1, g0 = ck * GC;
+#pragma unroll
+        for (int gl = 0; gl < GC; gl++) {
+            if (g0 + gl < G) group(buf, gl, wq[gl % PF]);  // uniform
+            w_load(g0 + gl + PF, wq[gl % PF]);
         }
-        fold(ck, 0, wa);
-        __syncthreads();
-        if (ck + 1 >= nck) break;  // uniform
-        if (ck + 2 < nck) {
-            wload(ck + 2, wa);
-            stage(ck + 2, 0);
-        }
-        fold(ck + 1, 1, wb);
-        __syncthreads();
+        stage(buf ^ 1);  // past the end: the last chunk again, never read
+        x_load(min(ck + 2, nck - 1));
+        lds_barrier();
     }
-    // lanes 0..7 of each (weight row, activation row) summed left to right
-    const int base = tid & ~7;
 #pragma unroll
-    for (int r = 0; r < R; r++)
+    for (int r = 0; r < RN; r++)
 #pragma unroll
-        for (int p = 0; p < P; p++) {
-            float s = __shfl(acc[r][p], base);
+        for (int n = 0; n < CN; n++) {
+            const int col = c0 + 16 * n + lc;
 #pragma unroll
-            for (int l = 1; l < 8; l++) s = s + __shfl(acc[r][p], base + l);
-            if (j == 0 && wr0 + r < N && p0 + p < n_xrows) out[(size_t)(p0 + p) * out_pitch + wr0 + r] = s;
+            for (int i = 0; i < 4; i++) {
+                const int row = r0 + 16 * r + 4 * lb + i;
+                float s = acc[r][n][0][i];
+#pragma unroll
+                for (int j = 1; j < 8; j++) s = s + acc[r][n][j >> 2][(j & 3) * 4 + i];
+                if (row < n_rows && col < N) {
+                    if constexpr (ODT == F32) reinterpret_cast<float*>(out)[(size_t)row * out_pitch + col] = s;
+                    else reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(out) + (size_t)row * out_pitch)[col] = f2h(s);
+                }
+            }
         }
 }
 
 // F16, one activation row (decode): a 64-thread workgroup owns 8 rows, thread
 // (row, lane j) folds lane j's chain over the 64-column groups in order
-// exactly as k_matvec_f16 does, but keeps two batches of kF16Batch weight
+// and keeps two batches of kF16Batch weight
 // runs in flight (the next batch is requested before the current one is
 // folded), so the fold is not serialised behind one load per group.
 constexpr int kF16Batch = 16;
-constexpr int kMmF16Rows = 8;  // activation rows per k_mm_f16 workgroup; matvec_raw takes it from this many rows
 
 __global__ __launch_bounds__(64) void k_matvec_f16_row(const uint8_t* __restrict__ x, const uint16_t* __restrict__ w,
                                                       float* __restrict__ out, int N, int K)
@@ -674,6 +609,36 @@ bool dmv_f16_dispatch(int G, Launch&& go)
     }
 }
 
+// fp16 products: rows of whole 64-value groups, up to 16384 values.
+static bool f16_shape_ok(const nc_tensor* w) { return w->cols % 64 == 0 && w->cols > 0 && w->cols <= 16384; }
+
+// The fp16 product of several rows.  Shapes by the number of 64-column tiles
+// of 16 and 32 rows (us at the shapes around the lines, in that order):
+// two row tiles share each weight operand once 640 such workgroups exist
+// (704: 65 against 71; 352: 45 against 39); below, one row tile, with four
+// groups of weights in flight up to 384 workgroups (256: 42 against 46) and
+// two beyond (528: 37 against 39, 704: 40 against 43).
+template <int ODT>
+static int mfma_f16(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, void* out, int out_pitch,
+                    hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop)
+{
+    const int N = w->rows, K = w->cols;
+    const int tc = (N + 63) / 64, t1 = tc * ((n_rows + 15) / 16), t2 = tc * ((n_rows + 31) / 32);
+    auto go = [&](auto kern, int rows) {
+        const dim3 grid(tc, (n_rows + rows - 1) / rows);
+        if (ev_start)
+            hipExtLaunchKernelGGL(kern, grid, dim3(256), 0, st, ev_start, ev_stop, 0, x, x_pitch, n_rows,
+                                  (const uint16_t*)w->data, out, out_pitch, N, K);
+        else
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x, x_pitch, n_rows, (const uint16_t*)w->data, out,
+                               out_pitch, N, K);
+    };
+    if (t2 >= 640) go(k_mfma_f16<2, 1, 2, 2, ODT>, 32);
+    else if (t1 > 384) go(k_mfma_f16<1, 1, 4, 2, ODT>, 16);
+    else go(k_mfma_f16<1, 1, 4, 4, ODT>, 16);
+    return launch_status("k_mfma_f16");
+}
+
 // out[r, c] = dot(x[r], w[c]) for x rows [0, n_rows) (pointers already at
 // the first row), fp32 out with `out_pitch` floats per row.
 int matvec_raw(const uint8_t* x, int x_dtype, int x_pitch, int n_rows, const nc_tensor* w, float* out, int out_pitch,
@@ -710,8 +675,8 @@ int matvec_raw(const uint8_t* x, int x_dtype, int x_pitch, int n_rows, const nc_
     if (w->dtype == NC_F16) {
         if (x_dtype != NC_F16) return fail(NC_ERR_ARG, "matmul: F16 weights need F16 activations");
         if (K % 64) return fail(NC_ERR_ARG, "matmul: F16 path needs K %% 64 == 0, K=%d", K);
+        if (!f16_shape_ok(w)) return fail(NC_ERR_ARG, "matmul: K=%d too large", K);
         const size_t lds = (size_t)K * 4;
-        if (lds > 64 * 1024) return fail(NC_ERR_ARG, "matmul: K=%d too large", K);
         if (n_rows == 1) {
             const dim3 grid((N + 7) / 8);
             auto go = [&](auto kern) {
@@ -732,26 +697,7 @@ int matvec_raw(const uint8_t* x, int x_dtype, int x_pitch, int n_rows, const nc_
                                    out, N, K);
             return launch_status("k_matvec_f16_row");
         }
-        if (n_rows >= kMmF16Rows) {
-            // 64 weight rows x 8 activation rows per workgroup (measured best of R x P x GC
-            // in {1, 2, 4, 8} x {4, 8, 16} x {1, 2, 4} on Zephyr's 128-row prefill)
-            const dim3 grid2((N + 63) / 64, (n_rows + kMmF16Rows - 1) / kMmF16Rows);
-            if (ev_start)
-                hipExtLaunchKernelGGL((k_mm_f16<2, kMmF16Rows, 2>), grid2, dim3(256), 0, st, ev_start, ev_stop, 0, x,
-                                      x_pitch, n_rows, (const uint16_t*)w->data, out, out_pitch, N, K);
-            else
-                hipLaunchKernelGGL((k_mm_f16<2, kMmF16Rows, 2>), grid2, dim3(256), 0, st, x, x_pitch, n_rows,
-                                   (const uint16_t*)w->data, out, out_pitch, N, K);
-            return launch_status("k_mm_f16");
-        }
-        const dim3 grid((N + 31) / 32);
-        if (n_rows >= 4) {
-            NC_MV_LAUNCH(k_matvec_f16_tile, grid, 0, x, x_pitch, n_rows, (const uint16_t*)w->data, out, out_pitch, N,
-                         K);
-            return launch_status("k_matvec_f16_tile");
-        }
-        NC_MV_LAUNCH(k_matvec_f16, grid, lds, x, x_pitch, n_rows, (const uint16_t*)w->data, out, out_pitch, N, K);
-        return launch_status("k_matvec_f16");
+        return mfma_f16<F32>(x, x_pitch, n_rows, w, out, out_pitch, st, ev_start, ev_stop);
     }
     return fail(NC_ERR_ARG, "matmul: weight dtype %d", w->dtype);
 #undef NC_MV_LAUNCH
@@ -909,13 +855,16 @@ bool overlap(const void* a, size_t na, const void* b, size_t nb)
 }
 
 // Whether the launch that computes x [rows] times w can store out's
-// activation rows itself: the rules of gemm_q_act, and no output byte that
-// the product still reads (a staged product has read everything before it
-// writes).
+// activation rows itself: a launch that does (gemm_q_act's, or several fp16
+// rows), and no output byte that the product still reads (a staged product
+// has read everything before it writes).
 bool stores_rows(const nc_tensor* x, const uint8_t* xr, const nc_tensor* w, const nc_tensor* out, const uint8_t* orow,
                  int rows)
 {
-    if (out->dtype != NC_Q8 || x->dtype != NC_Q8 || x->cols <= 0 || !gemm_q_act_supported(x->pitch, rows, w)) return false;
+    if (out->dtype != x->dtype || x->cols <= 0) return false;
+    if (x->dtype == NC_Q8 ? !gemm_q_act_supported(x->pitch, rows, w)
+                          : x->dtype != NC_F16 || w->dtype != NC_F16 || !f16_shape_ok(w) || rows < 2)
+        return false;
     const size_t on = (size_t)rows * out->pitch;
     size_t cb, db;
     if (nc_weight_bytes(w->dtype, w->rows, w->cols, &cb, &db)) return false;
@@ -946,7 +895,9 @@ int matmul_2d(const char* name, const nc_tensor* x, const nc_tensor* w, nc_tenso
     float* sp = nullptr;
     int s = stage((size_t)rows * w->rows * 4, rows, &sp);
     if (s) return s;
-    if (stores_rows(x, xr, w, out, orow, rows)) return gemm_q_act(xr, x->pitch, rows, w, orow, out->pitch, st);
+    if (stores_rows(x, xr, w, out, orow, rows))
+        return x->dtype == NC_Q8 ? gemm_q_act(xr, x->pitch, rows, w, orow, out->pitch, st)
+                                 : mfma_f16<F16>(xr, x->pitch, rows, w, orow, out->pitch, st, nullptr, nullptr);
     if ((s = matvec_raw(xr, x->dtype, x->pitch, rows, w, sp, w->rows, st))) return s;
     return write_rows(sp, w->rows, orow, out->pitch, out->dtype, w->rows, rows, st);
 }

@@ -140,6 +140,33 @@ def test_matmul_wide(gpu, oracle, wdt, K, N, rows, start, odt):
     assert_same(got[start:], want[start:], f"matmul Q{8 if wdt == Q8 else 4} K={K} N={N} out {odt}")
 
 
+F16_CASES = [
+    # (K, N, rows, start): fp16 products of several rows on the matrix cores:
+    # one group, groups past a staged chunk, rows and columns past a tile, and
+    # the three launch shapes (up to 384 workgroups of 16 rows, more, and from
+    # 640 of 32 rows)
+    (64, 70, 2, 0),
+    (320, 129, 18, 1),
+    (128, 8, 7, 0),
+    (192, 1300, 300, 0),
+    (64, 1000, 1281, 0),
+]
+
+
+@pytest.mark.parametrize("K,N,rows,start", F16_CASES)
+@pytest.mark.parametrize("odt", [F32, F16])
+def test_matmul_f16_rows(gpu, oracle, K, N, rows, start, odt):
+    rng = np.random.default_rng(K + N)
+    x = rand_act(oracle, rng, F16, rows, K, 30.0)
+    w = rand_weight(oracle, rng, F16, N, K, 4.0)
+    want = np.zeros((rows, N), np.float32) if odt == F32 else np.zeros((rows, OL.row_bytes(F16, N)), np.uint8)
+    oracle.matmul(OL.ptr(x), F16, OL.ptr(w), F16, OL.ptr(want), odt, K, N, start, rows, None)
+    dx, dw, out = DevAct(x, F16, rows, K), DevWeight(w, F16, N, K), DevAct.empty(odt, rows, N)
+    gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), start, rows, None), "matmul")
+    got = out.ref() if odt == F16 else out.ref().view(np.float32)
+    assert_same(got[start:], want[start:], f"matmul f16 K={K} N={N} rows={rows} out {odt}")
+
+
 def test_matmul_in_place(gpu, oracle):
     """Output rows over the input rows: the product is read whole first."""
     rng = np.random.default_rng(17)
