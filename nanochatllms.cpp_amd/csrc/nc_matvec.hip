@@ -103,6 +103,208 @@ __global__ __launch_bounds__(kMvThreads) void k_matvec_q(const uint8_t* __restri
     }
 }
 
+// One to seven activation rows times a Q4 / Q8 weight, stored as Q8 rows by
+// the launch itself (k_matvec_q and write_rows in one): a workgroup owns the
+// 32 columns of one output block.  512 threads hold its weight blocks in
+// registers and park the lane terms in LDS; a ninth wavefront folds the
+// chains and quantizes the block.
+//
+// What bounds it: latency.  One row (MULTI false): load, terms, one fold of
+// nb dependent adds (two chains per lane, 128 in all), the quantize.  More
+// rows (MULTI): the columns go in two halves of 16, each with a term buffer
+// of its own, and in phase t = 2 p + half the terms of t are computed while
+// the ninth wavefront folds those of t - 1, one barrier per phase; the next
+// row is staged in the phase before it is used.
+// Measured with the fp32 pass it replaces (us): 1 row x 5632 x 2048 Q4 7.8 ->
+// 4.3; 5 rows x 5760 x 2304 Q8 20.8 -> 12.4 (the terms' reads of the staged
+// rows, 64 bytes of LDS per lane and block, set the pace there).
+constexpr int kMaTerm = 512;              // term threads
+constexpr int kMaThreads = kMaTerm + kWave;
+
+template <int WT, int IH, bool MULTI>
+__global__ __launch_bounds__(kMaThreads) void k_matvec_qa(const uint8_t* __restrict__ x, int x_pitch, int n_xrows,
+                                                          const uint32_t* __restrict__ wq,
+                                                          const uint16_t* __restrict__ wd, uint8_t* __restrict__ out,
+                                                          int out_pitch, int N, int nb)
+{
+    constexpr int WD = WT == Q4 ? 4 : 8;
+    extern __shared__ __align__(16) uint32_t lds[];
+    const int tp = ((nb + 3) & ~3) + 4;
+    const int xstride = nb * kStage;                                     // staged rows: MULTI two, else one
+    float* T = reinterpret_cast<float*>(lds + (MULTI ? 2 : 1) * xstride);  // [half][64 chains][tp]
+    const int tid = threadIdx.x;
+    const int col0 = blockIdx.x * 32;
+
+    if (tid < kMaTerm) {
+        // the first row's block, then every weight block of this thread
+        const bool stager = tid < nb;
+        XRaw xr{};
+        if (stager) xr = load_x_block(x, nb, tid);
+        uint4 w[2][IH][WD / 4];
+        uint16_t dw16[2][IH];
+        int tix[IH], bix[IH];
+#pragma unroll
+        for (int it = 0; it < IH; it++) {
+            const int j = tid + it * kMaTerm;
+            const int r = j / nb, i = j - r * nb;
+            tix[it] = j < 16 * nb ? r * 4 * tp + i : -1;
+            bix[it] = i;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                // columns past N (and items past the half) read a valid block
+                const int c = min(col0 + 16 * h + min(r, 15), N - 1);
+                const size_t b = (size_t)c * nb + i;
+                const uint4* src = reinterpret_cast<const uint4*>(wq + b * WD);
+#pragma unroll
+                for (int v = 0; v < WD / 4; v++) w[h][it][v] = load_stream(src + v);
+                dw16[h][it] = load_stream(wd + b);
+            }
+        }
+        auto terms = [&](int h, const uint32_t* xs) {
+#pragma unroll
+            for (int it = 0; it < IH; it++) {
+                // the codes are unpacked here, not once for all rows (which
+                // would hold twice the registers)
+#pragma unroll
+                for (int v = 0; v < WD / 4; v++)
+                    asm volatile("" : "+v"(w[h][it][v].x), "+v"(w[h][it][v].y), "+v"(w[h][it][v].z), "+v"(w[h][it][v].w));
+                if (tix[it] < 0) continue;
+                float tv[4];
+                q_block_terms<WT>(xs + bix[it] * kStage, w[h][it], dw16[h][it], tv);
+                float* t = T + h * 64 * tp + tix[it];
+#pragma unroll
+                for (int k = 0; k < 4; k++) t[k * tp] = tv[k];
+            }
+        };
+        if (stager) stage_x_block(xr, lds + tid * kStage);
+        lds_barrier();
+        if constexpr (!MULTI) {
+            terms(0, lds);
+            terms(1, lds);
+            lds_barrier();
+        } else {
+            for (int p = 0; p < n_xrows; p++) {
+                const uint32_t* xs = lds + (p & 1) * xstride;
+                const bool more = p + 1 < n_xrows;
+                if (more && stager) xr = load_x_block(x + (size_t)(p + 1) * x_pitch, nb, tid);
+                terms(0, xs);
+                lds_barrier();  // phase 2 p
+                terms(1, xs);
+                if (more && stager) stage_x_block(xr, lds + ((p + 1) & 1) * xstride + tid * kStage);
+                lds_barrier();  // phase 2 p + 1
+            }
+        }
+        return;
+    }
+
+    // the fold wavefront: lane = chain (column lane >> 2 of a half, AVX lane
+    // lane & 3)
+    const int lane = tid & (kWave - 1);
+    auto column = [&](float acc) {
+        const int g = lane & ~3;
+        const float a0 = __shfl(acc, g), a1 = __shfl(acc, g + 1), a2 = __shfl(acc, g + 2), a3 = __shfl(acc, g + 3);
+        return (a0 + a1) + (a2 + a3);
+    };
+    auto store = [&](int p, float va, float vb) {
+        // q8_quant_lane over the block's 32 columns (each on four lanes)
+        const int ca = col0 + (lane >> 2), cb = ca + 16;
+        float a = fmaxf(ca < N ? fabsf(va) : 0.0f, cb < N ? fabsf(vb) : 0.0f);
+        a = half_wave_max(a);
+        a = fmaxf(a, __shfl_xor(a, 32));
+        const float delta = a / 127.0f;
+        const float scale = delta != 0.0f ? 1.0f / delta : 0.0f;
+        uint8_t* o = out + (size_t)p * out_pitch;
+        if ((lane & 3) == 0) {
+            if (ca < N) o[ca] = (uint8_t)(int8_t)roundf(va * scale);
+            if (cb < N) o[cb] = (uint8_t)(int8_t)roundf(vb * scale);
+        }
+        if (lane == 0) reinterpret_cast<uint16_t*>(o + act_delta_offset(N))[col0 >> 5] = f2h(delta);
+    };
+    lds_barrier();  // the first row's staging
+    if constexpr (!MULTI) {
+        lds_barrier();  // the terms
+        const float *ta = T + lane * tp, *tb = ta + 64 * tp;
+        float sa = 0.0f, sb = 0.0f;
+        int c = 0;
+        for (; c + 16 <= nb; c += 16) {
+            float4 a[4], b[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                a[q] = reinterpret_cast<const float4*>(ta + c)[q];
+                b[q] = reinterpret_cast<const float4*>(tb + c)[q];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                sa = sa + a[q].x;
+                sb = sb + b[q].x;
+                sa = sa + a[q].y;
+                sb = sb + b[q].y;
+                sa = sa + a[q].z;
+                sb = sb + b[q].z;
+                sa = sa + a[q].w;
+                sb = sb + b[q].w;
+            }
+        }
+        for (; c < nb; c++) {
+            sa = sa + ta[c];
+            sb = sb + tb[c];
+        }
+        const float va = column(sa), vb = column(sb);
+        store(0, va, vb);
+    } else {
+        for (int p = 0; p < n_xrows; p++) {
+            lds_barrier();  // phase 2 p: half 0's terms are there
+            const float va = column(seq_sum<16>(T + lane * tp, nb));
+            lds_barrier();  // phase 2 p + 1: half 1's
+            const float vb = column(seq_sum<16>(T + (64 + lane) * tp, nb));
+            store(p, va, vb);
+        }
+    }
+}
+
+static size_t matvec_qa_lds(int nb, bool multi)
+{
+    const int tp = ((nb + 3) & ~3) + 4;
+    return ((size_t)(multi ? 2 : 1) * nb * kStage + (size_t)128 * tp) * 4;
+}
+
+// Whether k_matvec_qa takes this product: rows below the prefill matmul's,
+// and shared memory and registers for its blocks.
+static bool matvec_qa_supported(int n_rows, const nc_tensor* w)
+{
+    const int nb = w->cols / 32;
+    return (w->dtype == NC_Q4 || w->dtype == NC_Q8) && w->cols > 0 && w->cols % 32 == 0 && w->rows > 0 && n_rows >= 1 &&
+           n_rows < kGemmMinRows && nb <= 256 && matvec_qa_lds(nb, n_rows > 1) <= 160 * 1024;
+}
+
+static int matvec_qa(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, uint8_t* out, int out_pitch,
+                     hipStream_t st)
+{
+    const int N = w->rows, nb = w->cols / 32;
+    const dim3 grid((N + 31) / 32);
+    auto go = [&](auto kern, bool multi) {
+        const size_t lds = matvec_qa_lds(nb, multi);
+        hipLaunchKernelGGL(kern, grid, dim3(kMaThreads), lds, st, x, x_pitch, n_rows, (const uint32_t*)w->data,
+                           (const uint16_t*)w->deltas, out, out_pitch, N, nb);
+        return launch_status("k_matvec_qa");
+    };
+    auto by_items = [&](auto wt, auto multi) {
+        constexpr int WT = decltype(wt)::value;
+        constexpr bool M = decltype(multi)::value;
+        const int ih = (16 * nb + kMaTerm - 1) / kMaTerm;  // weight blocks per thread and half
+        if (ih <= 1) return go(k_matvec_qa<WT, 1, M>, M);
+        if (ih <= 2) return go(k_matvec_qa<WT, 2, M>, M);
+        if (ih <= 3) return go(k_matvec_qa<WT, 3, M>, M);
+        if (ih <= 4) return go(k_matvec_qa<WT, 4, M>, M);
+        if (ih <= 6) return go(k_matvec_qa<WT, 6, M>, M);
+        return go(k_matvec_qa<WT, 8, M>, M);
+    };
+    auto by_rows = [&](auto wt) {
+        return n_rows > 1 ? by_items(wt, std::true_type{}) : by_items(wt, std::false_type{});
+    };
+    return w->dtype == NC_Q4 ? by_rows(std::integral_constant<int, Q4>{}) : by_rows(std::integral_constant<int, Q8>{});
+}
+
 // F16, prefill, on the matrix cores.  v_mfma_f32_16x16x1_4b_f32 multiplies
 // four independent pairs of 16-vectors (one K step each) and adds them to
 // four 16 x 16 fp32 accumulators: one fused multiply-add per entry, which on
@@ -289,8 +491,9 @@ __global__ __launch_bounds__(256) void k_mfma_f16(const uint8_t* __restrict__ x,
 // folded), so the fold is not serialised behind one load per group.
 constexpr int kF16Batch = 16;
 
+template <bool H16>
 __global__ __launch_bounds__(64) void k_matvec_f16_row(const uint8_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                      float* __restrict__ out, int N, int K)
+                                                      void* __restrict__ out, int N, int K)
 {
     extern __shared__ __align__(16) float xsf[];  // [K/64][8 lanes][8]
     const int tid = threadIdx.x;
@@ -366,7 +569,10 @@ __global__ __launch_bounds__(64) void k_matvec_f16_row(const uint8_t* __restrict
     float s = __shfl(acc, base);
 #pragma unroll
     for (int l = 1; l < 8; l++) s = s + __shfl(acc, base + l);
-    if (j == 0 && row < N) out[row] = s;
+    if (j == 0 && row < N) {
+        if constexpr (H16) static_cast<uint16_t*>(out)[row] = f2h(s);
+        else static_cast<float*>(out)[row] = s;
+    }
 }
 
 // Fold of one wavefront's 64 lane chains (8 rows x 8 lanes, thread (row,
@@ -422,7 +628,8 @@ __device__ __forceinline__ int dmv_f16_row(int q, int sub, int N)
 // out.  GLU: the fp16 SwiGLU values m[4q + i] = Act(Act(silu(Act(g))) *
 // Act(u)) as k_silu_mul does them (tinyllama/tinyllama.cpp:88-97 in the
 // fp16 dtype).
-template <bool GLU>
+// With H16 (not GLU) the fp16 values to m_out[row].
+template <bool GLU, bool H16 = false>
 __device__ __forceinline__ void dmv_f16_finish(float acc, int lane, int q, int row, int N, float* out,
                                                uint16_t* m_out)
 {
@@ -431,7 +638,10 @@ __device__ __forceinline__ void dmv_f16_finish(float acc, int lane, int q, int r
 #pragma unroll
     for (int l = 1; l < 8; l++) s = s + __shfl(acc, base + l);
     if (!GLU) {
-        if ((lane & 7) == 0 && row < N) out[row] = s;
+        if ((lane & 7) == 0 && row < N) {
+            if constexpr (H16) m_out[row] = f2h(s);
+            else out[row] = s;
+        }
         return;
     }
     const float gsum = __shfl(s, (lane & 3) * 8), usum = __shfl(s, ((lane & 3) + 4) * 8);
@@ -446,7 +656,7 @@ __device__ __forceinline__ void dmv_f16_finish(float acc, int lane, int q, int r
 // F16, one activation row (decode), for the group counts G = K / 64 it is
 // built for: one wavefront per 8 rows (dmv_f16_fold); the row is staged
 // into LDS as fp16 in the fold's order while the weight ring is in flight.
-template <int G, int D, int P, bool GLU>
+template <int G, int D, int P, bool GLU, bool H16 = false>
 __global__ __launch_bounds__(64) void k_dmv_f16(const uint8_t* __restrict__ x, const uint16_t* __restrict__ w,
                                                float* __restrict__ out, int N, uint16_t* __restrict__ m_out)
 {
@@ -480,7 +690,7 @@ __global__ __launch_bounds__(64) void k_dmv_f16(const uint8_t* __restrict__ x, c
     }
     __syncthreads();
     const float acc = dmv_f16_fold<G, D, P>(xs, wv, wrow, gstride, j);
-    dmv_f16_finish<GLU>(acc, lane, q, row, N, out, m_out);
+    dmv_f16_finish<GLU, H16>(acc, lane, q, row, N, out, m_out);
 }
 
 // The norm of the row fused into the fp16 decode matvec that consumes it
@@ -597,14 +807,14 @@ __global__ __launch_bounds__(kNrmNorm + kNrmFold) void k_dmv_f16_nrm(
 
 // The group counts k_dmv_f16 is built for (d_model and d_ffn of the fp16
 // models: 2048 / 5632 and 2304 / 5760), with the ring depths measured best.
-template <bool GLU, class Launch>
+template <bool GLU, bool H16 = false, class Launch>
 bool dmv_f16_dispatch(int G, Launch&& go)
 {
     switch (G) {
-    case 32: go(k_dmv_f16<32, 32, 8, GLU>); return true;
-    case 36: go(k_dmv_f16<36, 36, 8, GLU>); return true;
-    case 88: go(k_dmv_f16<88, 32, 8, GLU>); return true;
-    case 90: go(k_dmv_f16<90, 32, 8, GLU>); return true;
+    case 32: go(k_dmv_f16<32, 32, 8, GLU, H16>); return true;
+    case 36: go(k_dmv_f16<36, 36, 8, GLU, H16>); return true;
+    case 88: go(k_dmv_f16<88, 32, 8, GLU, H16>); return true;
+    case 90: go(k_dmv_f16<90, 32, 8, GLU, H16>); return true;
     default: return false;
     }
 }
@@ -637,6 +847,32 @@ static int mfma_f16(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* 
     else if (t1 > 384) go(k_mfma_f16<1, 1, 4, 2, ODT>, 16);
     else go(k_mfma_f16<1, 1, 4, 4, ODT>, 16);
     return launch_status("k_mfma_f16");
+}
+
+// One fp16 row (K up to 8192) times w: fp32 dots, or (H16) their fp16 values.
+template <bool H16>
+static int f16_row(const uint8_t* x, const nc_tensor* w, void* out, hipStream_t st, hipEvent_t ev_start,
+                   hipEvent_t ev_stop)
+{
+    const int N = w->rows, K = w->cols;
+    const dim3 grid((N + 7) / 8);
+    float* of = H16 ? nullptr : static_cast<float*>(out);
+    uint16_t* oh = H16 ? static_cast<uint16_t*>(out) : nullptr;
+    auto go = [&](auto kern) {
+        if (ev_start)
+            hipExtLaunchKernelGGL(kern, grid, dim3(64), 0, st, ev_start, ev_stop, 0, x, (const uint16_t*)w->data, of, N,
+                                  oh);
+        else
+            hipLaunchKernelGGL(kern, grid, dim3(64), 0, st, x, (const uint16_t*)w->data, of, N, oh);
+    };
+    if (dmv_f16_dispatch<false, H16>(K / 64, go)) return launch_status("k_dmv_f16");
+    const size_t lds = (size_t)K * 4;
+    if (ev_start)
+        hipExtLaunchKernelGGL(k_matvec_f16_row<H16>, grid, dim3(64), lds, st, ev_start, ev_stop, 0, x,
+                              (const uint16_t*)w->data, out, N, K);
+    else
+        hipLaunchKernelGGL(k_matvec_f16_row<H16>, grid, dim3(64), lds, st, x, (const uint16_t*)w->data, out, N, K);
+    return launch_status("k_matvec_f16_row");
 }
 
 // out[r, c] = dot(x[r], w[c]) for x rows [0, n_rows) (pointers already at
@@ -676,27 +912,7 @@ int matvec_raw(const uint8_t* x, int x_dtype, int x_pitch, int n_rows, const nc_
         if (x_dtype != NC_F16) return fail(NC_ERR_ARG, "matmul: F16 weights need F16 activations");
         if (K % 64) return fail(NC_ERR_ARG, "matmul: F16 path needs K %% 64 == 0, K=%d", K);
         if (!f16_shape_ok(w)) return fail(NC_ERR_ARG, "matmul: K=%d too large", K);
-        const size_t lds = (size_t)K * 4;
-        if (n_rows == 1) {
-            const dim3 grid((N + 7) / 8);
-            auto go = [&](auto kern) {
-                if (ev_start)
-                    hipExtLaunchKernelGGL(kern, grid, dim3(64), 0, st, ev_start, ev_stop, 0, x,
-                                          (const uint16_t*)w->data, out, N, nullptr);
-                else
-                    hipLaunchKernelGGL(kern, grid, dim3(64), 0, st, x, (const uint16_t*)w->data, out, N, nullptr);
-            };
-            if (dmv_f16_dispatch<false>(K / 64, go)) return launch_status("k_dmv_f16");
-        }
-        if (n_rows == 1 && K <= 8192) {
-            if (ev_start)
-                hipExtLaunchKernelGGL(k_matvec_f16_row, dim3((N + 7) / 8), dim3(64), lds, st, ev_start, ev_stop, 0, x,
-                                      (const uint16_t*)w->data, out, N, K);
-            else
-                hipLaunchKernelGGL(k_matvec_f16_row, dim3((N + 7) / 8), dim3(64), lds, st, x, (const uint16_t*)w->data,
-                                   out, N, K);
-            return launch_status("k_matvec_f16_row");
-        }
+        if (n_rows == 1 && K <= 8192) return f16_row<false>(x, w, out, st, ev_start, ev_stop);
         return mfma_f16<F32>(x, x_pitch, n_rows, w, out, out_pitch, st, ev_start, ev_stop);
     }
     return fail(NC_ERR_ARG, "matmul: weight dtype %d", w->dtype);
@@ -855,15 +1071,15 @@ bool overlap(const void* a, size_t na, const void* b, size_t nb)
 }
 
 // Whether the launch that computes x [rows] times w can store out's
-// activation rows itself: a launch that does (gemm_q_act's, or several fp16
-// rows), and no output byte that the product still reads (a staged product
+// activation rows itself: a launch that does (gemm_q_act's, k_matvec_qa's, the
+// fp16 ones), and no output byte that the product still reads (a staged product
 // has read everything before it writes).
 bool stores_rows(const nc_tensor* x, const uint8_t* xr, const nc_tensor* w, const nc_tensor* out, const uint8_t* orow,
                  int rows)
 {
     if (out->dtype != x->dtype || x->cols <= 0) return false;
-    if (x->dtype == NC_Q8 ? !gemm_q_act_supported(x->pitch, rows, w)
-                          : x->dtype != NC_F16 || w->dtype != NC_F16 || !f16_shape_ok(w) || rows < 2)
+    if (x->dtype == NC_Q8 ? !gemm_q_act_supported(x->pitch, rows, w) && !matvec_qa_supported(rows, w)
+                          : x->dtype != NC_F16 || w->dtype != NC_F16 || !f16_shape_ok(w))
         return false;
     const size_t on = (size_t)rows * out->pitch;
     size_t cb, db;
@@ -895,9 +1111,13 @@ int matmul_2d(const char* name, const nc_tensor* x, const nc_tensor* w, nc_tenso
     float* sp = nullptr;
     int s = stage((size_t)rows * w->rows * 4, rows, &sp);
     if (s) return s;
-    if (stores_rows(x, xr, w, out, orow, rows))
-        return x->dtype == NC_Q8 ? gemm_q_act(xr, x->pitch, rows, w, orow, out->pitch, st)
-                                 : mfma_f16<F16>(xr, x->pitch, rows, w, orow, out->pitch, st, nullptr, nullptr);
+    if (stores_rows(x, xr, w, out, orow, rows)) {
+        if (x->dtype == NC_Q8)
+            return rows < kGemmMinRows ? matvec_qa(xr, x->pitch, rows, w, orow, out->pitch, st)
+                                       : gemm_q_act(xr, x->pitch, rows, w, orow, out->pitch, st);
+        if (rows == 1 && w->cols <= 8192) return f16_row<true>(xr, w, orow, st, nullptr, nullptr);
+        return mfma_f16<F16>(xr, x->pitch, rows, w, orow, out->pitch, st, nullptr, nullptr);
+    }
     if ((s = matvec_raw(xr, x->dtype, x->pitch, rows, w, sp, w->rows, st))) return s;
     return write_rows(sp, w->rows, orow, out->pitch, out->dtype, w->rows, rows, st);
 }
