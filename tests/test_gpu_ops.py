@@ -167,6 +167,48 @@ def test_matmul_f16_rows(gpu, oracle, K, N, rows, start, odt):
     assert_same(got[start:], want[start:], f"matmul f16 K={K} N={N} rows={rows} out {odt}")
 
 
+FEW_CASES = [
+    # (w dtype, K, N, rows, start): one to seven rows stored as Q8 rows by the
+    # launch: one block, a part of a thread's last item, the shared memory
+    # limit for several rows (224 blocks) and past it (the staged route), a
+    # partial last output block
+    (Q4, 32, 40, 1, 0),
+    (Q4, 2304, 2304, 1, 2),
+    (Q8, 5760, 70, 1, 0),
+    (Q4, 8192, 96, 1, 0),
+    (Q8, 64, 33, 7, 0),
+    (Q8, 2304, 100, 5, 1),
+    (Q4, 5632, 64, 2, 0),
+    (Q8, 7168, 48, 3, 0),
+    (Q4, 7200, 48, 3, 0),
+]
+
+
+@pytest.mark.parametrize("wdt,K,N,rows,start", FEW_CASES)
+def test_matmul_few_rows(gpu, oracle, wdt, K, N, rows, start):
+    rng = np.random.default_rng(K + N)
+    rows += start
+    x = rand_act(oracle, rng, Q8, rows, K)
+    w = rand_weight(oracle, rng, wdt, N, K)
+    want = np.zeros((rows, OL.row_bytes(Q8, N)), np.uint8)
+    oracle.matmul(OL.ptr(x), Q8, OL.ptr(w), wdt, OL.ptr(want), Q8, K, N, start, rows, None)
+    dx, dw, out = DevAct(x, Q8, rows, K), DevWeight(w, wdt, N, K), DevAct.empty(Q8, rows, N)
+    gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), start, rows, None), "matmul")
+    assert_same(out.ref()[start:], want[start:], f"matmul K={K} N={N} rows={rows}")
+
+
+@pytest.mark.parametrize("K,N", [(2048, 300), (1280, 44)])
+def test_matmul_f16_row(gpu, oracle, K, N):
+    rng = np.random.default_rng(K)
+    x = rand_act(oracle, rng, F16, 1, K)
+    w = rand_weight(oracle, rng, F16, N, K)
+    want = np.zeros((1, OL.row_bytes(F16, N)), np.uint8)
+    oracle.matmul(OL.ptr(x), F16, OL.ptr(w), F16, OL.ptr(want), F16, K, N, 0, 1, None)
+    dx, dw, out = DevAct(x, F16, 1, K), DevWeight(w, F16, N, K), DevAct.empty(F16, 1, N)
+    gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), 0, 1, None), "matmul")
+    assert_same(out.ref(), want, "matmul f16 row")
+
+
 def test_matmul_in_place(gpu, oracle):
     """Output rows over the input rows: the product is read whole first."""
     rng = np.random.default_rng(17)
@@ -342,6 +384,24 @@ def test_token_embed(gpu, oracle, wdt):
     dtab, dtok, out = DevWeight(table, wdt, vocab, d), dev_array(toks), DevAct.empty(adt, rows, d)
     gpu.check(gpu.lib().nc_token_embed(C.byref(dtab.t), C.c_void_p(dtok.ptr), C.byref(out.t), 0, rows, None), "embed")
     assert_same(out.ref(), want, "token_embed")
+
+
+@pytest.mark.parametrize("n,offset", [(1, 3), (2, 1), (4099, 2), (32771, 3), (40000, 1)])
+@pytest.mark.parametrize("kind", ["ties", "all -inf", "nan"])
+def test_argmax_edges(gpu, oracle, n, offset, kind):
+    """Vectors at any 4-byte alignment, values before and after the vector
+    part, nothing above -inf, NaN never taken."""
+    rng = np.random.default_rng(n + offset)
+    x = rng.integers(-3, 4, n + offset).astype(np.float32)
+    if kind == "all -inf":
+        x[:] = -np.inf
+    if kind == "nan":
+        x[rng.integers(0, n + offset, max(1, n // 3))] = np.nan
+    dx, out = dev_array(x), np.zeros(1, np.int32)
+    dout = dev_array(out)
+    gpu.check(gpu.lib().nc_argmax(C.c_void_p(dx.ptr + 4 * offset), n, C.c_void_p(dout.ptr), None), "argmax")
+    dout.download(out)
+    assert out[0] == oracle.argmax(OL.ptr(np.ascontiguousarray(x[offset:])), n)
 
 
 @pytest.mark.parametrize("n", [1, 1000, 32000, 122753])
