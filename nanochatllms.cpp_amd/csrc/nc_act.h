@@ -52,6 +52,102 @@ __device__ __forceinline__ float act_roundtrip(float v, bool valid)
     return v;
 }
 
+// ---- eight values per lane --------------------------------------------------
+//
+// The same per lane for eight consecutive values 8 c .. 8 c + 7 of a row
+// whose width is a multiple of 32 (Q8; a block on a quad of lanes, all four
+// active) or 8: one 8- or 16-byte access instead of eight, and the block's
+// absmax takes seven in-lane maxima and two lane moves instead of five moves
+// per value.  Rows must be 16-byte aligned (8 for Q8 rows).
+
+template <int ADT>
+__device__ __forceinline__ void act_load8(const uint8_t* row, int c, int dofs, float (&v)[8])
+{
+    if (ADT == Q8) {
+        const uint2 q = reinterpret_cast<const uint2*>(row)[c];
+        const float d = h2f(reinterpret_cast<const uint16_t*>(row + dofs)[c >> 2]);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = (float)(int8_t)((i < 4 ? q.x >> (8 * i) : q.y >> (8 * (i - 4))) & 0xFFu) * d;
+    } else if (ADT == F16) {
+        const uint4 q = reinterpret_cast<const uint4*>(row)[c];
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = h2f((uint16_t)(i & 1 ? w[i >> 1] >> 16 : w[i >> 1] & 0xFFFFu));
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 q = reinterpret_cast<const float4*>(row)[2 * c + h];
+            v[4 * h] = q.x;
+            v[4 * h + 1] = q.y;
+            v[4 * h + 2] = q.z;
+            v[4 * h + 3] = q.w;
+        }
+    }
+}
+
+// q8_quant_lane for a block on four lanes.
+__device__ __forceinline__ void q8_quant8(const float (&v)[8], int8_t (&q)[8], uint16_t* d16)
+{
+    float a = fabsf(v[0]);
+#pragma unroll
+    for (int i = 1; i < 8; i++) a = fmaxf(a, fabsf(v[i]));
+    a = quad_max(a);
+    const float delta = a / 127.0f;
+    *d16 = f2h(delta);
+    const float scale = delta != 0.0f ? 1.0f / delta : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) q[i] = (int8_t)roundf(v[i] * scale);
+}
+
+// Writes v; with BACK, v becomes what is read back.
+template <int ADT, bool BACK = false>
+__device__ __forceinline__ void act_store8(uint8_t* row, int c, int dofs, float (&v)[8])
+{
+    if (ADT == Q8) {
+        int8_t q[8];
+        uint16_t d16;
+        q8_quant8(v, q, &d16);
+        uint32_t w[2] = {0, 0};
+#pragma unroll
+        for (int i = 0; i < 8; i++) w[i >> 2] |= (uint32_t)(uint8_t)q[i] << (8 * (i & 3));
+        reinterpret_cast<uint2*>(row)[c] = make_uint2(w[0], w[1]);
+        if ((c & 3) == 0) reinterpret_cast<uint16_t*>(row + dofs)[c >> 2] = d16;
+        if (BACK) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = (float)q[i] * h2f(d16);
+        }
+    } else if (ADT == F16) {
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[i] = (uint32_t)f2h(v[2 * i]) | (uint32_t)f2h(v[2 * i + 1]) << 16;
+        reinterpret_cast<uint4*>(row)[c] = make_uint4(w[0], w[1], w[2], w[3]);
+        if (BACK) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = f16_roundtrip(v[i]);
+        }
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            reinterpret_cast<float4*>(row)[2 * c + h] = make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
+    }
+}
+
+// act_roundtrip of the eight values.
+template <int ADT>
+__device__ __forceinline__ void act_round8(float (&v)[8])
+{
+    if (ADT == Q8) {
+        int8_t q[8];
+        uint16_t d16;
+        q8_quant8(v, q, &d16);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = (float)q[i] * h2f(d16);
+    } else if (ADT == F16) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = f16_roundtrip(v[i]);
+    }
+}
+
 // (x_j, x_{j+d/2}) -> (x_j cos - x_{j+d/2} sin, x_j sin + x_{j+d/2} cos) on
 // the first d_r dims of a 64-wide head held one value per lane.
 __device__ __forceinline__ float rope_lane(float x, int lane, int d_half, const float2* cs)

@@ -10,6 +10,7 @@
 // (gten/modules.cpp:89-104), so their results equal the unfused op chain.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "nc_act.h"
@@ -145,6 +146,109 @@ __global__ __launch_bounds__(1024) void k_norm(const uint8_t* __restrict__ a, in
     }
 }
 
+// k_norm for segments of a multiple of 256 values in aligned rows: 256 threads
+// of eight values each (two slots past 2048), all of them in the exact sums.
+// What bounds it: the latency of those sums (2-3 us each), so a CU should
+// hold many rows at once; k_norm's 1024 threads, 768 of them waiting, left
+// it two.  Measured (us, 2048 values): rms_norm of Q8 rows, 1 row 6.1 -> 5.1,
+// 512 rows 12.0 -> 6.2, 1500 rows 31 -> 15; layer_norm of fp16 rows, 1500 rows
+// 96 -> 34.
+template <int ADT, int KIND, bool ADD>
+__global__ __launch_bounds__(kSsThreads) void k_norm8(const uint8_t* __restrict__ a, int a_pitch,
+                                                      const float* __restrict__ braw, int b_pitch, float bscale,
+                                                      uint8_t* __restrict__ h_out, int h_pitch,
+                                                      const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
+                                                      uint8_t* __restrict__ out, int out_pitch, int n, int row_cols,
+                                                      float post_scale, const int* __restrict__ dpos)
+{
+    constexpr int kSlots = kNormMaxCols / 8 / kSsThreads;
+    __shared__ __align__(16) float buf[kNormMaxCols];
+    __shared__ SsShared ssh;
+    __shared__ SgShared sgh;
+    const int tid = threadIdx.x, nc8 = n / 8;
+    const int r = blockIdx.y, s8 = blockIdx.x * nc8;  // first chunk of this segment in the row
+    const int dofs = act_delta_offset(row_cols);
+    const size_t prow = dpos ? (size_t)dpos[0] : (size_t)r;
+    const uint8_t* arow = a + prow * a_pitch;
+    uint8_t* orow = out + (size_t)r * out_pitch;
+
+    float xv[kSlots][8];
+#pragma unroll
+    for (int q = 0; q < kSlots; q++) {
+        const int c = tid + q * kSsThreads;
+        if (c >= nc8) break;  // uniform within a lane quad: nc8 is a multiple of 32
+        float (&x)[8] = xv[q];
+        act_load8<ADT>(arow, s8 + c, dofs, x);
+        if (ADD) {
+            float b[8];
+            act_load8<F32>(reinterpret_cast<const uint8_t*>(braw + (size_t)r * b_pitch), s8 + c, 0, b);
+            act_round8<ADT>(b);
+            if (bscale != 1.0f) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) b[i] = b[i] * bscale;
+                act_round8<ADT>(b);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[i] = x[i] + b[i];
+            act_store8<ADT, true>(h_out + prow * h_pitch, s8 + c, dofs, x);
+        }
+        float4* t = reinterpret_cast<float4*>(buf + 8 * c);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            float4 v = make_float4(x[4 * h], x[4 * h + 1], x[4 * h + 2], x[4 * h + 3]);
+            if (KIND == kRms) v = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
+            t[h] = v;
+        }
+    }
+    __syncthreads();
+    float mean = 0.0f;
+    if (KIND == kLayerNorm) {
+        float s1;
+        switch (n / kSsThreads) {
+        case 4: s1 = block_seq_sum_grid<4, kSsThreads>(buf, sgh); break;
+        case 5: s1 = block_seq_sum_grid<5, kSsThreads>(buf, sgh); break;
+        case 6: s1 = block_seq_sum_grid<6, kSsThreads>(buf, sgh); break;
+        case 8: s1 = block_seq_sum_grid<8, kSsThreads>(buf, sgh); break;
+        case 9: s1 = block_seq_sum_grid<9, kSsThreads>(buf, sgh); break;
+        default: s1 = seq_sum(buf, n); break;
+        }
+        mean = s1 / (float)n;
+        __syncthreads();  // the values have been read
+#pragma unroll
+        for (int q = 0; q < kSlots; q++) {
+            const int c = tid + q * kSsThreads;
+            if (c >= nc8) break;
+#pragma unroll
+            for (int i = 0; i < 8; i++) buf[8 * c + i] = (xv[q][i] - mean) * (xv[q][i] - mean);
+        }
+        __syncthreads();
+    }
+    const float ss = block_seq_sum_nonneg(buf, n, ssh);
+    const float denom = KIND == kRms ? sqrtf(ss / (float)n) + 1e-6f : sqrtf(ss / (float)n) + 1e-05f;
+#pragma unroll
+    for (int q = 0; q < kSlots; q++) {
+        const int c = tid + q * kSsThreads;
+        if (c >= nc8) break;
+        float g[8], y[8];
+        act_load8<F16>(reinterpret_cast<const uint8_t*>(w), c, 0, g);
+        if (KIND == kRms) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = xv[q][i] / denom * g[i];
+        } else {
+            float b[8];
+            act_load8<F16>(reinterpret_cast<const uint8_t*>(bias), c, 0, b);
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = ((xv[q][i] - mean) / denom) * g[i] + b[i];
+        }
+        if (post_scale != 1.0f) {
+            act_round8<ADT>(y);
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = y[i] * post_scale;
+        }
+        act_store8<ADT>(orow, s8 + c, dofs, y);
+    }
+}
+
 // ------------------------------------------------------------------- rope --
 
 // rotary_emb (gten/ops.cpp:775-821) on stored activation rows: one
@@ -161,6 +265,47 @@ __global__ __launch_bounds__(64) void k_rope(const uint8_t* __restrict__ in, int
     const float x = act_load<ADT>(in + (size_t)r * in_pitch, e, dofs);
     const float y = rope_lane(x, lane, d_half, table + (size_t)(start + r) * d_half);
     act_store<ADT>(out + (size_t)r * out_pitch, e, dofs, y, true);
+}
+
+// rope_lane for eight values per lane, l = the lane's place among the eight
+// of its 64-wide head, d_half a multiple of 8: the partner values sit in the
+// same registers d_half / 8 lanes away.
+__device__ __forceinline__ void rope8(float (&x)[8], int l, int d_half, const float2* cs)
+{
+    const int nl = d_half >> 3;
+    const bool lo = l < nl, in = l < 2 * nl;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int partner = lo ? lane + nl : (in ? lane - nl : lane);
+    float xp[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) xp[i] = __shfl(x[i], partner);
+    if (!in) return;
+    const float2* t = cs + (lo ? l : l - nl) * 8;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float2 c = t[i];
+        x[i] = lo ? x[i] * c.x - xp[i] * c.y : xp[i] * c.y + x[i] * c.x;
+    }
+}
+
+// k_rope for aligned rows and d_half a multiple of 8, eight values per thread
+// over every (row, chunk): k_rope's one value per thread and 64-thread
+// workgroups were bound by launching them (512 rows x 36 heads Q8: 7.0 ->
+// 4.4 us).
+template <int ADT>
+__global__ __launch_bounds__(256) void k_rope8(const uint8_t* __restrict__ in, int in_pitch, uint8_t* __restrict__ out,
+                                               int out_pitch, int cols, int rows, const float2* __restrict__ table,
+                                               int d_half, int start)
+{
+    const int nc8 = cols >> 3;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int r = t / nc8, c = t - r * nc8;
+    if (r >= rows) return;  // whole heads: nc8 is a multiple of 8
+    const int dofs = act_delta_offset(cols);
+    float x[8];
+    act_load8<ADT>(in + (size_t)r * in_pitch, c, dofs, x);
+    rope8(x, c & 7, d_half, table + (size_t)(start + r) * d_half);
+    act_store8<ADT>(out + (size_t)r * out_pitch, c, dofs, x);
 }
 
 // Decode-step epilogue of the fused q|k|v matvec: per 64-wide head segment
@@ -207,6 +352,42 @@ __global__ __launch_bounds__(64) void k_qkv_post(const float* __restrict__ raw, 
     act_store<ADT>(dst, h * 64 + lane, act_delta_offset(cols), x, true);
 }
 
+// k_qkv_post without q / k norms for aligned rows and d_half a multiple of 8,
+// eight values per thread (512 rows x 108 segments Q8: 15.9 -> 7.5 us).
+template <int ADT, bool BIAS>
+__global__ __launch_bounds__(256) void k_qkv_post8(const float* __restrict__ raw, int raw_pitch, int hq, int hkv,
+                                                   const uint16_t* __restrict__ bq, const uint16_t* __restrict__ bk,
+                                                   const uint16_t* __restrict__ bv, const float2* __restrict__ table,
+                                                   int d_half, int start, int rows, uint8_t* __restrict__ q_out,
+                                                   int q_pitch, uint8_t* __restrict__ k_cache, int k_pitch,
+                                                   uint8_t* __restrict__ v_cache, int v_pitch)
+{
+    const int nc8 = (hq + 2 * hkv) * 8;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int r = t / nc8, c = t - r * nc8;
+    if (r >= rows) return;
+    const int seg = c >> 3, l = c & 7, pos = start + r;
+    const int kind = seg < hq ? 0 : (seg < hq + hkv ? 1 : 2);
+    const int cc = kind == 0 ? c : (kind == 1 ? c - hq * 8 : c - (hq + hkv) * 8);  // chunk within q, k or v
+    float x[8];
+    act_load8<F32>(reinterpret_cast<const uint8_t*>(raw + (size_t)r * raw_pitch), c, 0, x);
+    act_round8<ADT>(x);
+    if (BIAS) {
+        float b[8];
+        act_load8<F16>(reinterpret_cast<const uint8_t*>(kind == 0 ? bq : (kind == 1 ? bk : bv)), cc, 0, b);
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = x[i] + b[i];
+        act_round8<ADT>(x);
+    }
+    if (kind < 2) rope8(x, l, d_half, table + (size_t)pos * d_half);  // uniform within a head's lanes
+    uint8_t* dst;
+    int cols;
+    if (kind == 0) { dst = q_out + (size_t)r * q_pitch; cols = hq * 64; }
+    else if (kind == 1) { dst = k_cache + (size_t)pos * k_pitch; cols = hkv * 64; }
+    else { dst = v_cache + (size_t)pos * v_pitch; cols = hkv * 64; }
+    act_store8<ADT>(dst, cc, act_delta_offset(cols), x);
+}
+
 // ------------------------------------------------------------ elementwise --
 
 enum EwOp { kSilu = 0, kMul = 1, kAdd = 2, kScale = 3, kBias = 4 };
@@ -233,6 +414,32 @@ __global__ __launch_bounds__(256) void k_ew(const uint8_t* __restrict__ a, int a
     act_store<ADT>(out + (size_t)r * out_pitch, e, dofs, y, valid);
 }
 
+// k_ew for aligned rows of whole blocks, eight values per thread over every
+// (row, chunk).
+template <int ADT, int OP>
+__global__ __launch_bounds__(256) void k_ew8(const uint8_t* __restrict__ a, int a_pitch, const uint8_t* __restrict__ b,
+                                             int b_pitch, const uint16_t* __restrict__ bias, float s,
+                                             uint8_t* __restrict__ out, int out_pitch, int cols, int rows)
+{
+    const int nc8 = cols >> 3;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int r = t / nc8, c = t - r * nc8;
+    if (r >= rows) return;  // whole quads: Q8 rows have a multiple of 4 chunks
+    const int dofs = act_delta_offset(cols);
+    float x[8], y[8];
+    act_load8<ADT>(a + (size_t)r * a_pitch, c, dofs, x);
+    if (OP == kMul || OP == kAdd) act_load8<ADT>(b + (size_t)r * b_pitch, c, dofs, y);
+    if (OP == kBias) act_load8<F16>(reinterpret_cast<const uint8_t*>(bias), c, 0, y);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        if (OP == kSilu) x[i] = x[i] / (1.0f + expf_ref(-x[i]));
+        else if (OP == kMul) x[i] = x[i] * y[i];
+        else if (OP == kScale) x[i] = x[i] * s;
+        else x[i] = x[i] + y[i];
+    }
+    act_store8<ADT>(out + (size_t)r * out_pitch, c, dofs, x);
+}
+
 // Decode-step SwiGLU from the fused gate|up matvec output [gate | up]:
 // gate and up requantized as Linear outputs, SiLU in place (requantized),
 // multiply in place (requantized) -- ffn_forward, tinyllama/tinyllama.cpp:88-97.
@@ -249,6 +456,30 @@ __global__ __launch_bounds__(256) void k_silu_mul(const float* __restrict__ raw,
     const float gs = act_roundtrip<ADT>(g / (1.0f + expf_ref(-g)), valid);
     const float u = act_roundtrip<ADT>(rr[f + ec], valid);
     act_store<ADT>(out + (size_t)r * out_pitch, e, act_delta_offset(f), gs * u, valid);
+}
+
+// k_silu_mul for aligned rows of whole blocks, eight values per thread (512
+// rows x 5760 Q8: 19.0 -> 10.9 us).
+template <int ADT>
+__global__ __launch_bounds__(256) void k_silu_mul8(const float* __restrict__ raw, int raw_pitch, int f,
+                                                   uint8_t* __restrict__ out, int out_pitch, int rows)
+{
+    const int nc8 = f >> 3;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int r = t / nc8, c = t - r * nc8;
+    if (r >= rows) return;
+    const uint8_t* rr = reinterpret_cast<const uint8_t*>(raw + (size_t)r * raw_pitch);
+    float g[8], u[8];
+    act_load8<F32>(rr, c, 0, g);
+    act_load8<F32>(rr, nc8 + c, 0, u);
+    act_round8<ADT>(g);
+#pragma unroll
+    for (int i = 0; i < 8; i++) g[i] = g[i] / (1.0f + expf_ref(-g[i]));
+    act_round8<ADT>(g);
+    act_round8<ADT>(u);
+#pragma unroll
+    for (int i = 0; i < 8; i++) g[i] = g[i] * u[i];
+    act_store8<ADT>(out + (size_t)r * out_pitch, c, act_delta_offset(f), g);
 }
 
 // -------------------------------------------------------------- embedding --
@@ -410,6 +641,26 @@ int write_rows(const float* in, int in_pitch, uint8_t* out, int out_pitch, int d
     return launch_status("k_write_rows");
 }
 
+// Whether rows (a base and a pitch in bytes) can be accessed eight values at
+// a time (act_load8).
+static bool act_vec(int dtype, const void* p, int pitch)
+{
+    const uintptr_t m = dtype == NC_Q8 ? 7 : 15;
+    return (((uintptr_t)p | (uintptr_t)(unsigned)pitch) & m) == 0;
+}
+
+// Whether rows of `cols` values split into lane-held chunks of eight (whole
+// Q8 blocks), and the workgroups of one chunk per thread.
+static bool rows8(int dtype, int cols) { return cols % (dtype == NC_Q8 ? 32 : 8) == 0; }
+static unsigned grid8(int rows, int cols) { return (unsigned)(((int64_t)rows * (cols / 8) + 255) / 256); }
+static bool fits8(int rows, int cols) { return (int64_t)rows * cols < ((int64_t)1 << 31); }
+// Values from which eight per thread win (us, one value per thread against
+// eight, Q8 rows): add 90K values 2.4 / 2.3, 360K 2.7 / 2.4, 1.2M 4.3 / 3.2, 3.1M
+// 8.1 / 4.3; rotary embedding 2.5 / 3.0, 3.6 / 3.1, 7.0 / 4.4, 13.7 / 6.2; with
+// an exponential (eight in turn per thread) 360K 3.0 / 3.8, 1.2M 5.0 / 5.0, 3.1M
+// 9.1 / 7.4.
+constexpr int kEw8Min = 1 << 18, kSilu8Min = 1 << 20;
+
 // Threads per norm workgroup: the largest multiple of 64 up to 1024 that
 // divides the segment (each thread then owns n / bs values).
 static int norm_block(int n)
@@ -429,6 +680,29 @@ int norm_launch(int kind, int adt, bool add, const uint8_t* a, int a_pitch, cons
         return fail(NC_ERR_ARG, "norm: unsupported size %d (row %d)", d_norm, row_cols);
     if (adt != NC_Q8 && adt != NC_F16) return fail(NC_ERR_ARG, "norm: activation dtype %d", adt);
     const dim3 grid(row_cols / d_norm, rows);
+    // eight values per thread where the widths and every row's alignment allow
+    const bool vec = d_norm % kSsThreads == 0 && act_vec(adt, a, a_pitch) && act_vec(adt, out, out_pitch) &&
+                     act_vec(NC_F16, w, 0) && (kind == kRms || act_vec(NC_F16, bias, 0)) &&
+                     (!add || (act_vec(NC_F32, braw, b_pitch * 4) && act_vec(adt, h_out, h_pitch)));
+    if (vec) {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(kSsThreads), 0, st, a, a_pitch, braw, b_pitch, bscale, h_out, h_pitch, w,
+                               bias, out, out_pitch, d_norm, row_cols, post_scale, dpos);
+        };
+        auto by_kind = [&](auto t) {
+            constexpr int ADT = decltype(t)::value;
+            if (kind == kRms) {
+                if (add) go(k_norm8<ADT, kRms, true>);
+                else go(k_norm8<ADT, kRms, false>);
+            } else {
+                if (add) go(k_norm8<ADT, kLayerNorm, true>);
+                else go(k_norm8<ADT, kLayerNorm, false>);
+            }
+        };
+        if (adt == NC_Q8) by_kind(std::integral_constant<int, Q8>{});
+        else by_kind(std::integral_constant<int, F16>{});
+        return launch_status("k_norm8");
+    }
 #define NORM_CALL(K, A)                                                                                           \
     hipLaunchKernelGGL((k_norm<ADT, K, A>), grid, dim3(bs), 0, st, a, a_pitch, braw, b_pitch, bscale, h_out, h_pitch, \
                        w, bias, out, out_pitch, d_norm, row_cols, post_scale, dpos)
@@ -453,6 +727,20 @@ int qkv_post_launch(int adt, const float* raw, int raw_pitch, int hq, int hkv, c
     if (rows <= 0) return NC_OK;
     const dim3 grid(hq + 2 * hkv, rows);
     const bool bias = bq != nullptr, qkn = qn_w != nullptr;
+    if (!qkn && !dpos && d_half % 8 == 0 && (adt == NC_Q8 || adt == NC_F16) && fits8(rows, (hq + 2 * hkv) * 64) &&
+        (int64_t)rows * (hq + 2 * hkv) * 64 >= kEw8Min &&
+        act_vec(NC_F32, raw, raw_pitch * 4) && act_vec(adt, q_out, q_pitch) && act_vec(adt, k_cache, k_pitch) &&
+        act_vec(adt, v_cache, v_pitch) &&
+        (!bias || (act_vec(NC_F16, bq, 0) && act_vec(NC_F16, bk, 0) && act_vec(NC_F16, bv, 0)))) {
+        const dim3 g8(grid8(rows, (hq + 2 * hkv) * 64));
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, g8, dim3(256), 0, st, raw, raw_pitch, hq, hkv, bq, bk, bv, (const float2*)table,
+                               d_half, start, rows, q_out, q_pitch, k_cache, k_pitch, v_cache, v_pitch);
+        };
+        if (adt == NC_Q8) { if (bias) go(k_qkv_post8<Q8, true>); else go(k_qkv_post8<Q8, false>); }
+        else { if (bias) go(k_qkv_post8<F16, true>); else go(k_qkv_post8<F16, false>); }
+        return launch_status("k_qkv_post8");
+    }
 #define QKV_CALL(B, N)                                                                                              \
     hipLaunchKernelGGL((k_qkv_post<ADT, B, N>), grid, dim3(64), 0, st, raw, raw_pitch, hq, hkv, bq, bk, bv, qn_w, kn_w, \
                        (const float2*)table, d_half, start, q_out, q_pitch, k_cache, k_pitch, v_cache, v_pitch, dpos)
@@ -475,6 +763,14 @@ int silu_mul_launch(int adt, const float* raw, int raw_pitch, int f, uint8_t* ou
                     hipStream_t st)
 {
     if (rows <= 0) return NC_OK;
+    if ((adt == NC_Q8 || adt == NC_F16) && rows8(adt, f) && fits8(rows, f) && (int64_t)rows * f >= kSilu8Min &&
+        act_vec(NC_F32, raw, raw_pitch * 4) &&
+        act_vec(adt, out, out_pitch)) {
+        const dim3 g8(grid8(rows, f));
+        if (adt == NC_Q8) hipLaunchKernelGGL((k_silu_mul8<Q8>), g8, dim3(256), 0, st, raw, raw_pitch, f, out, out_pitch, rows);
+        else hipLaunchKernelGGL((k_silu_mul8<F16>), g8, dim3(256), 0, st, raw, raw_pitch, f, out, out_pitch, rows);
+        return launch_status("k_silu_mul8");
+    }
     const dim3 grid((f + 255) / 256, rows);
     if (adt == NC_Q8) hipLaunchKernelGGL((k_silu_mul<Q8>), grid, dim3(256), 0, st, raw, raw_pitch, f, out, out_pitch);
     else if (adt == NC_F16) hipLaunchKernelGGL((k_silu_mul<F16>), grid, dim3(256), 0, st, raw, raw_pitch, f, out, out_pitch);
@@ -522,6 +818,22 @@ int ew_launch(int op, int adt, const uint8_t* a, int a_pitch, const uint8_t* b, 
               float s, uint8_t* out, int out_pitch, int cols, int rows, hipStream_t st)
 {
     if (rows <= 0) return NC_OK;
+    if (rows8(adt, cols) && fits8(rows, cols) && (int64_t)rows * cols >= (op == kSilu ? kSilu8Min : kEw8Min) && act_vec(adt, a, a_pitch) &&
+        act_vec(adt, out, out_pitch) && (!b || act_vec(adt, b, b_pitch)) && (!bias || act_vec(NC_F16, bias, 0))) {
+        const dim3 g8(grid8(rows, cols));
+#define EW8_CALL(OPV) hipLaunchKernelGGL((k_ew8<ADT, OPV>), g8, dim3(256), 0, st, a, a_pitch, b, b_pitch, bias, s, out, out_pitch, cols, rows)
+        NC_ADT_DISPATCH(adt, {
+            switch (op) {
+            case kSilu: EW8_CALL(kSilu); break;
+            case kMul: EW8_CALL(kMul); break;
+            case kAdd: EW8_CALL(kAdd); break;
+            case kScale: EW8_CALL(kScale); break;
+            default: EW8_CALL(kBias); break;
+            }
+        });
+#undef EW8_CALL
+        return launch_status("k_ew8");
+    }
     const dim3 grid((cols + 255) / 256, rows);
 #define EW_CALL(OPV) hipLaunchKernelGGL((k_ew<ADT, OPV>), grid, dim3(256), 0, st, a, a_pitch, b, b_pitch, bias, s, out, out_pitch, cols)
     NC_ADT_DISPATCH(adt, {
@@ -542,6 +854,11 @@ int rope_launch(int adt, const uint8_t* in, int in_pitch, uint8_t* out, int out_
 {
     if (rows <= 0) return NC_OK;
     if (cols % 64) return fail(NC_ERR_ARG, "rotary_emb: width %d is not a multiple of the 64-wide head", cols);
+    if (d_half % 8 == 0 && fits8(rows, cols) && (int64_t)rows * cols >= kEw8Min && act_vec(adt, in, in_pitch) && act_vec(adt, out, out_pitch)) {
+        NC_ADT_DISPATCH(adt, hipLaunchKernelGGL((k_rope8<ADT>), dim3(grid8(rows, cols)), dim3(256), 0, st, in, in_pitch,
+                                                out, out_pitch, cols, rows, (const float2*)table, d_half, start));
+        return launch_status("k_rope8");
+    }
     const dim3 grid(cols / 64, rows);
     NC_ADT_DISPATCH(adt, hipLaunchKernelGGL((k_rope<ADT>), grid, dim3(64), 0, st, in, in_pitch, out, out_pitch, cols,
                                             (const float2*)table, d_half, start));

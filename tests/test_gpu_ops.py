@@ -237,6 +237,61 @@ def test_rms_norm(gpu, oracle, dt, d, scale):
 
 
 @pytest.mark.parametrize("dt", [Q8, F16])
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+@pytest.mark.parametrize("d,shift", [(256, 0), (1024, 0), (1280, 0), (1536, 0), (2304, 0), (3072, 0), (4096, 0),
+                                     (2048, 2), (320, 0)])
+def test_norm_widths(gpu, oracle, dt, kind, d, shift):
+    """Every width the eight-value norm takes (one and two slots per thread,
+    means with and without the exact grid sum), a width it leaves to the other
+    kernel, and gains at an address it does not take (shift bytes)."""
+    rng = np.random.default_rng(d + shift)
+    rows, start = 3, 1
+    x = rand_act(oracle, rng, dt, rows, d, 3.0)
+    w = (1 + 0.2 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
+    b = (0.1 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
+    want = np.zeros_like(x)
+    dx, out = DevAct(x, dt, rows, d), DevAct.empty(dt, rows, d)
+    pad = np.zeros(shift // 2, np.uint16)
+    dw_, db_ = dev_array(np.concatenate([pad, w])), dev_array(b)
+    L = gpu.lib()
+    if kind == "rms":
+        oracle.rms_norm(OL.ptr(x), dt, OL.ptr(w), OL.ptr(want), d, start, rows)
+        st = L.nc_rms_norm(C.byref(dx.t), C.c_void_p(dw_.ptr + shift), C.byref(out.t), d, start, rows, None)
+    else:
+        oracle.layer_norm(OL.ptr(x), dt, OL.ptr(w), OL.ptr(b), OL.ptr(want), d, start, rows)
+        st = L.nc_layer_norm(C.byref(dx.t), C.c_void_p(dw_.ptr + shift), C.c_void_p(db_.ptr), C.byref(out.t), start,
+                             rows, None)
+    gpu.check(st, "norm")
+    assert_same(out.ref()[start:], want[start:], f"{kind} norm of {d}")
+
+
+@pytest.mark.parametrize("dt", [Q8, F16])
+@pytest.mark.parametrize("op", ["silu", "mul", "add", "rope"])
+@pytest.mark.parametrize("d,rows", [(2048, 515), (2112, 510)])
+def test_elementwise_many_rows(gpu, oracle, dt, op, d, rows):
+    """Enough values for eight per thread, a last workgroup that is not full."""
+    rng = np.random.default_rng(d + rows)
+    a, b = rand_act(oracle, rng, dt, rows, d, 4.0), rand_act(oracle, rng, dt, rows, d, 1.0)
+    want = a.copy()
+    da, db_, out = DevAct(a, dt, rows, d), DevAct(b, dt, rows, d), DevAct.empty(dt, rows, d)
+    L = gpu.lib()
+    if op == "silu":
+        oracle.silu(OL.ptr(a), OL.ptr(want), dt, d, 0, rows)
+        st = L.nc_silu(C.byref(da.t), C.byref(out.t), 0, rows, None)
+    elif op == "rope":
+        tab = np.zeros((rows, 8, 2), np.float32)
+        gpu.check(L.nc_rope_table(rows, 64, 0.25, ptr(tab)), "rope_table")
+        dtab = dev_array(tab)
+        oracle.rotary_emb(OL.ptr(a), OL.ptr(want), dt, d, 64, 0.25, 0, rows)
+        st = L.nc_rotary_emb(C.byref(da.t), C.byref(out.t), 64, 0.25, C.c_void_p(dtab.ptr), 0, rows, None)
+    else:
+        (oracle.multiply if op == "mul" else oracle.add)(OL.ptr(a), OL.ptr(b), OL.ptr(want), dt, d, 0, rows)
+        st = (L.nc_multiply if op == "mul" else L.nc_add)(C.byref(da.t), C.byref(db_.t), C.byref(out.t), 0, rows, None)
+    gpu.check(st, op)
+    assert_same(out.ref(), want, op)
+
+
+@pytest.mark.parametrize("dt", [Q8, F16])
 def test_rms_norm_per_head(gpu, oracle, dt):
     rng = np.random.default_rng(5)
     rows, heads = 3, 20
