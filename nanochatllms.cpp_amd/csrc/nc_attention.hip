@@ -558,6 +558,226 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_rows(const uint8_t* __res
         act_store<ADT>(out + (size_t)(qr0 + i) * out_pitch, h * 64 + lane, qd, outs[i][lane], true);
 }
 
+// ---- sixteen fp16 query rows per workgroup, on the matrix cores --------------
+//
+// The products of fp16 values are exact in fp32, so one K step of
+// v_mfma_f32_16x16x1_4b_f32 is the reference's multiply then add for every
+// entry of a 16 x 16 tile (see k_mfma_f16), its four blocks four of the eight
+// lane chains:
+//   scores: lanes j of the 64-value dot (K steps its 8-wide chunks), tile =
+//           16 query rows x 16 positions; one thread ends up with all eight
+//           chains of its four scores;
+//   P.V:    lanes l = position mod 8 (K steps position / 8), tile = 16 query
+//           rows x 16 columns; wavefront (column group, chain half) runs one
+//           accumulator over all positions in order.
+// Positions past the first row's (which some rows do not attend) are added on
+// the vector unit, row by row, so a masked value never enters a product.
+//
+// What bounds it: per 16 x 16 scores 512 cycles of products on one SIMD
+// against 2048 on its vector unit before, then the chain of P.V products (32
+// cycles per 8 positions), the softmax's sequential sums (two rows side by
+// side on the halves of a wavefront) and its exponentials.  Shared memory
+// holds 16 rows of scores, so contexts past kFaMaxCtx keep k_attn_rows.
+// Measured (us): 1500 rows x 32 heads 792 -> 365, 2100 rows 1815 -> 654, 512
+// rows x 36 heads 82 -> 55, 100 rows after 600 61.6 -> 30.2; 128 rows 14.6 -> 13.7,
+// but 64 rows 7.7 -> 11.4, so shorter contexts keep k_attn_rows too.
+typedef float f16x_t __attribute__((ext_vector_type(16)));
+constexpr int kFaThreads = 512;
+constexpr int kFaRows = 16;
+constexpr int kFaChunk = 128;   // positions of K or V staged at a time
+constexpr int kFaStride = 144;  // bytes per staged position: 128 and a pad that spreads the banks
+constexpr int kFaMinCtx = 128, kFaMaxCtx = 2176;
+
+// Floats per row of scores: a multiple of 64 and 4 more, so that 16 rows x 4
+// positions fall in 64 banks.
+__host__ __device__ constexpr int fa_row(int m) { return ((m + 63) & ~63) + 4; }
+constexpr size_t fa_lds(int m) { return (size_t)kFaRows * fa_row(m) * 4 + kFaChunk * kFaStride + 4 * 16 * 16 * 4; }
+static_assert(fa_lds(kFaMaxCtx) <= 160 * 1024, "shared memory of a CU");
+
+__global__ __launch_bounds__(kFaThreads) void k_attn_f16(const uint8_t* __restrict__ q, int q_pitch,
+                                                         const uint8_t* __restrict__ kc, int k_pitch,
+                                                         const uint8_t* __restrict__ vc, int v_pitch,
+                                                         uint8_t* __restrict__ out, int out_pitch, int hq, int hkv,
+                                                         int start, int n_ctx, int rows, float scale)
+{
+    extern __shared__ __align__(16) float sm[];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lc = lane & 15, lb = lane >> 4;
+    // the longest row groups are dispatched first
+    const int h = blockIdx.x, qr0 = (gridDim.y - 1 - blockIdx.y) * kFaRows;
+    const int nr = min(kFaRows, rows - qr0);
+    const int m = start + qr0 + nr;  // positions attended by any of the rows
+    const int ms = fa_row(m);
+    float* S = sm;                                                  // [16][ms]
+    uint8_t* buf = reinterpret_cast<uint8_t*>(S + kFaRows * ms);    // [kFaChunk][kFaStride]
+    float* part = reinterpret_cast<float*>(buf + kFaChunk * kFaStride);  // [4][16][16]
+    const int g = h / (hq / hkv);
+    const int nch = (m + kFaChunk - 1) / kFaChunk;
+
+    // the thread's part of a chunk: 32 bytes of one position's head slice
+    const int s_pos = tid >> 2, s_t = tid & 3;
+    uint4 in[2];
+    auto load = [&](const uint8_t* base, int pitch, int ch) {
+        const int c = min(ch * kFaChunk + s_pos, m - 1);
+        const uint4* p = reinterpret_cast<const uint4*>(base + (size_t)c * pitch + g * 128) + 2 * s_t;
+        in[0] = p[0];
+        in[1] = p[1];
+    };
+
+    // ---- scores
+    {
+        float qa[2][8];  // lane j = 4 hh + lb of this thread's row, chunk v
+        const uint32_t* qrow =
+            reinterpret_cast<const uint32_t*>(q + (size_t)(qr0 + min(lc, nr - 1)) * q_pitch + h * 128);
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++)
+#pragma unroll
+            for (int v = 0; v < 8; v++) {
+                const uint32_t d = qrow[v * 4 + 2 * hh + (lb >> 1)];
+                qa[hh][v] = h2f((uint16_t)(lb & 1 ? d >> 16 : d & 0xFFFFu));
+            }
+        load(kc, k_pitch, 0);
+        for (int ch = 0; ch < nch; ch++) {
+            lds_barrier();  // the previous chunk has been read
+            // staged as [position][lane j][chunk v]
+            {
+                const uint32_t a[4] = {in[0].x, in[0].y, in[0].z, in[0].w}, b[4] = {in[1].x, in[1].y, in[1].z, in[1].w};
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    *reinterpret_cast<uint32_t*>(buf + s_pos * kFaStride + j * 16 + s_t * 4) =
+                        __builtin_amdgcn_perm(b[j >> 1], a[j >> 1], j & 1 ? 0x07060302u : 0x05040100u);
+            }
+            load(ch + 1 < nch ? kc : vc, ch + 1 < nch ? k_pitch : v_pitch, ch + 1 < nch ? ch + 1 : 0);
+            lds_barrier();
+            const int p0 = ch * kFaChunk + 16 * w;
+            if (p0 < m) {  // uniform per wavefront
+                float kb[2][8];
+#pragma unroll
+                for (int hh = 0; hh < 2; hh++) {
+                    const uint4 u =
+                        *reinterpret_cast<const uint4*>(buf + (16 * w + lc) * kFaStride + (4 * hh + lb) * 16);
+                    const uint32_t d[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                    for (int v = 0; v < 8; v++) kb[hh][v] = h2f((uint16_t)(v & 1 ? d[v >> 1] >> 16 : d[v >> 1] & 0xFFFFu));
+                }
+                f16x_t acc[2];
+#pragma unroll
+                for (int hh = 0; hh < 2; hh++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[hh][e] = 0.0f;
+#pragma unroll
+                for (int v = 0; v < 8; v++)
+#pragma unroll
+                    for (int hh = 0; hh < 2; hh++)
+                        acc[hh] = __builtin_amdgcn_mfma_f32_16x16x1f32(qa[hh][v], kb[hh][v], acc[hh], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float s = acc[0][i];
+#pragma unroll
+                    for (int j = 1; j < 8; j++) s = s + acc[j >> 2][(j & 3) * 4 + i];
+                    if (p0 + lc < m) S[(4 * lb + i) * ms + p0 + lc] = s * scale;
+                }
+            }
+        }
+    }
+    lds_barrier();  // the scores are there, the K chunk has been read
+    // V chunk 0 (requested with the last K chunk), staged as it lies
+    auto store_v = [&]() {
+        uint4* d = reinterpret_cast<uint4*>(buf + s_pos * kFaStride) + 2 * s_t;
+        d[0] = in[0];
+        d[1] = in[1];
+    };
+    store_v();
+    if (nch > 1) load(vc, v_pitch, 1);
+
+    // ---- softmax: rows w and w + 8 on the halves of wavefront w, as in
+    // k_attn_rows
+    {
+        const int hl = lane & 31, i = w + 8 * (lane >> 5);
+        const int n = i < nr ? start + qr0 + i + 1 : 0;
+        float* Si = S + i * ms;
+        float mx = -INFINITY;
+        for (int c = hl; c < n; c += 32) mx = fmaxf(mx, Si[c]);
+#pragma unroll
+        for (int o = 16; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+        for (int c = hl; c < n; c += 32) Si[c] = expf_ref(Si[c] - mx);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        const float sum = seq_sum(Si, n);
+        for (int c = hl; c < n; c += 32) Si[c] = f16_roundtrip(Si[c] / sum);
+    }
+    lds_barrier();
+
+    // ---- P.V: wavefront (column group dg, chain half hh)
+    const int dg = w >> 1, hh = w & 1;
+    const int n8 = (n_ctx / 8) * 8;
+    const int lim_max = min(m, n8);
+    const int lim_all = min(start + qr0 + 1, n8) & ~7;  // every row attends the positions before it
+    const uint8_t* vcol = buf + (16 * dg + lc) * 2;
+    auto v_at = [&](int r) { return h2f(*reinterpret_cast<const uint16_t*>(vcol + r * kFaStride)); };
+    f16x_t acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+    for (int ch = 0; ch < nch; ch++) {
+        const int c0 = ch * kFaChunk;
+        if (ch) {
+            lds_barrier();  // chunk ch - 1 has been read
+            store_v();
+            if (ch + 1 < nch) load(vc, v_pitch, ch + 1);
+            lds_barrier();
+        }
+        const int cend = min(c0 + kFaChunk, lim_all);
+        const float* P = S + lc * ms + 4 * hh + lb;
+        int c = c0;
+        for (; c + 64 <= cend; c += 64) {
+            float pa[8], vb[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                pa[u] = P[c + 8 * u];
+                vb[u] = v_at(c + 8 * u - c0 + 4 * hh + lb);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(pa[u], vb[u], acc, 0, 0, 0);
+        }
+        for (; c < cend; c += 8)
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(P[c], v_at(c - c0 + 4 * hh + lb), acc, 0, 0, 0);
+        // positions that not every row attends (at most three steps of 8)
+        for (c = max(c0, lim_all); c < min(c0 + kFaChunk, lim_max); c += 8)
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const int p = c + 4 * hh + b;
+                const float v = v_at(p - c0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int row = 4 * lb + i;
+                    if (p < min(start + qr0 + row + 1, n8)) acc[4 * b + i] = S[row * ms + p] * v + acc[4 * b + i];
+                }
+            }
+    }
+    // the eight chains left to right, then the tail [n8, n) in order (within
+    // the last chunk, still staged)
+    if (hh == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) part[(dg * 16 + 4 * lb + i) * 16 + lc] = acc[i] + acc[4 + i] + acc[8 + i] + acc[12 + i];
+    }
+    lds_barrier();
+    if (hh == 1) {
+        const int c0 = (nch - 1) * kFaChunk;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 4 * lb + i;
+            float t = part[(dg * 16 + row) * 16 + lc];
+#pragma unroll
+            for (int b = 0; b < 4; b++) t = t + acc[4 * b + i];
+            if (row < nr) {
+                for (int c = n8; c < start + qr0 + row + 1; c++) t = t + S[row * ms + c] * v_at(c - c0);
+                reinterpret_cast<uint16_t*>(out + (size_t)(qr0 + row) * out_pitch)[h * 64 + 16 * dg + lc] = f2h(t);
+            }
+        }
+    }
+}
+
 // ---- launchers -------------------------------------------------------------
 
 template <int ADT>
@@ -586,6 +806,12 @@ int attn_go(const uint8_t* q, int q_pitch, const uint8_t* kc, int k_pitch, const
         // prefill: several query rows per workgroup, fewer for long rows
         // (their scores stay within 32 KB of shared memory)
         const int m = n_ctx;  // the last group attends at most n_ctx positions
+        if (ADT == F16 && m >= kFaMinCtx && m <= kFaMaxCtx) {
+            const dim3 grid(hq, (rows + kFaRows - 1) / kFaRows);
+            hipLaunchKernelGGL(k_attn_f16, grid, dim3(kFaThreads), fa_lds(m), st, q, q_pitch, kc, k_pitch, vc, v_pitch,
+                               out, out_pitch, hq, hkv, start, n_ctx, rows, scale);
+            return launch_status("k_attn_f16");
+        }
         auto go_rows = [&](auto kern, size_t lds, int R) {
             const dim3 grid(hq, (rows + R - 1) / R);
             hipLaunchKernelGGL(kern, grid, dim3(kAttnThreads), lds, st, q, q_pitch, kc, k_pitch, vc, v_pitch, out,

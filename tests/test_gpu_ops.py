@@ -409,6 +409,16 @@ ATTN_CASES = [
     (F16, 32, 32, 4096, 4095),
     (F16, 4, 4, 4090, 4081),
     (F16, 4, 2, 1500, 0),
+    # several fp16 rows on the matrix cores: one tile and parts of it, rows
+    # across a tile's and a chunk's edge, every n mod 8, the longest context
+    # it takes and the next
+    (F16, 2, 1, 2, 0),
+    (F16, 2, 2, 129, 112),
+    (F16, 4, 2, 143, 5),
+    (F16, 2, 1, 257, 240),
+    (F16, 3, 1, 383, 350),
+    (F16, 2, 2, 2176, 2170),
+    (F16, 2, 2, 2177, 2170),
 ]
 
 
