@@ -23,9 +23,10 @@
 //
 // Three quarters of each activation operand are zeros: the matrix cores do
 // four times the necessary integer work, which is cheap next to the
-// vector-unit fold (13 fp32 operations per output and block).  k_gemm_qh
+// vector-unit fold (13 fp32 operations per output and block).  k_gemm_qw
 // (below) takes the same lane sums on the fp16 matrix cores and reads the
-// weights' chunk-major copy when the caller has one.
+// weights' chunk-major copy when the caller has one; this kernel keeps the
+// products it does not take (K not a multiple of 128).
 #include <hip/hip_ext.h>
 
 #include <type_traits>
@@ -227,7 +228,6 @@ __device__ __forceinline__ void bytes_to_h(uint32_t u, uint32_t bias2, uint32_t&
     hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, b) + bb);
 }
 constexpr uint32_t kHm1152 = 0xE480E480u;  // fp16 -1152, twice: (1024 + c + 128) - 1152 = c
-constexpr uint32_t kHm1031 = 0xE407E407u;  // fp16 -1031, twice: (1024 + n) - 1031 = n - 7
 
 // Four signed int8 codes -> four fp16 values (two dwords).
 __device__ __forceinline__ void s8x4_to_h(uint32_t v, uint32_t& lo, uint32_t& hi)
@@ -246,274 +246,23 @@ __device__ __forceinline__ void s8x4_to_h16(uint32_t v, uint32_t& lo, uint32_t& 
     hi = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2_t, b), sc, off));
 }
 
-// NW wavefronts per workgroup share the staged activation blocks of 4 MR
-// rows and own 16 weight columns each; a chunk is CH blocks (one LDS barrier
-// per chunk), and PF chunks of weights and activation blocks are in flight.
-// Within a chunk the MFMAs of block j + 1 are issued before the folds of
-// block j, so no fold waits on the MFMA just issued.  CL: the weights are
-// read from their chunk-major copy (k_chunk_layout), where a wavefront's
-// codes of four blocks are one contiguous 1 KB (Q4) and a thread's are one
-// 16-byte load, instead of four 4-byte loads from 16 rows each.  WPE: the
-// wavefronts per SIMD the registers are allotted for (the fold is
-// vector-unit work and needs wavefronts beside each other to cover its
-// latencies).
-template <int WT, int MR, int NW, int CH, int PF, bool CL, int WPE = 1>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) void k_gemm_qh(
-        const uint8_t* __restrict__ x, int x_pitch, int n_rows, const uint32_t* __restrict__ wq,
-        const uint16_t* __restrict__ wd, float* __restrict__ out, int out_pitch, int N, int nb)
-{
-    constexpr int WV = WT == Q4 ? 1 : 2;  // code dwords of one lane of a weight block
-    constexpr int WD = WT == Q4 ? 4 : 8;  // code dwords per weight block
-    constexpr int kRows = 4 * MR;         // rows per workgroup
-    constexpr int kThreads = 64 * NW;
-    static_assert(CH == 4 || CH == 8, "chunk of 4 or 8 blocks (one 8- or 16-byte delta load)");
-    // expanded activation operands [buffer][block][row group][lane] and the
-    // rows' deltas [buffer][block][row]
-    __shared__ __align__(16) uint4 xa[2][CH][MR][64];
-    __shared__ float xd[2][CH][kRows];
-    // CI (the long-prompt Q4 shape: chunk-major copy, at most 8 rows, one
-    // chunk in flight): the products' accumulator start per (block, row,
-    // lane k), -1031 x (sum of the lane's eight activation codes), and raw
-    // weight codes 1024 + n (four conversions fewer per block; the other
-    // shapes have no registers for the starts)
-    constexpr bool CI = WT == Q4 && CL && MR <= 2 && PF == 1;
-    __shared__ __align__(16) float xc[CI ? 2 : 1][CH][kRows][4];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int lc = lane & 15, lg = lane >> 4;
-    const int r0 = blockIdx.y * kRows;
-    const int col = min(blockIdx.x * 16 * NW + wv * 16 + lc, N - 1);  // this thread's weight column
-    const int nch = nb / CH;
-
-    // zero entries: lane l = lc + 16 lg with lg != lc % 4, never staged
-    for (int e = tid; e < 2 * CH * MR * 64; e += kThreads)
-        if (((e & 15) & 3) != ((e >> 4) & 3)) (&xa[0][0][0][0])[e] = make_uint4(0, 0, 0, 0);
-
-    // staging, spread over every thread: a task is one AVX lane k of one
-    // (row, block) of the chunk -- its eight codes as fp16 (16 bytes) -- and
-    // lane 0's task also stages the block's delta.  Rows past the end repeat
-    // the last row (their outputs are not stored).
-    constexpr int kTasks = 4 * kRows * CH;
-    constexpr int TPT = (kTasks + kThreads - 1) / kThreads;  // tasks per thread
-    struct XLane {
-        uint32_t d[4];  // dwords k/2, 2 + k/2, 4 + k/2, 6 + k/2 of the block
-        uint16_t d16;
-    };
-    int t_row[TPT], t_blk[TPT], t_k[TPT];
-    const uint8_t* t_src[TPT];
-#pragma unroll
-    for (int i = 0; i < TPT; i++) {
-        const int t = min(tid + i * kThreads, kTasks - 1);  // surplus slots repeat the last task
-        t_k[i] = t & 3;
-        t_row[i] = (t >> 2) % kRows;
-        t_blk[i] = (t >> 2) / kRows;
-        t_src[i] = x + (size_t)min(r0 + t_row[i], n_rows - 1) * x_pitch;
-    }
-    auto x_load = [&](int ch, XLane (&q)[TPT]) {
-        const int b0 = min(ch, nch - 1) * CH;
-#pragma unroll
-        for (int i = 0; i < TPT; i++) {
-            const int b = b0 + t_blk[i];
-            const uint32_t* blk = reinterpret_cast<const uint32_t*>(t_src[i] + (size_t)b * 32);
-            const int h = t_k[i] >> 1;
-#pragma unroll
-            for (int v = 0; v < 4; v++) q[i].d[v] = blk[2 * v + h];
-            q[i].d16 = reinterpret_cast<const uint16_t*>(t_src[i] + (size_t)nb * 32)[b];
-        }
-    };
-    auto stage = [&](const XLane (&q)[TPT], int buf) {
-#pragma unroll
-        for (int i = 0; i < TPT; i++) {
-            if (tid + i * kThreads >= kTasks) break;  // uniform per wave: kTasks is a multiple of 64
-            const int k = t_k[i], r = t_row[i], j = t_blk[i];
-            const uint32_t a = pick_pair(q[i].d[0], q[i].d[1], k & 1);
-            const uint32_t bq = pick_pair(q[i].d[2], q[i].d[3], k & 1);
-            uint4 hv;
-            s8x4_to_h(a, hv.x, hv.y);
-            s8x4_to_h(bq, hv.z, hv.w);
-            xa[buf][j][r >> 2][(r & 3) * 4 + k + 16 * k] = hv;
-            if (k == 0) xd[buf][j][r] = h2f(q[i].d16);
-            if constexpr (CI)
-                xc[buf][j][r][k] = -1031.0f * (float)(__builtin_amdgcn_sdot4((int)a, 0x01010101, 0, false) +
-                                                       __builtin_amdgcn_sdot4((int)bq, 0x01010101, 0, false));
-        }
-    };
-
-    const uint32_t* wcol = wq + (size_t)col * nb * WD + WV * lg;
-    const uint16_t* dcol = wd + (size_t)col * nb;
-    struct WChunk {
-        uint32_t c[CH][WV];
-        uint32_t d[CH / 2];  // the chunk's fp16 deltas, two per dword
-    };
-    auto w_load = [&](int ch, WChunk& w) {
-        const int b0 = min(ch, nch - 1) * CH;
-        if constexpr (CL) {
-            // codes [nb/4][N][4 lanes][4 blocks x WV dwords], deltas [nb/4][N][4]
-#pragma unroll
-            for (int h = 0; h < CH / 4; h++) {
-                const size_t c4 = (size_t)(b0 / 4 + h) * N + col;
-                const uint4* src = reinterpret_cast<const uint4*>(wq + (c4 * 4 + lg) * 4 * WV);
-#pragma unroll
-                for (int q = 0; q < WV; q++) {
-                    const uint4 t = src[q];
-                    const uint32_t tv[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-                    for (int e = 0; e < 4; e++) w.c[4 * h + (4 * q + e) / WV][(4 * q + e) % WV] = tv[e];
-                }
-                const uint2 d = *reinterpret_cast<const uint2*>(wd + c4 * 4);
-                w.d[2 * h] = d.x;
-                w.d[2 * h + 1] = d.y;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < CH; j++)
-#pragma unroll
-                for (int v = 0; v < WV; v++) w.c[j][v] = wcol[(size_t)(b0 + j) * WD + v];
-            if constexpr (CH == 4) {
-                const uint2 d = *reinterpret_cast<const uint2*>(dcol + b0);
-                w.d[0] = d.x;
-                w.d[1] = d.y;
-            } else {
-                const uint4 d = *reinterpret_cast<const uint4*>(dcol + b0);
-                w.d[0] = d.x;
-                w.d[1] = d.y;
-                w.d[2] = d.z;
-                w.d[3] = d.w;
-            }
-        }
-    };
-
-    float acc[MR][4];
-#pragma unroll
-    for (int m = 0; m < MR; m++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) acc[m][k] = 0.0f;
-
-    // one block's B operand (fp16 codes) and delta
-    auto b_operand = [&](const WChunk& w, int j, h8_t& Bh, float& dw) {
-        uint4 B;
-        if (CI) {
-            // high nibbles pair with the lane's codes {2k,2k+1,2k+8,2k+9},
-            // low nibbles with those + 16; raw 1024 + n (the accumulator
-            // start takes off 1031 x the activation codes' sum, so the
-            // result is sum (n - 7) x: every value on the way an integer
-            // below 2^22)
-            const uint32_t P = w.c[j][0];
-            bytes_to_h1024((P >> 4) & 0x0F0F0F0Fu, B.x, B.y);
-            bytes_to_h1024(P & 0x0F0F0F0Fu, B.z, B.w);
-        } else if (WT == Q4) {
-            // the same nibbles as code - 7
-            const uint32_t P = w.c[j][0];
-            bytes_to_h((P >> 4) & 0x0F0F0F0Fu, kHm1031, B.x, B.y);
-            bytes_to_h(P & 0x0F0F0F0Fu, kHm1031, B.z, B.w);
-        } else {
-            s8x4_to_h(w.c[j][0], B.x, B.y);
-            s8x4_to_h(w.c[j][1], B.z, B.w);
-        }
-        Bh = __builtin_bit_cast(h8_t, B);
-        dw = h2f((uint16_t)(w.d[j >> 1] >> (16 * (j & 1))));
-    };
-
-    // weights and activation blocks in a ring of PF chunks (requested PF
-    // chunks ahead, every request issued so the waits are exact counts)
-    WChunk wr[PF];
-    XLane xq[PF][TPT];
-#pragma unroll
-    for (int p = 0; p < PF; p++) {
-        w_load(p, wr[p]);
-        x_load(p, xq[p]);
-    }
-    stage(xq[0], 0);
-    lds_barrier();
-    for (int cb = 0; cb < nch; cb += PF) {
-#pragma unroll
-        for (int p = 0; p < PF; p++) {
-            const int ch = cb + p;
-            if (ch >= nch) break;  // uniform
-            const int buf = ch & 1;
-            // the chunk's row deltas, and the activation operands two
-            // blocks ahead in a ring of two (block j + 2 is read into block
-            // j's slot once block j's products are issued), which keeps the
-            // registers within three wavefronts per SIMD
-            uint4 Ar[2][MR];
-            f4_t Cr[2][MR];  // CI: accumulator starts, in the same ring
-            float dxr[CH][MR];
-            auto c_init = [&](int j, int m) {
-                if constexpr (CI) return *reinterpret_cast<const f4_t*>(&xc[buf][j][4 * m + lg][0]);
-                else return f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            };
-#pragma unroll
-            for (int j = 0; j < CH; j++)
-#pragma unroll
-                for (int m = 0; m < MR; m++) {
-                    if (j < 2) {
-                        Ar[j][m] = xa[buf][j][m][lane];
-                        Cr[j][m] = c_init(j, m);
-                    }
-                    dxr[j][m] = xd[buf][j][4 * m + lg];
-                }
-            f4_t L[2][MR];
-            float dw[2];
-            {
-                h8_t Bh;
-                b_operand(wr[p], 0, Bh, dw[0]);
-#pragma unroll
-                for (int m = 0; m < MR; m++)
-                    L[0][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, Ar[0][m]), Bh, Cr[0][m],
-                                                                      0, 0, 0);
-            }
-#pragma unroll
-            for (int j = 0; j < CH; j++) {
-                const int cur = j & 1;
-                if (j + 1 < CH) {
-                    h8_t Bh;
-                    b_operand(wr[p], j + 1, Bh, dw[cur ^ 1]);
-#pragma unroll
-                    for (int m = 0; m < MR; m++)
-                        L[cur ^ 1][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            __builtin_bit_cast(h8_t, Ar[cur ^ 1][m]), Bh, Cr[cur ^ 1][m], 0, 0, 0);
-                }
-                if (j + 2 < CH) {
-#pragma unroll
-                    for (int m = 0; m < MR; m++) {
-                        Ar[cur][m] = xa[buf][j + 2][m][lane];
-                        Cr[cur][m] = c_init(j + 2, m);
-                    }
-                }
-                // block j's folds in block order: row 4m + lg, lane sums k
-#pragma unroll
-                for (int m = 0; m < MR; m++) {
-                    const float dd = dxr[j][m] * dw[cur];
-#pragma unroll
-                    for (int k = 0; k < 4; k++) acc[m][k] = acc[m][k] + L[cur][m][k] * dd;
-                }
-            }
-            w_load(ch + PF, wr[p]);
-            x_load(ch + PF, xq[p]);
-            if (ch + 1 < nch) stage(xq[(p + 1) % PF], buf ^ 1);
-            lds_barrier();
-        }
-    }
-    const int oc = blockIdx.x * 16 * NW + wv * 16 + lc;
-#pragma unroll
-    for (int m = 0; m < MR; m++) {
-        const int row = r0 + 4 * m + lg;
-        if (row < n_rows && oc < N)
-            out[(size_t)row * out_pitch + oc] = (acc[m][0] + acc[m][1]) + (acc[m][2] + acc[m][3]);
-    }
-}
-
 // ---------------------------------------------------------------------------
-// The same products for prompts with enough (row, column) tiles to fill the
-// chip: a wavefront owns 4 MR rows x 16 NG columns, so each activation
-// operand, accumulator start and row delta it reads from LDS serves NG
-// weight operands, and each converted weight operand MR row groups.
+// k_gemm_qw: a wavefront owns 4 MR rows x 16 NG columns, so each activation
+// operand, accumulator start and row delta it reads from LDS serves NG weight
+// operands, and each converted weight operand MR row groups; NW wavefronts
+// side by side in columns share the staged rows; a chunk is CH blocks, one
+// LDS barrier each.
 //
-// What bounds it: the vector unit.  Per block a wavefront issues 9 fp32
-// operations per 64 (row, column) pairs (the reference's rounding steps, none
-// of which can go) beside 11 per weight operand; with one column group (NG =
-// 1, k_gemm_qh) the LDS reads were the limit instead: per block and row group
-// 18 LDS cycles (two 16-byte reads and a dword per lane) on a unit that four
-// SIMDs share, against 9 + 11 / MR vector operations of 4 cycles each on one.
+// What bounds it with enough (row, column) tiles to fill the chip (NG = 2):
+// the vector unit.  Per block a wavefront issues 9 fp32 operations per 64
+// (row, column) pairs (the reference's rounding steps, none of which can go)
+// beside 11 per weight operand.  With NG = 1 there the LDS reads are the
+// limit instead: per block and row group 18 LDS cycles (two 16-byte reads and
+// a dword per lane) on a unit that four SIMDs share, against 9 + 11 / MR
+// vector operations of 4 cycles each on one.  With few tiles a SIMD has one
+// wavefront or none, and the chain over the blocks is bound by latencies: NG
+// = 1 then gives twice the wavefronts, CH = 8 halves the barriers and the
+// LDS reads run RD steps ahead.
 //
 // The weights are read in their own layout, 16 bytes per lane: lane (column,
 // g) of a 16 x 4 arrangement reads block b0 + g of its column, and a 4 x 4
@@ -551,18 +300,17 @@ __device__ __forceinline__ void lane_rows_transpose4(uint32_t (&r)[4])
     swap16(r[2], r[3]);
 }
 
-template <int WT, int MR, int NG, int NW, bool CL, int WPE, int ODT>
+template <int WT, int MR, int NG, int NW, int CH, int RD, bool CL, int WPE, int ODT>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) void k_gemm_qw(
         const uint8_t* __restrict__ x, int x_pitch, int n_rows, const uint32_t* __restrict__ wq,
         const uint16_t* __restrict__ wd, void* __restrict__ out, int out_pitch, int N, int nb)
 {
     constexpr int WV = WT == Q4 ? 1 : 2;  // code dwords of one lane of a weight block
     constexpr int WD = WT == Q4 ? 4 : 8;  // code dwords per weight block
-    constexpr int CH = 4;                 // blocks per chunk
     constexpr int PF = 2;                 // chunks in flight
     constexpr int kRows = 4 * MR, kThreads = 64 * NW;
     static_assert(ODT != Q8 || NG % 2 == 0, "a Q8 output block is two column groups");
-    __shared__ __align__(16) uint4 xa[2][CH][MR][64];                   // expanded operands (see k_gemm_qh)
+    __shared__ __align__(16) uint4 xa[2][CH][MR][64];                   // expanded operands (see above)
     __shared__ __align__(16) float xd[2][CH][4][MR];                    // deltas of rows 4m + g as [g][m]
     __shared__ __align__(16) float xc[2][CH][kRows][4];  // accumulator starts
     static_assert(MR >= 2, "the row deltas of two blocks are held in turn");
@@ -644,75 +392,73 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
     typedef uint32_t U4 __attribute__((ext_vector_type(4)));
     typedef uint32_t U2 __attribute__((ext_vector_type(2)));
     struct WChunk {
-        uint32_t c[NG][WV][4];  // CL: block b's lane-lg codes; plain: block lg's codes, before the transpose
-        uint32_t d[NG][2];      // the four blocks' deltas
+        // per four blocks: CL: block b's lane-lg codes; plain: block lg's codes, before the transpose
+        uint32_t c[CH / 4][NG][WV][4];
+        uint32_t d[CH / 4][NG][2];  // the four blocks' deltas
     };
     auto w_load = [&](int ch, WChunk& w) {
-        const int cc = min(ch, nch - 1);
-        const int ws = CL ? cc * N * 64 * WV : cc * CH * WD * 4, ds = CL ? cc * N * 8 : cc * CH * 2;
 #pragma unroll
-        for (int n = 0; n < NG; n++) {
+        for (int f = 0; f < CH / 4; f++) {
+            const int cc = min(ch, nch - 1) * (CH / 4) + f;
+            const int ws = CL ? cc * N * 64 * WV : cc * 4 * WD * 4, ds = CL ? cc * N * 8 : cc * 8;
 #pragma unroll
-            for (int q = 0; q < WV; q++) {
-                const U4 t = __builtin_amdgcn_raw_buffer_load_b128(wres, w_off[n] + 16 * q, ws, 0);
+            for (int n = 0; n < NG; n++) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) w.c[n][q][e] = t[e];
+                for (int q = 0; q < WV; q++) {
+                    const U4 t = __builtin_amdgcn_raw_buffer_load_b128(wres, w_off[n] + 16 * q, ws, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) w.c[f][n][q][e] = t[e];
+                }
+                const U2 d = __builtin_amdgcn_raw_buffer_load_b64(dres, d_off[n], ds, 0);
+                w.d[f][n][0] = d[0];
+                w.d[f][n][1] = d[1];
             }
-            const U2 d = __builtin_amdgcn_raw_buffer_load_b64(dres, d_off[n], ds, 0);
-            w.d[n][0] = d[0];
-            w.d[n][1] = d[1];
         }
     };
     // one lane's code dwords of block b, after the transpose (plain) or as
     // the copy has them
-    auto w_order = [&](WChunk& w) {
+    auto w_order = [&](uint32_t (&c)[WV][4]) {
         if constexpr (CL) {
-            if constexpr (WV == 2)
+            if constexpr (WV == 2) {
+                // [block][2 dwords] in order -> [dword][block]
+                uint32_t a[8];
 #pragma unroll
-                for (int n = 0; n < NG; n++) {
-                    // [block][2 dwords] in order -> [dword][block]
-                    uint32_t a[8];
+                for (int e = 0; e < 8; e++) a[e] = c[e >> 2][e & 3];
 #pragma unroll
-                    for (int e = 0; e < 8; e++) a[e] = w.c[n][e >> 2][e & 3];
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        w.c[n][0][b] = a[2 * b];
-                        w.c[n][1][b] = a[2 * b + 1];
-                    }
+                for (int b = 0; b < 4; b++) {
+                    c[0][b] = a[2 * b];
+                    c[1][b] = a[2 * b + 1];
                 }
+            }
+        } else if constexpr (WV == 1) {
+            lane_rows_transpose4(c[0]);
         } else {
+            // dwords 2k, 2k + 1 of a block belong to lane k
+            uint32_t lo[4] = {c[0][0], c[0][2], c[1][0], c[1][2]};
+            uint32_t hi[4] = {c[0][1], c[0][3], c[1][1], c[1][3]};
+            lane_rows_transpose4(lo);
+            lane_rows_transpose4(hi);
 #pragma unroll
-            for (int n = 0; n < NG; n++) {
-                if constexpr (WV == 1) {
-                    lane_rows_transpose4(w.c[n][0]);
-                } else {
-                    // dwords 2k, 2k + 1 of a block belong to lane k
-                    uint32_t lo[4] = {w.c[n][0][0], w.c[n][0][2], w.c[n][1][0], w.c[n][1][2]};
-                    uint32_t hi[4] = {w.c[n][0][1], w.c[n][0][3], w.c[n][1][1], w.c[n][1][3]};
-                    lane_rows_transpose4(lo);
-                    lane_rows_transpose4(hi);
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        w.c[n][0][b] = lo[b];
-                        w.c[n][1][b] = hi[b];
-                    }
-                }
+            for (int b = 0; b < 4; b++) {
+                c[0][b] = lo[b];
+                c[1][b] = hi[b];
             }
         }
     };
     auto b_operand = [&](const WChunk& w, int n, int j, h8_t& Bh, float& dw) {
         uint4 B;
+        const uint32_t(&c)[WV][4] = w.c[j / 4][n];
         if constexpr (WT == Q4) {
             // high nibbles in place: 1024 + 16 n
-            const uint32_t P = w.c[n][0][j];
+            const uint32_t P = c[0][j % 4];
             bytes_to_h1024(P & 0xF0F0F0F0u, B.x, B.y);
             bytes_to_h1024(P & 0x0F0F0F0Fu, B.z, B.w);
         } else {
-            bytes_to_h1024(w.c[n][0][j] ^ 0x80808080u, B.x, B.y);
-            bytes_to_h1024(w.c[n][WV - 1][j] ^ 0x80808080u, B.z, B.w);
+            bytes_to_h1024(c[0][j % 4] ^ 0x80808080u, B.x, B.y);
+            bytes_to_h1024(c[WV - 1][j % 4] ^ 0x80808080u, B.z, B.w);
         }
         Bh = __builtin_bit_cast(h8_t, B);
-        dw = h2f((uint16_t)(w.d[n][j >> 1] >> (16 * (j & 1))));
+        dw = h2f((uint16_t)(w.d[j / 4][n][(j >> 1) & 1] >> (16 * (j & 1))));
     };
 
     float acc[MR][NG][4];
@@ -723,7 +469,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
 #pragma unroll
             for (int k = 0; k < 4; k++) acc[m][n][k] = 0.0f;
 
-    // weights and activation blocks in a ring of PF chunks, as k_gemm_qh
+    // weights and activation blocks in a ring of PF chunks (requested PF
+    // chunks ahead, every request issued so the waits are exact counts)
     WChunk wr[PF];
     XLane xq[PF][TPT];
 #pragma unroll
@@ -735,20 +482,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
     lds_barrier();
     auto chunk = [&](int ch, auto pc) {
             constexpr int p = decltype(pc)::value, buf = p;
-            w_order(wr[p]);
+#pragma unroll
+            for (int f = 0; f < CH / 4; f++)
+#pragma unroll
+                for (int n = 0; n < NG; n++) w_order(wr[p].c[f][n]);
             // steps s = (block j, row group m) in turn: step s's products are
-            // issued, then step s - 1's are folded, with step s + 1's LDS
-            // reads in flight; the fences keep that order (and the registers
-            // a deeper interleaving would take)
+            // issued, then step s - 1's are folded, with the LDS reads of the
+            // next RD steps in flight; the fences keep that order (and the
+            // registers a deeper interleaving would take)
             auto a_read = [&](int s, uint4& A, f4_t& ci) {
                 A = xa[buf][s / MR][s % MR][lane];
                 ci = *reinterpret_cast<const f4_t*>(&xc[buf][s / MR][4 * (s % MR) + lg][0]);
             };
-            uint4 A[2];
-            f4_t ci[2], L[2][NG];
+            uint4 A[RD + 1];
+            f4_t ci[RD + 1], L[2][NG];
             h8_t Bh[NG];
             float dw[2][NG], dx[2][MR];
-            a_read(0, A[0], ci[0]);
+#pragma unroll
+            for (int s = 0; s < RD; s++) a_read(s, A[s], ci[s]);
 #pragma unroll
             for (int m = 0; m < MR; m++) dx[0][m] = xd[buf][0][lg][m];
             auto fold = [&](int s) {
@@ -769,20 +520,21 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
                 if (m == 0) {
 #pragma unroll
                     for (int n = 0; n < NG; n++) {
+                        // convert here, not earlier
 #pragma unroll
-                        for (int q = 0; q < WV; q++) asm volatile("" : "+v"(wr[p].c[n][q][j]));  // convert here, not earlier
+                        for (int q = 0; q < WV; q++) asm volatile("" : "+v"(wr[p].c[j / 4][n][q][j % 4]));
                         b_operand(wr[p], n, j, Bh[n], dw[j & 1][n]);
                     }
                 }
-                if (s + 1 < CH * MR) a_read(s + 1, A[(s + 1) & 1], ci[(s + 1) & 1]);
+                if (s + RD < CH * MR) a_read(s + RD, A[(s + RD) % (RD + 1)], ci[(s + RD) % (RD + 1)]);
                 if (m == MR - 1 && j + 1 < CH) {
 #pragma unroll
                     for (int mm = 0; mm < MR; mm++) dx[(j + 1) & 1][mm] = xd[buf][j + 1][lg][mm];
                 }
 #pragma unroll
                 for (int n = 0; n < NG; n++)
-                    L[s & 1][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, A[s & 1]), Bh[n],
-                                                                        ci[s & 1], 0, 0, 0);
+                    L[s & 1][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, A[s % (RD + 1)]), Bh[n],
+                                                                        ci[s % (RD + 1)], 0, 0, 0);
                 if (s > 0) fold(s - 1);
                 asm volatile("" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);
@@ -874,82 +626,65 @@ int chunk_layout_launch(const nc_tensor* w, void* codes, void* deltas, hipStream
     return launch_status("k_chunk_layout");
 }
 
-// Workgroup shapes, measured on MI355X with Q4 weights (us per launch,
-// exact results in every shape).  k_gemm_q: NG 16-wide column groups per
-// wavefront, NW wavefronts per workgroup sharing one staging of 4 MR rows,
-// PF weight chunks in flight (MF: a variant that issued a chunk's MFMAs
-// before its folds, since replaced by k_gemm_qh).
-//   64 rows:   q|k|v (2560 x 2048) 30.6 -> 22.1 with (1, 1, 4, 3, MF);
-//              o 28.5 -> 21.2, down (2048 x 5632) 67.0 -> 49.8 the same;
-//              gate|up (11264 x 2048) 81.6 -> 56.4 with (1, 2, 8, 4)
-//   512 rows:  (1, 2, 8, 4): q|k|v 138 -> 74, o 93 -> 62, down 196 -> 138;
-//              gate|up 503 -> 265 with (2, 2, 8, 3)
-// k_gemm_qh over the chunk-major copy (MR, NW, CH, PF), every launch after
-// a 512 MB write that evicts L2 and the memory-side cache, as a prefill
-// meets its weights (k_gemm_q in brackets):
-//   64 rows, (2, 4, 8, 2):  q|k|v (2560 x 2048) 18.2 [24.5]; o 14.2 [22.2];
-//              down (2048 x 5632) 29.5 [47.3]; Q8 q|k|v 20.5 [24.7], down
-//              32.6 [48.8]
-//   gate|up (11264 x 2048, 64 rows) and every 512-row shape, (4, 4, 4, 2):
-//              gate|up 40.0 [61.5], Q8 48.6 [64.5]; MiniCPM q|k|v (6912 x
-//              2304) 162 [210], o 63 [81], gate|up (11520 x 2304) 266
-//              [318], down (2304 x 5760) 145 [186]
-// Where the time goes (the same shapes with parts of the work left out of a
-// copy of the kernel): at 64 rows the fold was a few percent, the weight
-// loads a quarter and the activation staging another quarter -- a launch
-// is bound by load latency and request count, not by the arithmetic.  The
-// chunk-major copy turns four 4-byte loads from 16 rows into one 16-byte
-// load per thread and chunk; at 512 rows the staging was the largest part
-// (28%) while one wavefront of four did it, so every thread now stages one
-// AVX lane of one (row, block).
-// k_gemm_qw (MR, NG, NW) against k_gemm_qh, the same cold-cache timing (us
-// over the chunk-major copy / the weight's own layout; Q4, Q8 in brackets):
-//   512 rows x 11520 x 2304:  (4, 2, 4) 175 / 193 [199 / 210], k_gemm_qh 258
-//       / (k_gemm_q) 312 [305 / 310]; 6912 x 2304: 103 / 111 [115 / 124]
-//       against 152 / 214 [182 / 212]; 2304 x 5760: 106 / 115 [112 / 123]
-//       against 134 / 195 [161 / 194]
-//   201 rows x 5632 x 2048:  42 / 47 [47 / 54] against 55 / 77 [63 / 75]
-//   128 rows x 6144 x 2048:  (2, 2, 4) 30, (4, 2, 4) 32 / 36 [36 / 38]
-//       against 39 / 51 [42 / 50]
-//   201 rows x 2048 x 5632 (208 and 416 workgroups of 16 and 8 rows):
-//       (2, 2, 4) 53 / 60 [61 / 71], (4, 2, 4) 61 / 64 [67 / 72], k_gemm_qh
-//       66 / 76 [65 / 79]
-//   64 rows x 2048 x 5632 (64 and 128 workgroups): (2, 2, 4) 43 / 44,
-//       k_gemm_qh 28 / 41: too few workgroups, every one a serial chain over
-//       the blocks, so the smaller tiles win.
+// Workgroup shapes, measured on MI355X (us per launch, every launch after a
+// 512 MB write that evicts L2 and the memory-side cache, as a prefill meets
+// its weights; over the chunk-major copy / the weight's own layout; Q4, Q8 in
+// brackets).  (MR, NG, NW); "before": one column group per wavefront, the
+// compiler's order of LDS reads and folds.
+//   512 rows x 11520 x 2304:  (4, 2, 4) 175 / 193 [199 / 210], before 258 /
+//       312 [305 / 310]; 6912 x 2304: 103 / 111 [115 / 124], before 152 / 214
+//       [182 / 212]; 2304 x 5760: 106 / 115 [112 / 123], before 134 / 195
+//       [161 / 194]
+//   201 rows x 5632 x 2048:  (4, 2, 4) 42 / 47 [47 / 54], before 55 / 77 [63 /
+//       75]
+//   128 rows x 6144 x 2048 (384 and 768 workgroups of 16 and 8 rows x 128
+//       columns):  (2, 2, 4) 29 / 38 [40 / 48], (4, 2, 4) 32 / 36 [36 / 38],
+//       (2, 1, 4) 32 / 43 [45 / 52], before 39 / 51 [42 / 50]
+//   201 rows x 2048 x 5632 (208 and 416):  (2, 2, 4) 51 / 59 [59 / 69], (2, 1,
+//       4) 48 / 54 [63 / 68], (4, 2, 4) 61 / 64 [67 / 72], before 66 / 76 [65 /
+//       79]
+//   100 rows x 2304 x 5760 (126 and 234):  (2, 1, 4) 37 / 41 [42 / 46], (2, 2,
+//       4) 42 / 47 [50 / 53], before 61 / 61 [51 / 62]
+//   64 rows x 2048 x 5632 (64 and 128):  (2, 1, 4) 27 / 30 [31 / 34], (2, 2, 4)
+//       44 / 45 [49 / 53], before 28 / 41 [31 / 42]; 2560 x 2048: (2, 1, 4) 15 /
+//       18 [18 / 20], before 17 / 23 [19 / 23]
 // At 512 x 11520 x 2304 the (4, 2, 4) launch issues a vector instruction in
 // 87% of the SIMDs' slots (counters); holding LDS operands two steps ahead
-// or taking the d_x d_w products from the matrix cores changed nothing.
+// or taking the d_x d_w products from the matrix cores changed nothing there.
 //
-// The rule follows the workgroups a shape would have: 16 rows per workgroup
+// The rule follows the workgroups a shape would have: 16 rows x 128 columns
 // from kWide16 of them (Q8's weight operands cost more to form, so it shares
-// them over 16 rows earlier), else 8 rows from kWide8, else k_gemm_qh.
+// them over 16 rows earlier), else 8 x 128 from kWide8, else 8 x 64.
 template <int WT>
 constexpr int kWide16 = WT == Q4 ? 448 : 320;
-constexpr int kWide8 = 256;
+constexpr int kWide8 = 400;
 
 static int wide_groups(int N, int n_rows, int rows) { return ((N + 127) / 128) * ((n_rows + rows - 1) / rows); }
 
-// Rows per workgroup of k_gemm_qw for this product, 0 when it is not taken:
-// its chunks are four blocks, its loads 16 (codes) and 8 (deltas) bytes, and
-// its offsets 32 bits.
-static int gemm_wide_rows(int x_pitch, int n_rows, const nc_tensor* w)
+enum GemmShape { kGemmNone, kGemm8x64, kGemm8x128, kGemm16x128 };
+
+// The k_gemm_qw shape of this product, kGemmNone when it is not taken: its
+// chunks are four blocks, its loads need whole dwords, and its offsets are 32
+// bits.
+static GemmShape gemm_shape(int x_pitch, int n_rows, const nc_tensor* w)
 {
     const int N = w->rows, nb = w->cols / 32;
     const size_t lim = (size_t)1 << 31;
-    if (w->cols % 128 || ((uintptr_t)w->data & 15) || ((uintptr_t)w->deltas & 7)) return 0;
-    if ((size_t)N * nb * (w->dtype == NC_Q4 ? 16 : 32) >= lim || (size_t)n_rows * x_pitch >= lim) return 0;
-    if (wide_groups(N, n_rows, 16) >= (w->dtype == NC_Q4 ? kWide16<Q4> : kWide16<Q8>)) return 16;
-    return wide_groups(N, n_rows, 8) >= kWide8 ? 8 : 0;
+    if (w->cols % 128 || ((uintptr_t)w->data & 3) || ((uintptr_t)w->deltas & 3)) return kGemmNone;
+    if ((size_t)N * nb * (w->dtype == NC_Q4 ? 16 : 32) >= lim || (size_t)n_rows * x_pitch >= lim) return kGemmNone;
+    if (wide_groups(N, n_rows, 16) >= (w->dtype == NC_Q4 ? kWide16<Q4> : kWide16<Q8>)) return kGemm16x128;
+    return wide_groups(N, n_rows, 8) >= kWide8 ? kGemm8x128 : kGemm8x64;
 }
 
+// cl: w is the chunk-major copy.
 template <int ODT>
-static int gemm_wide(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, bool cl, int rows, void* out,
-                     int out_pitch, hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop)
+static int gemm_qw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, bool cl, GemmShape shape, void* out,
+                   int out_pitch, hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop)
 {
     const int N = w->rows, nb = w->cols / 32;
+    const int rows = shape == kGemm16x128 ? 16 : 8, cols = shape == kGemm8x64 ? 64 : 128;
     auto go = [&](auto kern) {
-        const dim3 grid((N + 127) / 128, (n_rows + rows - 1) / rows);
+        const dim3 grid((N + cols - 1) / cols, (n_rows + rows - 1) / rows);
         if (ev_start)
             hipExtLaunchKernelGGL(kern, grid, dim3(256), 0, st, ev_start, ev_stop, 0, x, x_pitch, n_rows,
                                   (const uint32_t*)w->data, (const uint16_t*)w->deltas, out, out_pitch, N, nb);
@@ -960,8 +695,12 @@ static int gemm_wide(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor*
     auto by_layout = [&](auto wt, auto c) {
         constexpr int WT = decltype(wt)::value;
         constexpr bool CL = decltype(c)::value;
-        if (rows == 16) go(k_gemm_qw<WT, 4, 2, 4, CL, 3, ODT>);
-        else go(k_gemm_qw<WT, 2, 2, 4, CL, 4, ODT>);
+        if (shape == kGemm16x128) go(k_gemm_qw<WT, 4, 2, 4, 4, 1, CL, 3, ODT>);
+        else if (shape == kGemm8x128) go(k_gemm_qw<WT, 2, 2, 4, 4, 1, CL, 4, ODT>);
+        else if constexpr (ODT == F32) {
+            if (nb % 8 == 0) go(k_gemm_qw<WT, 2, 1, 4, 8, 2, CL, 2, ODT>);
+            else go(k_gemm_qw<WT, 2, 1, 4, 4, 1, CL, 2, ODT>);
+        }
     };
     auto by_type = [&](auto wt) {
         if (cl) by_layout(wt, std::true_type{});
@@ -974,7 +713,8 @@ static int gemm_wide(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor*
 
 bool gemm_q_act_supported(int x_pitch, int n_rows, const nc_tensor* w)
 {
-    return (w->dtype == NC_Q4 || w->dtype == NC_Q8) && n_rows >= kGemmMinRows && gemm_wide_rows(x_pitch, n_rows, w) != 0;
+    return (w->dtype == NC_Q4 || w->dtype == NC_Q8) && n_rows >= kGemmMinRows &&
+           gemm_shape(x_pitch, n_rows, w) >= kGemm8x128;
 }
 
 int gemm_q_act(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, uint8_t* out, int out_pitch,
@@ -982,13 +722,9 @@ int gemm_q_act(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, ui
 {
     if (!gemm_q_act_supported(x_pitch, n_rows, w))
         return fail(NC_ERR_ARG, "gemm to Q8 rows: [%d x %d] weights, %d rows", w->rows, w->cols, n_rows);
-    return gemm_wide<Q8>(x, x_pitch, n_rows, w, false, gemm_wide_rows(x_pitch, n_rows, w), out, out_pitch, st, nullptr,
-                         nullptr);
+    return gemm_qw<Q8>(x, x_pitch, n_rows, w, false, gemm_shape(x_pitch, n_rows, w), out, out_pitch, st, nullptr,
+                       nullptr);
 }
-
-constexpr int kGemmTallCols = 8192;
-constexpr int kGemmWideRows = 256;
-constexpr int kGemmShortRows = 80;  // prompts up to this many rows take the short-prompt shapes
 
 int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, float* out, int out_pitch,
                hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop, const nc_tensor* wc)
@@ -999,54 +735,31 @@ int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, fl
     const int N = w->rows, nb = w->cols / 32;
     if (wc && (wc->dtype != w->dtype || wc->rows != N || wc->cols != w->cols || !chunk_layout_supported(wc)))
         return fail(NC_ERR_ARG, "gemm: chunk copy [%d x %d] of a [%d x %d] weight", wc->rows, wc->cols, N, w->cols);
-    if (const int rows = gemm_wide_rows(x_pitch, n_rows, wc ? wc : w))
-        return gemm_wide<F32>(x, x_pitch, n_rows, wc ? wc : w, wc != nullptr, rows, out, out_pitch, st, ev_start,
-                              ev_stop);
-    auto go = [&](auto kern, int mr, int ng, int nw, const nc_tensor* wt = nullptr) {
-        if (!wt) wt = w;
+    // the chunk-major copy, when the caller has one
+    const nc_tensor* wt = wc ? wc : w;
+    if (const GemmShape shape = gemm_shape(x_pitch, n_rows, wt))
+        return gemm_qw<F32>(x, x_pitch, n_rows, wt, wc != nullptr, shape, out, out_pitch, st, ev_start, ev_stop);
+    // (NG, NW, MR, PF): 512 rows (1, 2, 8, 4), tall weights (2, 2, 8, 3);
+    // 64 rows (1, 1, 4, 3), tall (1, 2, 8, 4)
+    auto go = [&](auto kern, int mr, int ng, int nw) {
         const dim3 grid((N + 16 * ng * nw - 1) / (16 * ng * nw), (n_rows + 4 * mr - 1) / (4 * mr));
         if (ev_start)
             hipExtLaunchKernelGGL(kern, grid, dim3(64 * nw), 0, st, ev_start, ev_stop, 0, x, x_pitch, n_rows,
-                                  (const uint32_t*)wt->data, (const uint16_t*)wt->deltas, out, out_pitch, N, nb);
+                                  (const uint32_t*)w->data, (const uint16_t*)w->deltas, out, out_pitch, N, nb);
         else
-            hipLaunchKernelGGL(kern, grid, dim3(64 * nw), 0, st, x, x_pitch, n_rows, (const uint32_t*)wt->data,
-                               (const uint16_t*)wt->deltas, out, out_pitch, N, nb);
+            hipLaunchKernelGGL(kern, grid, dim3(64 * nw), 0, st, x, x_pitch, n_rows, (const uint32_t*)w->data,
+                               (const uint16_t*)w->deltas, out, out_pitch, N, nb);
     };
-    const bool wide = n_rows >= kGemmWideRows, tall = N >= kGemmTallCols;
-    // the chunk-major copy, when the caller has one (shapes measured with
-    // cold caches, as a prefill meets its weights): few tiles, or a product
-    // past k_gemm_qw's offsets
-    if (wc) {
-        auto goc = [&](auto kern, int mr, int nw) { go(kern, mr, 1, nw, wc); };
-        auto by_type_c = [&](auto wt) {
-            constexpr int WT = decltype(wt)::value;
-            // chunks of 8 blocks need nb % 8 == 0 (the copy itself is in
-            // 4-block chunks)
-            if (tall || n_rows > kGemmShortRows || nb % 8)
-                goc(k_gemm_qh<WT, 4, 4, 4, 2, true, WT == Q4 ? 3 : 1>, 4, 4);
-            else goc(k_gemm_qh<WT, 2, 4, 8, 2, true>, 2, 4);
-        };
-        if (w->dtype == NC_Q4) by_type_c(std::integral_constant<int, Q4>{});
-        else by_type_c(std::integral_constant<int, Q8>{});
-        return launch_status("k_gemm_qh (chunk layout)");
-    }
-    // the fp16 matrix-core kernel: chunks of 4 (8) blocks, 8- (16-) byte
-    // delta loads
-    const bool qh4 = nb % 4 == 0 && ((uintptr_t)w->deltas & 7) == 0;
-    const bool qh8 = nb % 8 == 0 && ((uintptr_t)w->deltas & 15) == 0;
-    auto goh = [&](auto kern, int mr, int nw) { go(kern, mr, 1, nw); };
-    auto by_type = [&](auto wt) {
-        constexpr int WT = decltype(wt)::value;
-        if (qh4 && (wide || tall || n_rows > kGemmShortRows || !qh8)) goh(k_gemm_qh<WT, 4, 4, 4, 2, false>, 4, 4);
-        else if (qh8 && n_rows <= 16) goh(k_gemm_qh<WT, 2, 2, 8, 3, false>, 2, 2);
-        else if (qh8 && (N <= 2048 || nb >= 128)) goh(k_gemm_qh<WT, 2, 4, 8, 2, false>, 2, 4);
-        else if (qh8) goh(k_gemm_qh<WT, 4, 4, 4, 2, false>, 4, 4);
+    const bool wide = n_rows >= 256, tall = N >= 8192;
+    auto by_type = [&](auto t) {
+        constexpr int WT = decltype(t)::value;
+        if (wide && tall) go(k_gemm_q<WT, 2, 2, 8, 3>, 8, 2, 2);
         else if (wide || (tall && n_rows >= 32)) go(k_gemm_q<WT, 1, 2, 8, 4>, 8, 1, 2);
         else go(k_gemm_q<WT, 1, 1, 4, 3>, 4, 1, 1);
     };
     if (w->dtype == NC_Q4) by_type(std::integral_constant<int, Q4>{});
     else by_type(std::integral_constant<int, Q8>{});
-    return launch_status("k_gemm_q / k_gemm_qh");
+    return launch_status("k_gemm_q");
 }
 
 }  // namespace nc

@@ -114,15 +114,20 @@ def test_matmul_act_out(gpu, oracle, xdt, wdt, K, N):
 
 
 WIDE_CASES = [
-    # (w dtype, K, N, rows, start): the prefill matmul's launches that share
-    # activation operands over 32 columns, 16 rows per workgroup (Q4 from 448
-    # workgroups, Q8 from 320) and 8 (from 256): one, an odd and an even number
-    # of four-block chunks, rows and columns past a tile, a partial last block
+    # (w dtype, K, N, rows, start): the prefill matmul's launches of 16 rows x
+    # 128 columns per workgroup (Q4 from 448 workgroups, Q8 from 320), 8 x 128
+    # (from 400) and 8 x 64 (fewer, chunks of 8 and of 4 blocks): one, an odd
+    # and an even number of chunks, rows and columns past a tile, a partial
+    # last block
     (Q4, 128, 1010, 903, 3),
     (Q4, 384, 4100, 225, 0),
     (Q8, 640, 2050, 310, 0),
-    (Q4, 256, 1010, 260, 0),
-    (Q8, 384, 3000, 85, 0),
+    (Q4, 256, 1010, 420, 0),
+    (Q8, 384, 3000, 137, 0),
+    (Q4, 256, 1010, 21, 1),
+    (Q8, 768, 70, 9, 0),
+    (Q4, 640, 129, 33, 0),
+    (Q8, 128, 40, 8, 0),
 ]
 
 
