@@ -378,6 +378,135 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn(const uint8_t* __restrict
     }
 }
 
+// One query row with its whole V slice in shared memory (contexts up to
+// kA1MaxCtx): k_attn's arithmetic on 512 threads.  What bounds it: latency, of
+// the cache rows, of the softmax's sequential sum (one wavefront, 3 ns per
+// position) and of the P.V chains.  Every K row and V part of the context is
+// requested at the start (KR rows and VN parts per thread), and the chains run
+// with no barrier and no staging between them: wavefront l is lane l, thread
+// its column.  Q8 rows (us, k_attn / this): 512 positions 10.1 / 7.7, 700 13.5 /
+// 11.4, 1000 17.2 / 13.8; 64 positions 5.0 / 4.9, 130 5.1 / 5.5, so short contexts
+// keep k_attn.
+constexpr int kA1Threads = 512;
+constexpr int kA1MinCtx = 256, kA1MaxCtx = 1024;
+
+template <int ADT>
+size_t attn1_lds(int n)
+{
+    return ((size_t)((n + 3) & ~3) + 512) * 4 + (size_t)n * v_stage_bytes<ADT>();
+}
+
+template <int ADT, int KR>
+__global__ __launch_bounds__(kA1Threads) void k_attn1(const uint8_t* __restrict__ q, const uint8_t* __restrict__ kc,
+                                                      int k_pitch, const uint8_t* __restrict__ vc, int v_pitch,
+                                                      uint8_t* __restrict__ out, int hq, int hkv, int n, float scale)
+{
+    constexpr int VP = v_parts<ADT>(), VB = v_stage_bytes<ADT>(), VN = KR * VP;
+    extern __shared__ __align__(16) float sm[];
+    __shared__ float red[9];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int h = blockIdx.x, g = h / (hq / hkv);
+    const int qcols = hq * 64, kvcols = hkv * 64;
+    const int qd = act_delta_offset(qcols), kvd = act_delta_offset(kvcols);
+    float* S = sm;
+    float* acc = S + ((n + 3) & ~3);
+    uint8_t* V = reinterpret_cast<uint8_t*>(acc + 512);
+
+    QHead<ADT> Q;
+    load_q<ADT>(Q, q, h, qd);
+    KRowT<ADT> K[KR];
+#pragma unroll
+    for (int i = 0; i < KR; i++) K[i] = load_k<ADT>(kc, k_pitch, kvd, g, min(tid + i * kA1Threads, n - 1));
+    uint32_t vp[VN][4], vd[KR];
+#pragma unroll
+    for (int i = 0; i < VN; i++) {
+        const int idx = tid + i * kA1Threads;
+        const int c = min(idx / VP, n - 1);
+        const uint4 t = reinterpret_cast<const uint4*>(vc + (size_t)c * v_pitch + g * (ADT == Q8 ? 64 : 128))[idx % VP];
+        vp[i][0] = t.x;
+        vp[i][1] = t.y;
+        vp[i][2] = t.z;
+        vp[i][3] = t.w;
+    }
+    if (ADT == Q8) {
+#pragma unroll
+        for (int i = 0; i < KR; i++)
+            vd[i] = reinterpret_cast<const uint32_t*>(vc + (size_t)min(tid + i * kA1Threads, n - 1) * v_pitch + kvd)[g];
+    }
+    float mx = -INFINITY;
+    float sc[KR];
+#pragma unroll
+    for (int i = 0; i < KR; i++) {
+        sc[i] = score<ADT>(Q, K[i], scale);
+        if (tid + i * kA1Threads < n) mx = fmaxf(mx, sc[i]);
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if (lane == 0) red[w] = mx;
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 8; i++) mx = fmaxf(mx, red[i]);
+#pragma unroll
+    for (int i = 0; i < KR; i++) {
+        const int c = tid + i * kA1Threads;
+        sc[i] = expf_ref(sc[i] - mx);
+        if (c < n) S[c] = sc[i];
+    }
+    lds_barrier();
+    if (w == 0) {
+        const float ss = seq_sum(S, n);
+        if (lane == 0) red[8] = ss;
+    }
+    // (wavefront 0 stores its V parts after the sum, the others beside it)
+#pragma unroll
+    for (int i = 0; i < VN; i++) {
+        const int idx = tid + i * kA1Threads;
+        if (idx / VP < n) reinterpret_cast<uint4*>(V + (size_t)(idx / VP) * VB)[idx % VP] = make_uint4(vp[i][0], vp[i][1], vp[i][2], vp[i][3]);
+    }
+    if (ADT == Q8) {
+#pragma unroll
+        for (int i = 0; i < KR; i++) {
+            const int c = tid + i * kA1Threads;
+            if (c < n) reinterpret_cast<uint32_t*>(V + (size_t)c * VB + 64)[0] = vd[i];
+        }
+    }
+    lds_barrier();
+    const float sum = red[8];
+#pragma unroll
+    for (int i = 0; i < KR; i++) {
+        const int c = tid + i * kA1Threads;
+        const bool valid = c < n;
+        const float p = act_roundtrip<ADT>(valid ? sc[i] / sum : 0.0f, valid);
+        if (valid) S[c] = p;
+    }
+    lds_barrier();
+
+    // ---- P.V: lane l = w, column = lane
+    const int n8 = n & ~7;
+    float a = 0.0f;
+    int c = w;
+    for (; c + 56 < n8; c += 64) {
+        float p[8], v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            p[u] = S[c + 8 * u];
+            v[u] = v_one<ADT>(V + (size_t)(c + 8 * u) * VB, lane);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) a = p[u] * v[u] + a;
+    }
+    for (; c < n8; c += 8) a = S[c] * v_one<ADT>(V + (size_t)c * VB, lane) + a;
+    acc[tid] = a;
+    lds_barrier();
+    if (w == 0) {
+        float s = acc[lane];
+#pragma unroll
+        for (int l = 1; l < 8; l++) s = s + acc[l * 64 + lane];
+        for (int t = n8; t < n; t++) s = s + S[t] * v_one<ADT>(V + (size_t)t * VB, lane);
+        act_store<ADT>(out, h * 64 + lane, qd, s, true);
+    }
+}
+
 // ---- R query rows per workgroup (prefill) ---------------------------------
 
 // R consecutive query rows of one head per workgroup, with the arithmetic of
@@ -826,6 +955,14 @@ int attn_go(const uint8_t* q, int q_pitch, const uint8_t* kc, int k_pitch, const
         if (m <= 1024 && !few) return go_rows(k_attn_rows<ADT, 8>, attn_rows_lds<ADT, 8>(m), 8);
         if (m <= 2048) return go_rows(k_attn_rows<ADT, 4>, attn_rows_lds<ADT, 4>(m), 4);
         return go_rows(k_attn_rows<ADT, 2>, attn_rows_lds<ADT, 2>(m), 2);
+    }
+    if (!dpos && n_ctx >= kA1MinCtx && n_ctx <= kA1MaxCtx) {
+        auto go1 = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(hq), dim3(kA1Threads), attn1_lds<ADT>(n_ctx), st, q, kc, k_pitch, vc, v_pitch,
+                               out, hq, hkv, n_ctx, scale);
+            return launch_status("k_attn1");
+        };
+        return n_ctx <= kA1Threads ? go1(k_attn1<ADT, 1>) : go1(k_attn1<ADT, 2>);
     }
     const int lds_ctx = dpos ? max_ctx : n_ctx;
     hipLaunchKernelGGL(k_attn<ADT>, dim3(hq, rows), dim3(kAttnThreads), attn_lds<ADT>(lds_ctx), st, q, q_pitch, kc,

@@ -414,6 +414,14 @@ ATTN_CASES = [
     (F16, 32, 32, 4096, 4095),
     (F16, 4, 4, 4090, 4081),
     (F16, 4, 2, 1500, 0),
+    # one row with its V slice in shared memory (256 to 1024 positions), n mod 8
+    # and mod 32 edges, both numbers of K rows per thread
+    (Q8, 2, 1, 256, 255),
+    (Q8, 2, 2, 511, 510),
+    (Q8, 3, 1, 517, 516),
+    (F16, 2, 1, 255, 254),
+    (F16, 2, 2, 513, 512),
+    (F16, 3, 3, 1023, 1022),
     # several fp16 rows on the matrix cores: one tile and parts of it, rows
     # across a tile's and a chunk's edge, every n mod 8, the longest context
     # it takes and the next
