@@ -17,12 +17,11 @@
 //      the double below 1); the token is lower_bound(c, u).
 //
 // On the device, workgroups of 1024 threads:
-//   * candidates: a systematic sample of 1024 logits sets a threshold (each
-//     wavefront sorts its 64 in registers and offers the quantile that would
-//     keep about 1.5 k + 256 logits; the median offer is taken; every
-//     workgroup computes the same one), and every logit at or above it is
-//     gathered (up to 4096): each workgroup gathers a slice of at least 4096
-//     logits, and the last one to finish takes the candidates into LDS and
+//   * candidates: a systematic sample of 4096 logits sets a threshold (each
+//     wavefront offers the quantile of its own that would keep about
+//     1.5 k + 256 logits; the median offer is taken; every workgroup computes the
+//     same one), and every logit at or above it is gathered (up to 4096): each
+//     workgroup gathers a slice of at least 4096 logits, and the last one to finish takes the candidates into LDS and
 //     runs the rest of the step alone.  For k < 64 an
 //     8-bit radix select finds the (k+1)-th largest candidate and the k above
 //     it are sorted in one wavefront's registers; larger k bitonic-sort the
@@ -55,7 +54,8 @@ namespace nc {
 
 constexpr int kSmThreads = 1024;
 constexpr int kSmCap = 4096;      // candidates sorted in LDS
-constexpr int kSmSample = 1024;   // threshold sample size
+constexpr int kSmPer = 4;         // sampled logits per thread
+constexpr int kSmSample = 4096;   // threshold sample size
 constexpr int kSmStage = 8192;    // logits per LDS stage of the fallback
 
 // ---- std::mt19937 (state: 624 words, then the index of the next word) ----
@@ -261,7 +261,10 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
     const int lo = (int)blockIdx.x * slice, hi = min(n, lo + slice);
     // the threshold sample and the slice requested together
     const bool sampled = n > kSmCap;
-    const float sx = sampled ? A.logits[(long long)tid * n / kSmSample] : 0.0f;
+    float sx[kSmPer] = {};
+    if (sampled)
+#pragma unroll
+        for (int j = 0; j < kSmPer; j++) sx[j] = A.logits[(long long)(kSmPer * tid + j) * n / kSmSample];
     float x[kSmGu];
 #pragma unroll
     for (int u = 0; u < kSmGu; u++) {
@@ -272,19 +275,42 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
     for (int i = tid; i < 4 * 256; i += kSmThreads) (&hist[0][0])[i] = 0;
     if (tid == 0) s_top = 0;
 
-    // threshold: about the (1.5 k + 256) n / 1024-th largest logit, from a
-    // systematic sample of 1024 (only a candidate bound: any threshold gives
-    // the same result, the fallback covers the rest): each wavefront sorts
-    // its 64 sampled keys in registers and offers its r/16-th largest; the
-    // threshold is the median of the 16 offers (every workgroup finds the
-    // same one)
+    // threshold: about the T-th largest logit, T = 1.5 k + 256, from a
+    // systematic sample of 4096 (only a candidate bound: any threshold gives
+    // the same result, the fallback covers the rest).  Each thread keeps the
+    // largest of its four, each wavefront sorts its 64 of those in registers
+    // and offers one, and the threshold is the median of the 16 offers (every
+    // workgroup finds the same one).  lam of the 64 are expected above the
+    // wanted logit; the median of the offers of rank i (0-based) has about
+    // i + 0.69 above it, so the first i with i + 0.69 >= lam is taken.  For
+    // k < 64, where far more than k are kept anyway, the offer is the largest
+    // (no sort: 32000 logits, k = 50, 17 us against 19), each thread using as
+    // few of its four as keep T (0.8 T at least): fewer candidates in large
+    // vocabularies, 151936 logits, k = 50, 24 -> 20 us.
+    // One sampled logit per thread left 0.7 to 3 of them above it in a large
+    // vocabulary, too few: 3 of 12 draws of k = 850 of 100352 logits and 4 of
+    // 12 of k = 1000 of 122753 kept fewer than k or more than kSmCap and ran
+    // the serial fallback, 10 to 12.6 ms; with four none of
+    // 24 draws of any size from 5000 to 151936 logits and k from 2 to 1000 did.
     uint32_t thr = 0;
     if (sampled) {
-        const long long r = ((long long)(3 * k / 2 + 256) * kSmSample) / n;
-        const int rw = (int)(r / (kSmThreads / kWave)) < kWave - 1 ? (int)(r / (kSmThreads / kWave)) : kWave - 1;
+        const int T = min(3 * k / 2 + 256, n);
+        const float f = (float)T / (float)n;
+        const float large = 0.69f / (kWave * f);  // threads' logits for which lam = 0.69
+        const bool few = k < kWave && large >= 0.8f;
+        const int per = few ? min((int)large, kSmPer) : kSmPer;
+        uint32_t sk = fkey(sx[0]);
+        float none = 1.0f - f;
+#pragma unroll
+        for (int j = 1; j < kSmPer; j++) {
+            if (j < per) sk = max(sk, fkey(sx[j]));
+            none *= 1.0f - f;
+        }
+        const float lam = (float)kWave * (1.0f - none);
+        const int rw = few ? 0 : min(max((int)ceilf(lam - 0.69f), 0), kWave - 1);
         if (rw == 0) {
             // the wavefront's largest (the large vocabularies)
-            uint32_t v = fkey(sx);
+            uint32_t v = sk;
 #pragma unroll
             for (int o = kWave / 2; o > 0; o >>= 1) {
                 const uint32_t y = (uint32_t)__shfl_xor((int)v, o);
@@ -292,7 +318,7 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
             }
             if (lane == 0) s_wq[w] = v;
         } else {
-            const uint32_t v = wave_sort<true>(fkey(sx));
+            const uint32_t v = wave_sort<true>(sk);
             if (lane == rw) s_wq[w] = v;
         }
         lds_barrier();

@@ -81,6 +81,20 @@ def test_sample_topk_vocab_sizes_and_twist(gpu, oracle):
     run_draws(gpu, oracle, x, 40, 1.0, seed=5, draws=330)
 
 
+@pytest.mark.parametrize("n", [4096, 4097, 5000, 32000, 50304, 151936])
+def test_sample_topk_threshold_ranges(gpu, oracle, n):
+    """Either side of the sampled threshold's rules: no threshold (4096), the
+    wavefronts' largest (k < 64 from about 25000 logits) or a sorted rank, and
+    1 to 4 sampled logits per thread; logits in any order and in descending
+    order, where a sample of neighbours would mislead."""
+    x = logits_case("normal", n, seed=n)
+    for k in (1, 2, 63, 64, 850, 1000):
+        run_draws(gpu, oracle, x, k, 0.9, seed=n + k, draws=2)
+    x = np.sort(x)[::-1].copy()
+    for k in (50, 1000):
+        run_draws(gpu, oracle, x, k, 0.9, seed=n + k, draws=2)
+
+
 def test_sample_topk_rejects_bad_arguments(gpu):
     L = gpu.lib()
     d_x, d_st, d_tok = gpu.DeviceBuffer(4 * 100), gpu.DeviceBuffer(4 * 625), gpu.DeviceBuffer(4)
