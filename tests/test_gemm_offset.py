@@ -2,7 +2,7 @@
 
 The reference's Q4 block dot product (gten/ops.cpp:387-490) multiplies each
 activation code x by the decoded weight n - 7 (n the stored nibble) and sums
-eight such products per AVX lane.  The long-prompt shape of k_gemm_qh hands
+eight such products per AVX lane.  The prefill matmul (k_gemm_qw) hands
 the fp16 matrix cores the raw weight 1024 + n instead (fp16 bits 0x6400 | n,
 one v_perm_b32 per two codes) and starts each product sum from
 -1031 x (sum of the lane's activation codes).  That equals the reference's
