@@ -17,11 +17,12 @@
 //      the double below 1); the token is lower_bound(c, u).
 //
 // On the device, workgroups of 1024 threads:
-//   * candidates: a systematic sample of 4096 logits sets a threshold (each
-//     wavefront offers the quantile of its own that would keep about
-//     1.5 k + 256 logits; the median offer is taken; every workgroup computes the
-//     same one), and every logit at or above it is gathered (up to 4096): each
-//     workgroup gathers a slice of at least 4096 logits, and the last one to finish takes the candidates into LDS and
+//   * candidates: a systematic sample sets a threshold (1024 logits, 4096 of
+//     a large vocabulary; each wavefront offers the quantile of its own that
+//     would keep about 1.5 k + 256 logits; the median offer is taken; every
+//     workgroup computes the same one), and every logit at or above it is
+//     gathered (up to 4096): each workgroup gathers a slice of at least 4096
+//     logits, and the last one to finish takes the candidates into LDS and
 //     runs the rest of the step alone.  For k < 64 an
 //     8-bit radix select finds the (k+1)-th largest candidate and the k above
 //     it are sorted in one wavefront's registers; larger k bitonic-sort the
@@ -54,7 +55,8 @@ namespace nc {
 
 constexpr int kSmThreads = 1024;
 constexpr int kSmCap = 4096;      // candidates sorted in LDS
-constexpr int kSmPer = 4;         // sampled logits per thread
+constexpr int kSmPer = 4;         // sampled logits per thread,
+constexpr int kSmOneMax = 32768;  // one up to this many
 constexpr int kSmSample = 4096;   // threshold sample size
 constexpr int kSmStage = 8192;    // logits per LDS stage of the fallback
 
@@ -262,9 +264,14 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
     // the threshold sample and the slice requested together
     const bool sampled = n > kSmCap;
     float sx[kSmPer] = {};
-    if (sampled)
+    const int loaded = n > kSmOneMax ? kSmPer : 1;
+    if (sampled) {
+        sx[0] = A.logits[(long long)(kSmPer * tid) * n / kSmSample];
+        if (loaded > 1) {
 #pragma unroll
-        for (int j = 0; j < kSmPer; j++) sx[j] = A.logits[(long long)(kSmPer * tid + j) * n / kSmSample];
+            for (int j = 1; j < kSmPer; j++) sx[j] = A.logits[(long long)(kSmPer * tid + j) * n / kSmSample];
+        }
+    }
     float x[kSmGu];
 #pragma unroll
     for (int u = 0; u < kSmGu; u++) {
@@ -276,38 +283,46 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
     if (tid == 0) s_top = 0;
 
     // threshold: about the T-th largest logit, T = 1.5 k + 256, from a
-    // systematic sample of 4096 (only a candidate bound: any threshold gives
-    // the same result, the fallback covers the rest).  Each thread keeps the
-    // largest of its four, each wavefront sorts its 64 of those in registers
+    // systematic sample (only a candidate bound: any threshold gives the same
+    // result, the fallback covers the rest).  Each thread keeps the largest of
+    // its sampled logits, each wavefront sorts its 64 of those in registers
     // and offers one, and the threshold is the median of the 16 offers (every
     // workgroup finds the same one).  lam of the 64 are expected above the
     // wanted logit; the median of the offers of rank i (0-based) has about
-    // i + 0.69 above it, so the first i with i + 0.69 >= lam is taken.  For
+    // i + 0.69 above it, so the first i with i + 0.69 >= lam is taken (0.8 lam
+    // where that still keeps 4 k), or the i below lam with one logit per thread
+    // (32000 logits, k = 100: 38 us, 43 with the other rule).  For
     // k < 64, where far more than k are kept anyway, the offer is the largest
-    // (no sort: 32000 logits, k = 50, 17 us against 19), each thread using as
-    // few of its four as keep T (0.8 T at least): fewer candidates in large
+    // (no sort: 32000 logits, k = 50, 17 us against 19) of as few logits per
+    // thread as keep T (0.8 T at least): fewer candidates in large
     // vocabularies, 151936 logits, k = 50, 24 -> 20 us.
-    // One sampled logit per thread left 0.7 to 3 of them above it in a large
-    // vocabulary, too few: 3 of 12 draws of k = 850 of 100352 logits and 4 of
-    // 12 of k = 1000 of 122753 kept fewer than k or more than kSmCap and ran
-    // the serial fallback, 10 to 12.6 ms; with four none of
-    // 24 draws of any size from 5000 to 151936 logits and k from 2 to 1000 did.
+    // One sampled logit per thread leaves at least 3 above the wanted one for
+    // the largest k up to kSmOneMax logits; four cost 0.5 us there.  Beyond,
+    // one leaves 0.7 to 3, too few: 3 of 12 draws of k = 850 of 100352 logits
+    // and 4 of 12 of k = 1000 of 122753 kept fewer than k or more than kSmCap
+    // and ran the serial fallback, 10 to 12.6 ms; with four none of 24 draws
+    // of any k from 2 to 1000 of up to 151936 logits did.
     uint32_t thr = 0;
     if (sampled) {
         const int T = min(3 * k / 2 + 256, n);
         const float f = (float)T / (float)n;
         const float large = 0.69f / (kWave * f);  // threads' logits for which lam = 0.69
         const bool few = k < kWave && large >= 0.8f;
-        const int per = few ? min((int)large, kSmPer) : kSmPer;
+        const int per = few ? min(max((int)large, 1), loaded) : loaded;
         uint32_t sk = fkey(sx[0]);
         float none = 1.0f - f;
 #pragma unroll
         for (int j = 1; j < kSmPer; j++) {
-            if (j < per) sk = max(sk, fkey(sx[j]));
-            none *= 1.0f - f;
+            if (j < per) {
+                sk = max(sk, fkey(sx[j]));
+                none *= 1.0f - f;
+            }
         }
         const float lam = (float)kWave * (1.0f - none);
-        const int rw = few ? 0 : min(max((int)ceilf(lam - 0.69f), 0), kWave - 1);
+        const float want = lam * fmaxf(0.8f, fminf(1.0f, 4.0f * (float)k / (float)T));
+        const int rw = few         ? 0
+                       : loaded > 1 ? min(max((int)ceilf(want - 0.69f), 0), kWave - 1)
+                                    : min((int)((float)kWave * f), kWave - 1);
         if (rw == 0) {
             // the wavefront's largest (the large vocabularies)
             uint32_t v = sk;

@@ -81,11 +81,11 @@ def test_sample_topk_vocab_sizes_and_twist(gpu, oracle):
     run_draws(gpu, oracle, x, 40, 1.0, seed=5, draws=330)
 
 
-@pytest.mark.parametrize("n", [4096, 4097, 5000, 32000, 50304, 151936])
+@pytest.mark.parametrize("n", [4096, 4097, 5000, 32768, 32769, 50304, 151936])
 def test_sample_topk_threshold_ranges(gpu, oracle, n):
     """Either side of the sampled threshold's rules: no threshold (4096), the
-    wavefronts' largest (k < 64 from about 25000 logits) or a sorted rank, and
-    1 to 4 sampled logits per thread; logits in any order and in descending
+    wavefronts' largest (k < 64 from about 25000 logits) or a sorted rank, one
+    sampled logit per thread (to 32768) or up to four; logits in any order and in descending
     order, where a sample of neighbours would mislead."""
     x = logits_case("normal", n, seed=n)
     for k in (1, 2, 63, 64, 850, 1000):
