@@ -105,24 +105,23 @@ __global__ __launch_bounds__(kMvThreads) void k_matvec_q(const uint8_t* __restri
 
 // One to seven activation rows times a Q4 / Q8 weight, stored as Q8 rows by
 // the launch itself (k_matvec_q and write_rows in one): a workgroup owns the
-// 32 columns of one output block.  512 threads hold its weight blocks in
-// registers and park the lane terms in LDS; a ninth wavefront folds the
+// 32 columns of one output block.  512 or 960 threads hold its weight blocks in
+// registers and park the lane terms in LDS; one more wavefront folds the
 // chains and quantizes the block.
 //
 // What bounds it: latency.  One row (MULTI false): load, terms, one fold of
 // nb dependent adds (two chains per lane, 128 in all), the quantize.  More
 // rows (MULTI): the columns go in two halves of 16, each with a term buffer
 // of its own, and in phase t = 2 p + half the terms of t are computed while
-// the ninth wavefront folds those of t - 1, one barrier per phase; the next
+// that wavefront folds those of t - 1, one barrier per phase; the next
 // row is staged in the phase before it is used.
 // Measured with the fp32 pass it replaces (us): 1 row x 5632 x 2048 Q4 7.8 ->
 // 4.3; 5 rows x 5760 x 2304 Q8 20.8 -> 12.4 (the terms' reads of the staged
 // rows, 64 bytes of LDS per lane and block, set the pace there).
-constexpr int kMaTerm = 512;              // term threads
-constexpr int kMaThreads = kMaTerm + kWave;
+constexpr int kMaNarrow = 512, kMaWide = 960;  // term threads
 
-template <int WT, int IH, bool MULTI>
-__global__ __launch_bounds__(kMaThreads) void k_matvec_qa(const uint8_t* __restrict__ x, int x_pitch, int n_xrows,
+template <int WT, int IH, bool MULTI, int kMaTerm>
+__global__ __launch_bounds__(kMaTerm + kWave) void k_matvec_qa(const uint8_t* __restrict__ x, int x_pitch, int n_xrows,
                                                           const uint32_t* __restrict__ wq,
                                                           const uint16_t* __restrict__ wd, uint8_t* __restrict__ out,
                                                           int out_pitch, int N, int nb)
@@ -282,22 +281,26 @@ static int matvec_qa(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor*
 {
     const int N = w->rows, nb = w->cols / 32;
     const dim3 grid((N + 31) / 32);
-    auto go = [&](auto kern, bool multi) {
+    auto go = [&](auto kern, bool multi, int term) {
         const size_t lds = matvec_qa_lds(nb, multi);
-        hipLaunchKernelGGL(kern, grid, dim3(kMaThreads), lds, st, x, x_pitch, n_rows, (const uint32_t*)w->data,
+        hipLaunchKernelGGL(kern, grid, dim3(term + kWave), lds, st, x, x_pitch, n_rows, (const uint32_t*)w->data,
                            (const uint16_t*)w->deltas, out, out_pitch, N, nb);
         return launch_status("k_matvec_qa");
     };
     auto by_items = [&](auto wt, auto multi) {
         constexpr int WT = decltype(wt)::value;
         constexpr bool M = decltype(multi)::value;
-        const int ih = (16 * nb + kMaTerm - 1) / kMaTerm;  // weight blocks per thread and half
-        if (ih <= 1) return go(k_matvec_qa<WT, 1, M>, M);
-        if (ih <= 2) return go(k_matvec_qa<WT, 2, M>, M);
-        if (ih <= 3) return go(k_matvec_qa<WT, 3, M>, M);
-        if (ih <= 4) return go(k_matvec_qa<WT, 4, M>, M);
-        if (ih <= 6) return go(k_matvec_qa<WT, 6, M>, M);
-        return go(k_matvec_qa<WT, 8, M>, M);
+        // Weight blocks per thread and half.  More than three (K from 3104) go
+        // to 960 threads, which hold and convert three each instead of six (of
+        // Q8 some spilled): an MLP layer of five Q8 rows (K = 5760) 61.6 ->
+        // 59.7 us, of one Q4 row (K = 5632) 27.6-28.3, as before.  At three,
+        // 960 threads of two were slower (K = 2304: 61.4 for the same layer).
+        const int ih = (16 * nb + kMaNarrow - 1) / kMaNarrow, ihw = (16 * nb + kMaWide - 1) / kMaWide;
+        if (ih <= 1) return go(k_matvec_qa<WT, 1, M, kMaNarrow>, M, kMaNarrow);
+        if (ih <= 2) return go(k_matvec_qa<WT, 2, M, kMaNarrow>, M, kMaNarrow);
+        if (ih <= 3) return go(k_matvec_qa<WT, 3, M, kMaNarrow>, M, kMaNarrow);
+        if (ihw <= 3) return go(k_matvec_qa<WT, 3, M, kMaWide>, M, kMaWide);
+        return go(k_matvec_qa<WT, 5, M, kMaWide>, M, kMaWide);
     };
     auto by_rows = [&](auto wt) {
         return n_rows > 1 ? by_items(wt, std::true_type{}) : by_items(wt, std::false_type{});

@@ -184,6 +184,11 @@ FEW_CASES = [
     (Q8, 64, 33, 7, 0),
     (Q8, 2304, 100, 5, 1),
     (Q4, 5632, 64, 2, 0),
+    # either side of the 960-thread workgroups' lines (96, 180 and 256 blocks)
+    (Q8, 3072, 70, 2, 0),
+    (Q8, 3104, 70, 2, 0),
+    (Q4, 5792, 40, 7, 0),
+    (Q8, 5760, 33, 7, 0),
     (Q8, 7168, 48, 3, 0),
     (Q4, 7200, 48, 3, 0),
 ]
