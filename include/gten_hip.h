@@ -165,6 +165,10 @@ float nc_seq_sum_grid_host(const float* x, int n, int plant, int* passes);
  * recomputation; when fixups (device int) is not null, each workgroup that
  * recomputed adds one to it.  Results are the same for every skew > 0. */
 int nc_debug_spec(float skew, void* fixups);
+/* Test hook, on the host: the kernel nc_matmul_2d takes for rows x [N x K] of
+ * these dtypes, ", rows" after it where its launch stores activation rows
+ * itself (valid until the thread's next call). */
+const char* nc_debug_matmul_route(int x_dtype, int w_dtype, int out_dtype, int rows, int N, int K);
 /* Greedy pick of greedy_sample (src/gten/sampler.cpp:33-41): first index of
  * the maximum. */
 int nc_argmax(const float* x, int n, int32_t* out, void* stream);

@@ -29,6 +29,7 @@
 // lanes of a row meet through wavefront shuffles.
 #include <hip/hip_ext.h>
 
+#include <cstdio>
 #include <type_traits>
 
 #include "nc_kernels.h"
@@ -267,19 +268,55 @@ static size_t matvec_qa_lds(int nb, bool multi)
     return ((size_t)(multi ? 2 : 1) * nb * kStage + (size_t)128 * tp) * 4;
 }
 
-// Whether k_matvec_qa takes this product: rows below the prefill matmul's,
-// and shared memory and registers for its blocks.
-static bool matvec_qa_supported(int n_rows, const nc_tensor* w)
+// The k_matvec_qa launch of a product: its term threads and their weight blocks
+// per half; items 0 where k_matvec_q and a pass that quantizes its fp32 rows
+// (k_write_rows) take less time, or k_matvec_qa cannot hold the blocks.
+struct QaShape {
+    int term, items;
+};
+
+// The lines, measured back to back with cold weights on MI355X (us, staged /
+// direct):
+//  * k_matvec_q runs 1024 workgroups of four columns at once, so past 4096
+//    columns its time steps up by half and k_matvec_qa wins at any row count:
+//    7 rows x 4096 x 4096 Q4 17.4 / 17.3, x 5632 25.8 / 17.7; 7 x 5632 x 5632 Q8
+//    33.3 / 28.0.
+//  * up to there k_matvec_qa leaves CUs idle (a workgroup per 32 columns, its
+//    rows in turn), for a time that grows with the rows, the blocks of the
+//    fold's chain and the blocks per thread: the fewest columns it wins at are
+//    linear in work = rows nb^2.  Q4: 4 rows x 2048 x 4096 11.3 / 11.2, 5 rows 12.7 /
+//    13.1; 1 x 768 x 5632 6.6 / 6.6, 256 columns 5.9 / 6.4.  Q8 blocks take twice
+//    the registers and LDS reads, so its lines lie higher, the more so past two
+//    blocks per thread: 3 x 768 x 2048 7.6 / 7.5, 4 rows 8.6 / 8.7; 1 x 1024 x 2304
+//    5.9 / 6.2, 2 x 2048 x 2304 7.9 / 7.8; and past three only tall weights win
+//    (1 x 2048 x 3584 7.0 / 7.8), as Q4's past 180 blocks (1 x 2048 x 7680 8.0 / 8.3).
+//  * 960 threads instead of 512 pay past five blocks per thread (1 x 2048 x
+//    5632 Q4 7.6 with 512, 6.9 with 960; 1 x 2048 x 4096 5.5 / 6.0): below, the
+//    extra wavefronts only wait for the fold.  Q8 past 180 blocks would spill
+//    (2 x 2048 x 7680: 32 with five blocks per thread, 17.6 with four, staged 11.4).
+static QaShape qa_shape(int n_rows, const nc_tensor* w)
 {
-    const int nb = w->cols / 32;
-    return (w->dtype == NC_Q4 || w->dtype == NC_Q8) && w->cols > 0 && w->cols % 32 == 0 && w->rows > 0 && n_rows >= 1 &&
-           n_rows < kGemmMinRows && nb <= 256 && matvec_qa_lds(nb, n_rows > 1) <= 160 * 1024;
+    const int N = w->rows, nb = w->cols / 32;
+    const bool q4 = w->dtype == NC_Q4;
+    if ((!q4 && w->dtype != NC_Q8) || w->cols <= 0 || w->cols % 32 || N <= 0 || n_rows < 1 || n_rows >= kGemmMinRows)
+        return {0, 0};
+    if (nb > (q4 ? 256 : 180) || matvec_qa_lds(nb, n_rows > 1) > 160 * 1024) return {0, 0};
+    if (N <= 4096) {
+        const int work = n_rows * nb * nb;
+        const bool wins = q4         ? nb <= 180 && 22 * N >= work - 20000
+                          : nb <= 64 ? 8 * N >= work - 6000
+                                     : nb <= 96 && 16 * (N - 1400) >= work;
+        if (!wins) return {0, 0};
+    }
+    const int term = nb > 160 ? kMaWide : kMaNarrow;
+    return {term, (16 * nb + term - 1) / term};
 }
 
 static int matvec_qa(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, uint8_t* out, int out_pitch,
                      hipStream_t st)
 {
     const int N = w->rows, nb = w->cols / 32;
+    const QaShape shape = qa_shape(n_rows, w);
     const dim3 grid((N + 31) / 32);
     auto go = [&](auto kern, bool multi, int term) {
         const size_t lds = matvec_qa_lds(nb, multi);
@@ -290,17 +327,23 @@ static int matvec_qa(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor*
     auto by_items = [&](auto wt, auto multi) {
         constexpr int WT = decltype(wt)::value;
         constexpr bool M = decltype(multi)::value;
-        // Weight blocks per thread and half.  More than three (K from 3104) go
-        // to 960 threads, which hold and convert three each instead of six (of
-        // Q8 some spilled): an MLP layer of five Q8 rows (K = 5760) 61.6 ->
-        // 59.7 us, of one Q4 row (K = 5632) 27.6-28.3, as before.  At three,
-        // 960 threads of two were slower (K = 2304: 61.4 for the same layer).
-        const int ih = (16 * nb + kMaNarrow - 1) / kMaNarrow, ihw = (16 * nb + kMaWide - 1) / kMaWide;
-        if (ih <= 1) return go(k_matvec_qa<WT, 1, M, kMaNarrow>, M, kMaNarrow);
-        if (ih <= 2) return go(k_matvec_qa<WT, 2, M, kMaNarrow>, M, kMaNarrow);
-        if (ih <= 3) return go(k_matvec_qa<WT, 3, M, kMaNarrow>, M, kMaNarrow);
-        if (ihw <= 3) return go(k_matvec_qa<WT, 3, M, kMaWide>, M, kMaWide);
-        return go(k_matvec_qa<WT, 5, M, kMaWide>, M, kMaWide);
+        if (shape.term == kMaWide) {
+            if (shape.items == 3) return go(k_matvec_qa<WT, 3, M, kMaWide>, M, kMaWide);
+            if constexpr (WT == Q4) {
+                if (shape.items == 4) return go(k_matvec_qa<WT, 4, M, kMaWide>, M, kMaWide);
+                if constexpr (!M)  // several rows' shared memory ends at four
+                    if (shape.items == 5) return go(k_matvec_qa<WT, 5, M, kMaWide>, M, kMaWide);
+            }
+        } else {
+            switch (shape.items) {
+            case 1: return go(k_matvec_qa<WT, 1, M, kMaNarrow>, M, kMaNarrow);
+            case 2: return go(k_matvec_qa<WT, 2, M, kMaNarrow>, M, kMaNarrow);
+            case 3: return go(k_matvec_qa<WT, 3, M, kMaNarrow>, M, kMaNarrow);
+            case 4: return go(k_matvec_qa<WT, 4, M, kMaNarrow>, M, kMaNarrow);
+            case 5: return go(k_matvec_qa<WT, 5, M, kMaNarrow>, M, kMaNarrow);
+            }
+        }
+        return fail(NC_ERR_ARG, "matvec to Q8 rows: [%d x %d] weights, %d rows", N, w->cols, n_rows);
     };
     auto by_rows = [&](auto wt) {
         return n_rows > 1 ? by_items(wt, std::true_type{}) : by_items(wt, std::false_type{});
@@ -1073,17 +1116,22 @@ bool overlap(const void* a, size_t na, const void* b, size_t nb)
     return a && b && x < y + nb && y < x + na;
 }
 
-// Whether the launch that computes x [rows] times w can store out's
-// activation rows itself: a launch that does (gemm_q_act's, k_matvec_qa's, the
-// fp16 ones), and no output byte that the product still reads (a staged product
-// has read everything before it writes).
+// Whether a launch that computes x rows times w can store activation rows of
+// out_dtype itself: gemm_q_act's, k_matvec_qa's, the fp16 ones.
+bool direct_rows(int x_dtype, int x_pitch, int rows, const nc_tensor* w, int out_dtype)
+{
+    if (out_dtype != x_dtype || w->cols <= 0) return false;
+    if (x_dtype == NC_Q8) return gemm_q_act_supported(x_pitch, rows, w) || qa_shape(rows, w).items;
+    return x_dtype == NC_F16 && w->dtype == NC_F16 && f16_shape_ok(w);
+}
+
+// Whether this call's launch stores out's rows itself: such a launch, and no
+// output byte that the product still reads (a staged product has read
+// everything before it writes).
 bool stores_rows(const nc_tensor* x, const uint8_t* xr, const nc_tensor* w, const nc_tensor* out, const uint8_t* orow,
                  int rows)
 {
-    if (out->dtype != x->dtype || x->cols <= 0) return false;
-    if (x->dtype == NC_Q8 ? !gemm_q_act_supported(x->pitch, rows, w) && !matvec_qa_supported(rows, w)
-                          : x->dtype != NC_F16 || w->dtype != NC_F16 || !f16_shape_ok(w))
-        return false;
+    if (!direct_rows(x->dtype, x->pitch, rows, w, out->dtype)) return false;
     const size_t on = (size_t)rows * out->pitch;
     size_t cb, db;
     if (nc_weight_bytes(w->dtype, w->rows, w->cols, &cb, &db)) return false;
@@ -1111,6 +1159,9 @@ int matmul_2d(const char* name, const nc_tensor* x, const nc_tensor* w, nc_tenso
         NC_CHECK_ARG(out->pitch % 4 == 0, "%s: fp32 pitch %d", name, out->pitch);
         return matvec_raw(xr, x->dtype, x->pitch, rows, w, (float*)orow, out->pitch / 4, st);
     }
+    // staging comes first, also where the launch will not need it: what a call
+    // allocates or refuses then depends on its sizes alone, and a call warmed up
+    // before a capture has its staging whichever route a later one takes
     float* sp = nullptr;
     int s = stage((size_t)rows * w->rows * 4, rows, &sp);
     if (s) return s;
@@ -1145,4 +1196,24 @@ extern "C" int nc_matmul_2d(const nc_tensor* x, const nc_tensor* w, nc_tensor* o
 {
     return matmul_2d("matmul_2d", x, w, out, start, n_ctx, stream,
                      [&](size_t need, int, float** p) { return stage_buffer(need, p); });
+}
+
+// The kernel that nc_matmul_2d takes for a product of whole, aligned tensors
+// that do not overlap, and how its rows are stored.
+extern "C" const char* nc_debug_matmul_route(int x_dtype, int w_dtype, int out_dtype, int rows, int N, int K)
+{
+    static thread_local char name[64];
+    static const uint64_t aligned[2] = {0, 0};
+    const nc_tensor w{(void*)aligned, (void*)aligned, w_dtype, N, K, 0};
+    const int pitch = nc_act_pitch(x_dtype, K);
+    const bool direct = out_dtype != NC_F32 && direct_rows(x_dtype, pitch, rows, &w, out_dtype);
+    const char* tail = out_dtype == NC_F32 ? "" : direct ? ", rows" : " + k_write_rows";
+    if (w_dtype != NC_F16 && rows < kGemmMinRows) {
+        const QaShape q = qa_shape(rows, &w);
+        if (direct) snprintf(name, sizeof name, "k_matvec_qa %dx%d%s", q.term, q.items, tail);
+        else snprintf(name, sizeof name, "k_matvec_q%s", tail);
+    } else {
+        snprintf(name, sizeof name, "%s%s", w_dtype == NC_F16 ? "fp16" : "gemm", tail);
+    }
+    return name;
 }

@@ -173,10 +173,10 @@ def test_matmul_f16_rows(gpu, oracle, K, N, rows, start, odt):
 
 
 FEW_CASES = [
-    # (w dtype, K, N, rows, start): one to seven rows stored as Q8 rows by the
-    # launch: one block, a part of a thread's last item, the shared memory
-    # limit for several rows (224 blocks) and past it (the staged route), a
-    # partial last output block
+    # (w dtype, K, N, rows, start): one to seven rows to Q8 rows, on either
+    # side of the lines between k_matvec_qa and the staged route: one block, a
+    # part of a thread's last item, a partial last output block, every K on the
+    # staged route too
     (Q4, 32, 40, 1, 0),
     (Q4, 2304, 2304, 1, 2),
     (Q8, 5760, 70, 1, 0),
@@ -184,7 +184,6 @@ FEW_CASES = [
     (Q8, 64, 33, 7, 0),
     (Q8, 2304, 100, 5, 1),
     (Q4, 5632, 64, 2, 0),
-    # either side of the 960-thread workgroups' lines (96, 180 and 256 blocks)
     (Q8, 3072, 70, 2, 0),
     (Q8, 3104, 70, 2, 0),
     (Q4, 5792, 40, 7, 0),
@@ -192,6 +191,49 @@ FEW_CASES = [
     (Q8, 7168, 48, 3, 0),
     (Q4, 7200, 48, 3, 0),
 ]
+
+
+FEW_ROUTES = [
+    # (w dtype, K, N, rows, route): every workgroup of k_matvec_qa, one row and
+    # several, at the first N its line takes; the last K that several rows'
+    # shared memory holds (240 blocks) and the next, the last Q8 K (180 blocks)
+    # and the next
+    (Q4, 1024, 300, 2, "k_matvec_qa 512x1, rows"),
+    (Q4, 1280, 260, 1, "k_matvec_qa 512x2, rows"),
+    (Q4, 3072, 260, 2, "k_matvec_qa 512x3, rows"),
+    (Q4, 4096, 97, 1, "k_matvec_qa 512x4, rows"),
+    (Q4, 4096, 581, 2, "k_matvec_qa 512x4, rows"),
+    (Q4, 4096, 580, 2, "k_matvec_q + k_write_rows"),
+    (Q4, 5120, 260, 1, "k_matvec_qa 512x5, rows"),
+    (Q4, 5120, 1420, 2, "k_matvec_qa 512x5, rows"),
+    (Q4, 5760, 570, 1, "k_matvec_qa 960x3, rows"),
+    (Q4, 5632, 4097, 7, "k_matvec_qa 960x3, rows"),
+    (Q4, 7680, 4097, 1, "k_matvec_qa 960x4, rows"),
+    (Q4, 7680, 4097, 2, "k_matvec_qa 960x4, rows"),
+    (Q4, 7712, 4097, 2, "k_matvec_q + k_write_rows"),
+    (Q4, 8192, 4097, 1, "k_matvec_qa 960x5, rows"),
+    (Q4, 8192, 100, 3, "k_matvec_q + k_write_rows"),
+    (Q8, 1024, 300, 1, "k_matvec_qa 512x1, rows"),
+    (Q8, 2048, 786, 3, "k_matvec_qa 512x2, rows"),
+    (Q8, 2048, 785, 3, "k_matvec_q + k_write_rows"),
+    (Q8, 2304, 1724, 1, "k_matvec_qa 512x3, rows"),
+    (Q8, 2304, 2048, 2, "k_matvec_qa 512x3, rows"),
+    (Q8, 2304, 2047, 2, "k_matvec_q + k_write_rows"),
+    (Q8, 3104, 4096, 1, "k_matvec_q + k_write_rows"),
+    (Q8, 3104, 4097, 1, "k_matvec_qa 512x4, rows"),
+    (Q8, 4096, 4097, 3, "k_matvec_qa 512x4, rows"),
+    (Q8, 5120, 4100, 1, "k_matvec_qa 512x5, rows"),
+    (Q8, 5120, 4100, 2, "k_matvec_qa 512x5, rows"),
+    (Q8, 5760, 4100, 1, "k_matvec_qa 960x3, rows"),
+    (Q8, 5760, 4100, 7, "k_matvec_qa 960x3, rows"),
+    (Q8, 5792, 4100, 2, "k_matvec_q + k_write_rows"),
+]
+
+
+@pytest.mark.parametrize("wdt,K,N,rows,route", FEW_ROUTES)
+def test_matmul_few_rows_routes(gpu, oracle, wdt, K, N, rows, route):
+    assert gpu.lib().nc_debug_matmul_route(Q8, wdt, Q8, rows, N, K).decode() == route
+    test_matmul_few_rows(gpu, oracle, wdt, K, N, rows, 0)
 
 
 @pytest.mark.parametrize("wdt,K,N,rows,start", FEW_CASES)

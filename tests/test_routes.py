@@ -1,0 +1,39 @@
+"""The dispatch rules at sizes where both sides were measured, on the CPU.
+
+Each case is a call, the kernel its rule must take, and the times on one MI355X
+(us: the kernel the rule takes, the one it passes over).
+"""
+import pytest
+
+import oracle_lib as OL
+
+Q8, Q4, F16, F32 = OL.Q8, OL.Q4, OL.F16, OL.F32
+
+MATMUL = [
+    # (w dtype, rows, N, K, route): Q8 rows in and out
+    (Q4, 1, 2048, 2048, "k_matvec_qa 512x2, rows"),  # 4.1, staged 6.1
+    (Q4, 1, 256, 2048, "k_matvec_qa 512x2, rows"),  # 3.7, staged 4.5
+    (Q4, 1, 2048, 4096, "k_matvec_qa 512x4, rows"),  # 5.5, 960 threads 6.0, staged 6.8
+    (Q4, 5, 2048, 4096, "k_matvec_q + k_write_rows"),  # 12.7, direct 13.1
+    (Q4, 1, 2048, 5632, "k_matvec_qa 960x3, rows"),  # 6.9, 512 threads 7.6, staged 7.4
+    (Q4, 7, 2048, 5632, "k_matvec_q + k_write_rows"),  # 18.9, direct 23.0
+    (Q4, 7, 5632, 5632, "k_matvec_qa 960x3, rows"),  # 24.0, staged 32.3
+    (Q4, 7, 2048, 7680, "k_matvec_q + k_write_rows"),  # 22.5, direct 29.1
+    (Q4, 5, 320, 1280, "k_matvec_qa 512x2, rows"),  # 8.2, staged 8.7
+    (Q4, 1, 2048, 7680, "k_matvec_q + k_write_rows"),  # 8.0, direct 8.3
+    (Q8, 1, 256, 2048, "k_matvec_qa 512x2, rows"),  # 5.0, staged 7.3 (launch included)
+    (Q8, 1, 1024, 2304, "k_matvec_q + k_write_rows"),  # 5.9, direct 6.2
+    (Q8, 2, 5632, 2048, "k_matvec_qa 512x2, rows"),  # 7.0, staged 10.6
+    (Q8, 7, 2048, 2304, "k_matvec_q + k_write_rows"),  # 13.7, direct 15.0
+    (Q8, 1, 2048, 4096, "k_matvec_q + k_write_rows"),  # 7.2, direct 8.1
+    (Q8, 1, 2048, 5632, "k_matvec_q + k_write_rows"),  # 7.9, direct 10.4
+    (Q8, 5, 2304, 5760, "k_matvec_q + k_write_rows"),  # 17.3, direct 22.5
+    (Q8, 5, 5632, 5632, "k_matvec_qa 960x3, rows"),  # 22.7, staged 26.4
+    (Q8, 2, 2048, 7680, "k_matvec_q + k_write_rows"),  # 11.3, direct 21.4
+    (Q8, 1, 8192, 8192, "k_matvec_q + k_write_rows"),  # 19.1, direct 22.1
+]
+
+
+@pytest.mark.parametrize("wdt,rows,N,K,route", MATMUL)
+def test_few_row_products_take_the_faster_route(nc, wdt, rows, N, K, route):
+    assert nc.lib().nc_debug_matmul_route(Q8, wdt, Q8, rows, N, K).decode() == route
