@@ -169,6 +169,9 @@ int nc_debug_spec(float skew, void* fixups);
  * these dtypes, ", rows" after it where its launch stores activation rows
  * itself (valid until the thread's next call). */
 const char* nc_debug_matmul_route(int x_dtype, int w_dtype, int out_dtype, int rows, int N, int K);
+/* Test hook, on the host: the kernel nc_qkv_attn takes for rows [n_ctx - rows,
+ * n_ctx). */
+const char* nc_debug_attn_route(int dtype, int n_heads, int rows, int n_ctx);
 /* Greedy pick of greedy_sample (src/gten/sampler.cpp:33-41): first index of
  * the maximum. */
 int nc_argmax(const float* x, int n, int32_t* out, void* stream);

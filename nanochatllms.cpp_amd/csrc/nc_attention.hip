@@ -706,22 +706,42 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_rows(const uint8_t* __res
 // against 2048 on its vector unit before, then the chain of P.V products (32
 // cycles per 8 positions), the softmax's sequential sums (two rows side by
 // side on the halves of a wavefront) and its exponentials.  Shared memory
-// holds 16 rows of scores, so contexts past kFaMaxCtx keep k_attn_rows.
-// Measured (us): 1500 rows x 32 heads 792 -> 365, 2100 rows 1815 -> 654, 512
-// rows x 36 heads 82 -> 55, 100 rows after 600 61.6 -> 30.2; 128 rows 14.6 -> 13.7,
-// but 64 rows 7.7 -> 11.4, so shorter contexts keep k_attn_rows too.
+// holds 16 rows of scores, so contexts past kFaMaxCtx keep k_attn_rows; where
+// else it is slower, fa_takes says.  Measured (us, k_attn_rows / this): 1500 rows
+// x 32 heads 752 / 344, 512 x 36 heads 82 / 55, 100 rows up to position 700 x 32
+// heads 61 / 30.
 typedef float f16x_t __attribute__((ext_vector_type(16)));
 constexpr int kFaThreads = 512;
 constexpr int kFaRows = 16;
 constexpr int kFaChunk = 128;   // positions of K or V staged at a time
 constexpr int kFaStride = 144;  // bytes per staged position: 128 and a pad that spreads the banks
-constexpr int kFaMinCtx = 128, kFaMaxCtx = 2176;
+constexpr int kFaMaxCtx = 2176;
 
 // Floats per row of scores: a multiple of 64 and 4 more, so that 16 rows x 4
 // positions fall in 64 banks.
 __host__ __device__ constexpr int fa_row(int m) { return ((m + 63) & ~63) + 4; }
 constexpr size_t fa_lds(int m) { return (size_t)kFaRows * fa_row(m) * 4 + kFaChunk * kFaStride + 4 * 16 * 16 * 4; }
 static_assert(fa_lds(kFaMaxCtx) <= 160 * 1024, "shared memory of a CU");
+
+// Whether several fp16 rows take k_attn_f16 rather than k_attn_rows.  Its 16 x 16
+// tiles cut the work per row, but a workgroup runs a longer chain, so while
+// k_attn_rows' workgroups of four rows all run at once (704 of them, less than
+// three per CU) it loses at short contexts; the more of them, the sooner it wins.
+// Measured (us, k_attn_rows / k_attn_f16):
+//   800 workgroups (100 rows x 32 heads): 128 positions 14.8 / 13.9, 200 22.0 / 17.0;
+//     640 (128 x 20): 200 positions 15.4 / 16.2
+//   512 (64 x 32): 300 18.8 / 19.2, 400 22.6 / 21.4; 288 (33 x 32): 200 13.2 / 16.1, 512
+//     25.3 / 24.0
+//   128 (16 x 32): 128 10.0 / 12.9, 512 23.1 / 23.6, 600 26.2 / 26.0, 1000 39.6 / 37.0
+//   few rows of the tile, so a short softmax: 5 rows 200 12.4 / 12.4, 256 14.1 / 13.7;
+//     8 rows 300 15.9 / 16.8, 400 19.4 / 19.0
+inline bool fa_takes(int hq, int rows, int n_ctx)
+{
+    if (n_ctx > kFaMaxCtx) return false;
+    const int groups = hq * ((rows + 3) / 4);
+    const int from = groups > 704 ? 128 : rows <= 5 ? 256 : rows <= 8 || groups > 256 ? 400 : 600;
+    return n_ctx >= from;
+}
 
 __global__ __launch_bounds__(kFaThreads) void k_attn_f16(const uint8_t* __restrict__ q, int q_pitch,
                                                          const uint8_t* __restrict__ kc, int k_pitch,
@@ -935,7 +955,7 @@ int attn_go(const uint8_t* q, int q_pitch, const uint8_t* kc, int k_pitch, const
         // prefill: several query rows per workgroup, fewer for long rows
         // (their scores stay within 32 KB of shared memory)
         const int m = n_ctx;  // the last group attends at most n_ctx positions
-        if (ADT == F16 && m >= kFaMinCtx && m <= kFaMaxCtx) {
+        if (ADT == F16 && fa_takes(hq, rows, m)) {
             const dim3 grid(hq, (rows + kFaRows - 1) / kFaRows);
             hipLaunchKernelGGL(k_attn_f16, grid, dim3(kFaThreads), fa_lds(m), st, q, q_pitch, kc, k_pitch, vc, v_pitch,
                                out, out_pitch, hq, hkv, start, n_ctx, rows, scale);
@@ -1008,4 +1028,11 @@ extern "C" int nc_qkv_attn(const nc_tensor* q, const nc_tensor* k, const nc_tens
                        (const uint8_t*)k->data, k->pitch, (const uint8_t*)v->data, v->pitch,
                        (uint8_t*)out->data + (size_t)start * out->pitch, out->pitch, n_heads, n_kv_heads, start, n_ctx,
                        stream_of(stream), nullptr, n_ctx);
+}
+
+// The kernel that nc_qkv_attn takes for rows [n_ctx - rows, n_ctx).
+extern "C" const char* nc_debug_attn_route(int dtype, int n_heads, int rows, int n_ctx)
+{
+    if (rows == 1) return n_ctx >= kA1MinCtx && n_ctx <= kA1MaxCtx ? "k_attn1" : "k_attn";
+    return dtype == NC_F16 && fa_takes(n_heads, rows, n_ctx) ? "k_attn_f16" : "k_attn_rows";
 }

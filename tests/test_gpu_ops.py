@@ -469,9 +469,8 @@ ATTN_CASES = [
     (F16, 2, 1, 255, 254),
     (F16, 2, 2, 513, 512),
     (F16, 3, 3, 1023, 1022),
-    # several fp16 rows on the matrix cores: one tile and parts of it, rows
-    # across a tile's and a chunk's edge, every n mod 8, the longest context
-    # it takes and the next
+    # several fp16 rows of few heads and at most 600 positions, which keep
+    # k_attn_rows; the longest context that k_attn_f16 takes and the next
     (F16, 2, 1, 2, 0),
     (F16, 2, 2, 129, 112),
     (F16, 4, 2, 143, 5),
@@ -495,6 +494,32 @@ def test_qkv_attn(gpu, oracle, dt, hq, hkv, n, start):
     gpu.check(gpu.lib().nc_qkv_attn(C.byref(dq.t), C.byref(dk.t), C.byref(dv.t), C.byref(out.t), hq, hkv, 64, start,
                                     n, None), "qkv_attn")
     assert_same(out.ref()[start:], want[start:], "qkv_attn")
+
+
+F16_TILE_CASES = [
+    # (n_heads, n_kv_heads, n_ctx, start) that k_attn_f16 takes: a tile from its
+    # first row, parts of a tile, rows across a tile's edge, contexts at a staged
+    # chunk's edges (128 positions), every n mod 8, prompts from position 0
+    (64, 8, 128, 80),
+    (64, 64, 129, 75),
+    (36, 36, 143, 5),
+    (64, 8, 131, 0),
+    (2, 1, 256, 254),
+    (2, 2, 261, 256),
+    (2, 1, 406, 398),
+    (4, 2, 607, 590),
+    (3, 1, 639, 606),
+    (2, 1, 640, 624),
+    (2, 2, 641, 625),
+    (2, 1, 644, 627),
+    (2, 2, 2176, 2159),
+]
+
+
+@pytest.mark.parametrize("hq,hkv,n,start", F16_TILE_CASES)
+def test_qkv_attn_f16_tiles(gpu, oracle, hq, hkv, n, start):
+    assert gpu.lib().nc_debug_attn_route(F16, hq, n - start, n).decode() == "k_attn_f16"
+    test_qkv_attn(gpu, oracle, F16, hq, hkv, n, start)
 
 
 @pytest.mark.parametrize("wdt", [Q4, Q8, F16])

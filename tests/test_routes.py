@@ -37,3 +37,27 @@ MATMUL = [
 @pytest.mark.parametrize("wdt,rows,N,K,route", MATMUL)
 def test_few_row_products_take_the_faster_route(nc, wdt, rows, N, K, route):
     assert nc.lib().nc_debug_matmul_route(Q8, wdt, Q8, rows, N, K).decode() == route
+
+
+ATTN = [
+    # (dtype, heads, rows, n_ctx, kernel)
+    (F16, 32, 16, 128, "k_attn_rows"),  # 10.0, k_attn_f16 12.9
+    (F16, 12, 64, 200, "k_attn_rows"),  # 12.5, k_attn_f16 15.8
+    (F16, 20, 128, 200, "k_attn_rows"),  # 15.4, k_attn_f16 16.2
+    (F16, 32, 8, 300, "k_attn_rows"),  # 15.9, k_attn_f16 16.8
+    (F16, 32, 16, 512, "k_attn_rows"),  # 23.1, k_attn_f16 23.6
+    (F16, 32, 100, 128, "k_attn_f16"),  # 13.9, k_attn_rows 14.8
+    (F16, 32, 2, 256, "k_attn_f16"),  # 12.8, k_attn_rows 13.3
+    (F16, 32, 64, 400, "k_attn_f16"),  # 21.4, k_attn_rows 22.6
+    (F16, 32, 24, 1000, "k_attn_f16"),  # 36.8, k_attn_rows 40.3
+    (F16, 32, 1500, 1500, "k_attn_f16"),  # 344, k_attn_rows 752
+    (F16, 32, 8, 2177, "k_attn_rows"),  # its scores do not fit shared memory
+    (Q8, 32, 512, 512, "k_attn_rows"),
+    (F16, 32, 1, 512, "k_attn1"),  # 8.1, k_attn 9.6
+    (Q8, 32, 1, 255, "k_attn"),
+]
+
+
+@pytest.mark.parametrize("dtype,heads,rows,n_ctx,route", ATTN)
+def test_attention_takes_the_faster_route(nc, dtype, heads, rows, n_ctx, route):
+    assert nc.lib().nc_debug_attn_route(dtype, heads, rows, n_ctx).decode() == route
