@@ -43,8 +43,9 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 // NG 16-wide column groups per wavefront, NW wavefronts per workgroup (all
 // on the same rows, side by side in columns), MR groups of 4 rows (one MFMA
 // row operand each) per workgroup; the first 4 MR x kGmChunk threads stage
-// the activation blocks.  Kept for rows whose blocks do not come in fours and
-// for long prompts of tall weights without the chunk-major copy.
+// the activation blocks.  Kept for what k_gemm_qw does not take (gemm_shape): rows
+// whose blocks do not come in fours, weights not at whole dwords, operands of
+// 2 GiB and more.
 template <int WT, int NG, int NW, int MR, int PF>
 __global__ __launch_bounds__(64 * NW) void k_gemm_q(const uint8_t* __restrict__ x, int x_pitch, int n_rows,
                                                       const uint32_t* __restrict__ wq,
@@ -191,14 +192,12 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_q(const uint8_t* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // The same products with the lane sums taken on the fp16 matrix cores
-// (v_mfma_f32_16x16x32_f16): codes enter as fp16 integers (activation codes
-// -127..127, Q4 weights code - 7 in -7..8, Q8 weights -127..127), so each
-// product is an integer below 2^14 and each lane sum of eight products an
-// integer below 2^17.  Every partial sum the matrix core forms is then an
-// integer exactly representable in fp32, and the fp32 result is exactly
-// float(L_k): the conversion the integer path needs per lane and block is
-// gone, and the fold is 9 fp32 operations per (row, column, block) instead
-// of 13.
+// (v_mfma_f32_16x16x32_f16): codes enter as fp16 integers or exact sixteenths of
+// them (see k_gemm_qw), so that each product and each partial sum the matrix
+// core forms is an integer below 2^22, exactly representable in fp32, and the
+// fp32 result is exactly float(L_k): the conversion the integer path needs per
+// lane and block is gone, and the fold is 9 fp32 operations per (row, column,
+// block) instead of 13.
 //
 // The activation operand is staged once per workgroup already expanded: for
 // block j and row group m, lane l = (4r + k) + 16 g holds row 4m + r's lane-k
@@ -629,92 +628,133 @@ int chunk_layout_launch(const nc_tensor* w, void* codes, void* deltas, hipStream
 // Workgroup shapes, measured on MI355X (us per launch, every launch after a
 // 512 MB write that evicts L2 and the memory-side cache, as a prefill meets
 // its weights; over the chunk-major copy / the weight's own layout; Q4, Q8 in
-// brackets).  (MR, NG, NW); "before": one column group per wavefront, the
-// compiler's order of LDS reads and folds.
-//   512 rows x 11520 x 2304:  (4, 2, 4) 175 / 193 [199 / 210], before 258 /
-//       312 [305 / 310]; 6912 x 2304: 103 / 111 [115 / 124], before 152 / 214
-//       [182 / 212]; 2304 x 5760: 106 / 115 [112 / 123], before 134 / 195
-//       [161 / 194]
-//   201 rows x 5632 x 2048:  (4, 2, 4) 42 / 47 [47 / 54], before 55 / 77 [63 /
-//       75]
-//   128 rows x 6144 x 2048 (384 and 768 workgroups of 16 and 8 rows x 128
-//       columns):  (2, 2, 4) 29 / 38 [40 / 48], (4, 2, 4) 32 / 36 [36 / 38],
-//       (2, 1, 4) 32 / 43 [45 / 52], before 39 / 51 [42 / 50]
-//   201 rows x 2048 x 5632 (208 and 416):  (2, 2, 4) 51 / 59 [59 / 69], (2, 1,
-//       4) 48 / 54 [63 / 68], (4, 2, 4) 61 / 64 [67 / 72], before 66 / 76 [65 /
-//       79]
-//   100 rows x 2304 x 5760 (126 and 234):  (2, 1, 4) 37 / 41 [42 / 46], (2, 2,
-//       4) 42 / 47 [50 / 53], before 61 / 61 [51 / 62]
-//   64 rows x 2048 x 5632 (64 and 128):  (2, 1, 4) 27 / 30 [31 / 34], (2, 2, 4)
-//       44 / 45 [49 / 53], before 28 / 41 [31 / 42]; 2560 x 2048: (2, 1, 4) 15 /
-//       18 [18 / 20], before 17 / 23 [19 / 23]
-// At 512 x 11520 x 2304 the (4, 2, 4) launch issues a vector instruction in
-// 87% of the SIMDs' slots (counters); holding LDS operands two steps ahead
+// brackets).
+//   rows x N x K (groups)    8 x 32                     8 x 64
+//   16 x 2048 x 2048 (64)    12.2 / 12.8 [13.1 / 13.9]  12.2 / 13.6 [14.0 / 15.0]
+//   64 x 2560 x 2048 (320)   15.9 / 17.4 [17.6 / 20.1]  14.9 / 17.5 [17.9 / 21.1]
+//   128 x 2048 x 5632 (512)  35.8 / 38.8 [40.2 / 46.7]  33.4 / 37.2 [38.9 / 45.1]
+//   201 x 2048 x 2048 (832)  30.0 / 35.6 [36.9 / 43.8]  22.7 / 29.6 [32.0 / 37.8]
+//   128 x 6144 x 2048 (1536) 47.8 / 57.5 [59.0 / 68.8]  32.3 / 42.8 [45.9 / 55.2]
+//   512 x 6912 x 2304 (6912) 180 / 192 [203 / 220]      118 / 134 [163 / 171]
+//                            16 x 64                    16 x 128
+//   16 x 2048 x 2048         19.7 / 18.4 [21.2 / 22.6]  25.9 / 26.5 [28.3 / 30.7]
+//   64 x 2560 x 2048         19.3 / 18.9 [21.4 / 22.8]  25.0 / 26.6 [27.9 / 29.8]
+//   128 x 2048 x 5632        45.8 / 44.8 [50.2 / 52.6]  60.0 / 61.8 [66.0 / 71.6]
+//   201 x 2048 x 2048        22.7 / 23.9 [24.9 / 26.0]  26.1 / 28.1 [28.7 / 30.8]
+//   128 x 6144 x 2048        29.3 / 32.5 [32.6 / 37.2]  32.2 / 36.3 [36.6 / 39.8]
+//   512 x 6912 x 2304        109 / 118 [119 / 127]      99 / 109 [112 / 123]
+// 8 x 128 is not among them: of 1108 such calls it was the best by more than 3%
+// in one.  The kernel before (one column group per wavefront, the compiler's
+// order of LDS reads and folds): 201 x 2048 x 2048 27.0 / 31.5 [26.8 / 31.3], 512 x
+// 6912 x 2304 136 / 194 [162 / 194].  At 512 x 11520 x 2304 the 16 x 128 launch keeps
+// the vector unit busy (see the kernel); holding LDS operands two steps ahead
 // or taking the d_x d_w products from the matrix cores changed nothing there.
 //
-// The rule follows the workgroups a shape would have: 16 rows x 128 columns
-// from kWide16 of them (Q8's weight operands cost more to form, so it shares
-// them over 16 rows earlier), else 8 x 128 from kWide8, else 8 x 64.
-template <int WT>
-constexpr int kWide16 = WT == Q4 ? 448 : 320;
-constexpr int kWide8 = 400;
+// The rule follows the workgroups that 8 rows x 64 columns would have.  Up to
+// kTiny of them Q8 takes half the columns each, for twice as many (Q4, with half
+// the bytes to wait for, gains nothing: 8 x 1280 x 1280 9.4 / 9.6).  Up to three per
+// CU 8 x 64, whose time then steps up (Q8 plain 160 x 2560 x 2048, 800 of them:
+// 38.0, 16 x 64 26.1; 160 x 2304 x 2304, 720: 27.2 / 27.6); Q4 over the chunk-major
+// copy, with the cheapest operands, up to five.  Then 16 x 64, which shares the
+// converted weights over twice the rows, and from kBig 16 x 128, which shares
+// the activation operands too.
+constexpr int kTiny = 96, kBig = 1600;
+constexpr int small_groups(int dtype, bool cl) { return dtype == NC_Q4 && cl ? 1280 : 768; }
 
-static int wide_groups(int N, int n_rows, int rows) { return ((N + 127) / 128) * ((n_rows + rows - 1) / rows); }
+static int64_t groups8x64(int N, int n_rows) { return (int64_t)((N + 63) / 64) * ((n_rows + 7) / 8); }
 
-enum GemmShape { kGemmNone, kGemm8x64, kGemm8x128, kGemm16x128 };
+enum GemmShape { kGemmNone, kGemm8x32, kGemm8x64, kGemm8x128, kGemm16x64, kGemm16x128 };
 
 // The k_gemm_qw shape of this product, kGemmNone when it is not taken: its
 // chunks are four blocks, its loads need whole dwords, and its offsets are 32
-// bits.
-static GemmShape gemm_shape(int x_pitch, int n_rows, const nc_tensor* w)
+// bits.  cl: w is the chunk-major copy.
+static GemmShape gemm_shape(int x_pitch, int n_rows, const nc_tensor* w, bool cl)
 {
     const int N = w->rows, nb = w->cols / 32;
     const size_t lim = (size_t)1 << 31;
     if (w->cols % 128 || ((uintptr_t)w->data & 3) || ((uintptr_t)w->deltas & 3)) return kGemmNone;
     if ((size_t)N * nb * (w->dtype == NC_Q4 ? 16 : 32) >= lim || (size_t)n_rows * x_pitch >= lim) return kGemmNone;
-    if (wide_groups(N, n_rows, 16) >= (w->dtype == NC_Q4 ? kWide16<Q4> : kWide16<Q8>)) return kGemm16x128;
-    return wide_groups(N, n_rows, 8) >= kWide8 ? kGemm8x128 : kGemm8x64;
+    const int64_t groups = groups8x64(N, n_rows);
+    if (w->dtype == NC_Q8 && groups <= kTiny && nb % 8 == 0) return kGemm8x32;
+    if (groups <= small_groups(w->dtype, cl)) return kGemm8x64;
+    return groups <= kBig ? kGemm16x64 : kGemm16x128;
 }
 
-// cl: w is the chunk-major copy.
+// The shape that stores Q8 rows itself, kGemmNone where the fp32 product and
+// a pass that quantizes its rows take less time: a 32-column block needs both its
+// column groups in one wavefront, so 16 x 128 where that is the product's own
+// shape, else 8 x 128 for Q4 rows up to K = 2304, where it costs less than the
+// pass (us, 8 x 128 / 16 x 64 and the pass: 256 x 2048 x 1024 13.6 / 15.4, 160 x
+// 4096 x 1536 22.6 / 23.6, 33 x 11264 x 2048 25.9 / 29.0; 201 x 2048 x 5632 63 / 60; Q8
+// weights 201 x 2048 x 2048 35 / 30).
+static GemmShape gemm_act_shape(int x_pitch, int n_rows, const nc_tensor* w)
+{
+    const GemmShape shape = gemm_shape(x_pitch, n_rows, w, false);
+    if (shape == kGemm16x64 && w->dtype == NC_Q4 && w->cols <= 2304) return kGemm8x128;
+    return shape == kGemm16x128 ? shape : kGemmNone;
+}
+
 template <int ODT>
 static int gemm_qw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, bool cl, GemmShape shape, void* out,
                    int out_pitch, hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop)
 {
     const int N = w->rows, nb = w->cols / 32;
-    const int rows = shape == kGemm16x128 ? 16 : 8, cols = shape == kGemm8x64 ? 64 : 128;
+    const int rows = shape >= kGemm16x64 ? 16 : 8, cols = shape == kGemm8x32 ? 32 : shape == kGemm8x128 || shape == kGemm16x128 ? 128 : 64;
     auto go = [&](auto kern) {
-        const dim3 grid((N + cols - 1) / cols, (n_rows + rows - 1) / rows);
+        const dim3 grid((N + cols - 1) / cols, (n_rows + rows - 1) / rows), block(shape == kGemm8x32 ? 128 : 256);
         if (ev_start)
-            hipExtLaunchKernelGGL(kern, grid, dim3(256), 0, st, ev_start, ev_stop, 0, x, x_pitch, n_rows,
+            hipExtLaunchKernelGGL(kern, grid, block, 0, st, ev_start, ev_stop, 0, x, x_pitch, n_rows,
                                   (const uint32_t*)w->data, (const uint16_t*)w->deltas, out, out_pitch, N, nb);
         else
-            hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x, x_pitch, n_rows, (const uint32_t*)w->data,
+            hipLaunchKernelGGL(kern, grid, block, 0, st, x, x_pitch, n_rows, (const uint32_t*)w->data,
                                (const uint16_t*)w->deltas, out, out_pitch, N, nb);
     };
     auto by_layout = [&](auto wt, auto c) {
         constexpr int WT = decltype(wt)::value;
         constexpr bool CL = decltype(c)::value;
-        if (shape == kGemm16x128) go(k_gemm_qw<WT, 4, 2, 4, 4, 1, CL, 3, ODT>);
-        else if (shape == kGemm8x128) go(k_gemm_qw<WT, 2, 2, 4, 4, 1, CL, 4, ODT>);
-        else if constexpr (ODT == F32) {
-            if (nb % 8 == 0) go(k_gemm_qw<WT, 2, 1, 4, 8, 2, CL, 2, ODT>);
-            else go(k_gemm_qw<WT, 2, 1, 4, 4, 1, CL, 2, ODT>);
+        if (shape == kGemm16x128) return go(k_gemm_qw<WT, 4, 2, 4, 4, 1, CL, 3, ODT>);
+        if constexpr (ODT == Q8 && WT == Q4 && !CL) {
+            if (shape == kGemm8x128) return go(k_gemm_qw<WT, 2, 2, 4, 4, 1, CL, 4, ODT>);
+        }
+        if constexpr (ODT == F32) {
+            if (shape == kGemm16x64) return go(k_gemm_qw<WT, 4, 1, 4, 4, 1, CL, 2, ODT>);
+            if constexpr (WT == Q8)
+                if (shape == kGemm8x32) return go(k_gemm_qw<WT, 2, 1, 2, 8, 2, CL, 2, ODT>);
+            // eight blocks per barrier while the workgroups are few (64 x 2560 x
+            // 2048 Q4: 14.9, 16.1 with four), four where their smaller shared
+            // memory lets more of them share a CU (256 x 2048 x 2048: 22.9, 23.7
+            // with eight)
+            if (nb % 8 == 0 && groups8x64(N, n_rows) <= 512) return go(k_gemm_qw<WT, 2, 1, 4, 8, 2, CL, 2, ODT>);
+            return go(k_gemm_qw<WT, 2, 1, 4, 4, 1, CL, 2, ODT>);
         }
     };
     auto by_type = [&](auto wt) {
-        if (cl) by_layout(wt, std::true_type{});
-        else by_layout(wt, std::false_type{});
+        if constexpr (ODT == F32) {
+            if (cl) return by_layout(wt, std::true_type{});
+        }
+        by_layout(wt, std::false_type{});
     };
     if (w->dtype == NC_Q4) by_type(std::integral_constant<int, Q4>{});
     else by_type(std::integral_constant<int, Q8>{});
     return launch_status("k_gemm_qw");
 }
 
+const char* gemm_route(int x_pitch, int n_rows, const nc_tensor* w, bool act)
+{
+    switch (act ? gemm_act_shape(x_pitch, n_rows, w) : gemm_shape(x_pitch, n_rows, w, false)) {
+    case kGemm8x32: return "k_gemm_qw 8x32";
+    case kGemm8x64: return "k_gemm_qw 8x64";
+    case kGemm8x128: return "k_gemm_qw 8x128";
+    case kGemm16x64: return "k_gemm_qw 16x64";
+    case kGemm16x128: return "k_gemm_qw 16x128";
+    default: return "k_gemm_q";
+    }
+}
+
 bool gemm_q_act_supported(int x_pitch, int n_rows, const nc_tensor* w)
 {
     return (w->dtype == NC_Q4 || w->dtype == NC_Q8) && n_rows >= kGemmMinRows &&
-           gemm_shape(x_pitch, n_rows, w) >= kGemm8x128;
+           gemm_act_shape(x_pitch, n_rows, w) != kGemmNone;
 }
 
 int gemm_q_act(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, uint8_t* out, int out_pitch,
@@ -722,7 +762,7 @@ int gemm_q_act(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, ui
 {
     if (!gemm_q_act_supported(x_pitch, n_rows, w))
         return fail(NC_ERR_ARG, "gemm to Q8 rows: [%d x %d] weights, %d rows", w->rows, w->cols, n_rows);
-    return gemm_qw<Q8>(x, x_pitch, n_rows, w, false, gemm_shape(x_pitch, n_rows, w), out, out_pitch, st, nullptr,
+    return gemm_qw<Q8>(x, x_pitch, n_rows, w, false, gemm_act_shape(x_pitch, n_rows, w), out, out_pitch, st, nullptr,
                        nullptr);
 }
 
@@ -737,7 +777,7 @@ int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, fl
         return fail(NC_ERR_ARG, "gemm: chunk copy [%d x %d] of a [%d x %d] weight", wc->rows, wc->cols, N, w->cols);
     // the chunk-major copy, when the caller has one
     const nc_tensor* wt = wc ? wc : w;
-    if (const GemmShape shape = gemm_shape(x_pitch, n_rows, wt))
+    if (const GemmShape shape = gemm_shape(x_pitch, n_rows, wt, wc != nullptr))
         return gemm_qw<F32>(x, x_pitch, n_rows, wt, wc != nullptr, shape, out, out_pitch, st, ev_start, ev_stop);
     // (NG, NW, MR, PF): 512 rows (1, 2, 8, 4), tall weights (2, 2, 8, 3);
     // 64 rows (1, 1, 4, 3), tall (1, 2, 8, 4)

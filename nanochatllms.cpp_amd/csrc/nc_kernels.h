@@ -49,6 +49,9 @@ int gemm_q_raw(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, fl
 // The same product stored as Q8 activation rows (write_row_from_float of the
 // dots) by the launch itself; for the products whose launch can
 // (gemm_q_act_supported).
+// gemm_route: the name of the kernel and shape that gemm_q_act (act) or
+// gemm_q_raw over the weight's own layout takes.
+const char* gemm_route(int x_pitch, int n_rows, const nc_tensor* w, bool act);
 bool gemm_q_act_supported(int x_pitch, int n_rows, const nc_tensor* w);
 int gemm_q_act(const uint8_t* x, int x_pitch, int n_rows, const nc_tensor* w, uint8_t* out, int out_pitch,
                hipStream_t st);

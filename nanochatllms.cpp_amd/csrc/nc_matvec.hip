@@ -1213,7 +1213,7 @@ extern "C" const char* nc_debug_matmul_route(int x_dtype, int w_dtype, int out_d
         if (direct) snprintf(name, sizeof name, "k_matvec_qa %dx%d%s", q.term, q.items, tail);
         else snprintf(name, sizeof name, "k_matvec_q%s", tail);
     } else {
-        snprintf(name, sizeof name, "%s%s", w_dtype == NC_F16 ? "fp16" : "gemm", tail);
+        snprintf(name, sizeof name, "%s%s", w_dtype == NC_F16 ? "fp16" : gemm_route(pitch, rows, &w, direct), tail);
     }
     return name;
 }

@@ -97,6 +97,26 @@ def test_small_model_prefill_and_stream(gpu, oracle, name):
     m.close()
 
 
+@pytest.mark.parametrize("wdt,rows", [(OL.Q4, 9), (OL.Q4, 201), (OL.Q4, 350), (OL.Q4, 505), (OL.Q8, 9), (OL.Q8, 201),
+                                      (OL.Q8, 505)])
+def test_prefill_matmul_shapes(gpu, oracle, wdt, rows):
+    """Prompts whose products over the prefill's weight copy take every shape:
+    gate|up of 2048 rows as 8 x 64 columns with both chunk lengths (9 and 201
+    rows of Q4), 8 x 32 (9 of Q8), 16 x 64 (350 of Q4, 201 of Q8) and 16 x 128."""
+    w = dict(SMALL["small-llama-q4"], wdtype=wdt, n_layers=1, n_ffn=1024, prompt=rows, gen=4)
+    cfg = config_of(w)
+    prompt = np.random.default_rng(rows).integers(0, cfg.n_vocab, rows).astype(np.int32)
+    m = gpu.Model(config_of(w, cls=gpu.ModelConfig))
+    m.init_synthetic(w["seed"])
+    got = m.logits(prompt, 0)
+    om = oracle.model_create(cfg, w["seed"])
+    want = np.zeros(cfg.n_vocab, np.float32)
+    oracle.model_logits(om, OL.ptr(prompt), rows, 0, OL.ptr(want))
+    oracle.model_free(om)
+    m.close()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"rel-L2 {rel_l2(got, want):.3g}"
+
+
 FULL = ["tinyllama-q4", "tinyllama-q8", "openelm-q8", "zephyr-f16", "minicpm-q4", "tinyllama-f16", "zephyr-q4",
         "openelm-sm-q8", "openelm-md-q8", "zephyr-q8", "minicpm-q8", "minicpm-f16"]
 

@@ -114,11 +114,9 @@ def test_matmul_act_out(gpu, oracle, xdt, wdt, K, N):
 
 
 WIDE_CASES = [
-    # (w dtype, K, N, rows, start): the prefill matmul's launches of 16 rows x
-    # 128 columns per workgroup (Q4 from 448 workgroups, Q8 from 320), 8 x 128
-    # (from 400) and 8 x 64 (fewer, chunks of 8 and of 4 blocks): one, an odd
+    # (w dtype, K, N, rows, start): products of 8 rows and more: one, an odd
     # and an even number of chunks, rows and columns past a tile, a partial
-    # last block
+    # last block, Q8 rows stored by the launch and by a pass
     (Q4, 128, 1010, 903, 3),
     (Q4, 384, 4100, 225, 0),
     (Q8, 640, 2050, 310, 0),
@@ -143,6 +141,32 @@ def test_matmul_wide(gpu, oracle, wdt, K, N, rows, start, odt):
     gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), start, rows, None), "matmul")
     got = out.ref() if odt == Q8 else out.ref().view(np.float32)
     assert_same(got[start:], want[start:], f"matmul Q{8 if wdt == Q8 else 4} K={K} N={N} out {odt}")
+
+
+WIDE_ROUTES = [
+    # (w dtype, K, N, rows, out dtype, route): every shape of the prefill matmul
+    # over the weight's own layout, at its lines' edges
+    (Q8, 512, 1530, 32, F32, "k_gemm_qw 8x32"),
+    (Q8, 512, 1537, 32, F32, "k_gemm_qw 8x64"),
+    (Q8, 384, 70, 9, F32, "k_gemm_qw 8x64"),
+    (Q4, 256, 70, 9, F32, "k_gemm_qw 8x64"),
+    (Q4, 256, 2050, 150, F32, "k_gemm_qw 8x64"),
+    (Q8, 256, 3070, 128, Q8, "k_gemm_qw 8x64 + k_write_rows"),
+    (Q4, 384, 3073, 128, F32, "k_gemm_qw 16x64"),
+    (Q8, 640, 3075, 121, F32, "k_gemm_qw 16x64"),
+    (Q8, 128, 3075, 121, Q8, "k_gemm_qw 16x64 + k_write_rows"),
+    (Q4, 2304, 3080, 123, Q8, "k_gemm_qw 8x128, rows"),
+    (Q4, 2432, 3080, 121, Q8, "k_gemm_qw 16x64 + k_write_rows"),
+    (Q4, 128, 4097, 195, F32, "k_gemm_qw 16x128"),
+    (Q8, 256, 4100, 195, F32, "k_gemm_qw 16x128"),
+    (Q8, 384, 4100, 195, Q8, "k_gemm_qw 16x128, rows"),
+]
+
+
+@pytest.mark.parametrize("wdt,K,N,rows,odt,route", WIDE_ROUTES)
+def test_matmul_wide_routes(gpu, oracle, wdt, K, N, rows, odt, route):
+    assert gpu.lib().nc_debug_matmul_route(Q8, wdt, odt, rows, N, K).decode() == route
+    test_matmul_wide(gpu, oracle, wdt, K, N, rows, 0, odt)
 
 
 F16_CASES = [

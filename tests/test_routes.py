@@ -39,6 +39,26 @@ def test_few_row_products_take_the_faster_route(nc, wdt, rows, N, K, route):
     assert nc.lib().nc_debug_matmul_route(Q8, wdt, Q8, rows, N, K).decode() == route
 
 
+WIDE = [
+    # (w dtype, out dtype, rows, N, K, route)
+    (Q8, F32, 16, 2048, 2048, "k_gemm_qw 8x32"),  # 13.9, 8x64 15.0
+    (Q4, F32, 64, 2560, 2048, "k_gemm_qw 8x64"),  # 17.5, 16x64 18.9
+    (Q4, F32, 128, 2048, 5632, "k_gemm_qw 8x64"),  # 37.2, 16x64 44.8, 16x128 61.8
+    (Q8, F32, 201, 2048, 2048, "k_gemm_qw 16x64"),  # 26.0, 8x64 37.8, 8x128 33.4, 16x128 30.8
+    (Q8, F32, 256, 2048, 2048, "k_gemm_qw 16x64"),  # 26.6, 8x64 36.7, 8x128 35.1, 16x128 31.3
+    (Q8, F32, 16, 32000, 2048, "k_gemm_qw 16x64"),  # 34.4, 8x128 42.6, 16x128 37.4
+    (Q4, F32, 128, 6144, 2048, "k_gemm_qw 16x64"),  # 32.5, 16x128 36.3
+    (Q4, F32, 512, 6912, 2304, "k_gemm_qw 16x128"),  # 109, 16x64 118
+    (Q4, Q8, 256, 2048, 1024, "k_gemm_qw 8x128, rows"),  # 13.6, 16x64 and the pass 15.4
+    (Q8, Q8, 201, 2048, 2048, "k_gemm_qw 16x64 + k_write_rows"),  # 30.6, 8x128 35.0
+]
+
+
+@pytest.mark.parametrize("wdt,odt,rows,N,K,route", WIDE)
+def test_prefill_products_take_the_faster_shape(nc, wdt, odt, rows, N, K, route):
+    assert nc.lib().nc_debug_matmul_route(Q8, wdt, odt, rows, N, K).decode() == route
+
+
 ATTN = [
     # (dtype, heads, rows, n_ctx, kernel)
     (F16, 32, 16, 128, "k_attn_rows"),  # 10.0, k_attn_f16 12.9
