@@ -683,10 +683,10 @@ static GemmShape gemm_shape(int x_pitch, int n_rows, const nc_tensor* w, bool cl
 // The shape that stores Q8 rows itself, kGemmNone where the fp32 product and
 // a pass that quantizes its rows take less time: a 32-column block needs both its
 // column groups in one wavefront, so 16 x 128 where that is the product's own
-// shape, else 8 x 128 for Q4 rows up to K = 2304, where it costs less than the
-// pass (us, 8 x 128 / 16 x 64 and the pass: 256 x 2048 x 1024 13.6 / 15.4, 160 x
-// 4096 x 1536 22.6 / 23.6, 33 x 11264 x 2048 25.9 / 29.0; 201 x 2048 x 5632 63 / 60; Q8
-// weights 201 x 2048 x 2048 35 / 30).
+// shape, else 8 x 128 for Q4 weights up to K = 2304, where it costs less than the
+// pass (us back to back, 8 x 128 / 16 x 64 and the pass: 256 x 2048 x 1024 13.6 /
+// 15.4, 160 x 4096 x 1536 22.6 / 23.6, 33 x 11264 x 2048 25.9 / 29.0; 201 x 2048 x 5632
+// 56.2 / 53.3; Q8 weights 201 x 2048 x 2048 30.8 / 25.5).
 static GemmShape gemm_act_shape(int x_pitch, int n_rows, const nc_tensor* w)
 {
     const GemmShape shape = gemm_shape(x_pitch, n_rows, w, false);
