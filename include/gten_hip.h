@@ -172,6 +172,9 @@ const char* nc_debug_matmul_route(int x_dtype, int w_dtype, int out_dtype, int r
 /* Test hook, on the host: the kernel nc_qkv_attn takes for rows [n_ctx - rows,
  * n_ctx). */
 const char* nc_debug_attn_route(int dtype, int n_heads, int rows, int n_ctx);
+/* Test hook, on the host: the kernel of nc_rms_norm (layer 0) or
+ * nc_layer_norm for rows of d_norm values. */
+const char* nc_debug_norm_route(int layer, int dtype, int d_norm, int rows);
 /* Greedy pick of greedy_sample (src/gten/sampler.cpp:33-41): first index of
  * the maximum. */
 int nc_argmax(const float* x, int n, int32_t* out, void* stream);

@@ -146,20 +146,24 @@ __global__ __launch_bounds__(1024) void k_norm(const uint8_t* __restrict__ a, in
     }
 }
 
-// k_norm for segments of a multiple of 256 values in aligned rows: 256 threads
-// of eight values each (two slots past 2048), all of them in the exact sums.
-// What bounds it: the latency of those sums (2-3 us each), so a CU should
-// hold many rows at once; k_norm's 1024 threads, 768 of them waiting, left
-// it two.  Measured (us, 2048 values): rms_norm of Q8 rows, 1 row 6.1 -> 5.1,
-// 512 rows 12.0 -> 6.2, 1500 rows 31 -> 15; layer_norm of fp16 rows, 1500 rows
-// 96 -> 34.
+// k_norm for segments of a multiple of 256 values (512 and more) in aligned
+// rows: 256 threads of eight values each (two slots past 2048), all of them in
+// the exact sums.  What bounds it: the latency of those sums (2-3 us each, and
+// the whole loop's, 3 ns per value, for a row whose sum of squares falls back
+// or whose mean takes it), so a CU should hold many rows at once; k_norm's 1024
+// threads, 768 of them waiting, left it two.  Measured (us, k_norm / this):
+// rms_norm of Q8 rows of 2048, 1 row 6.2 / 5.2, 512 rows 17 / 11 (a row of them
+// falls back), 1500 rows 31 / 12-16; layer_norm of fp16 rows of 2304, 64 rows 13.4 /
+// 12.8, 1500 rows 72 / 28.  Slower only where k_norm's threads do not divide into
+// the block sum, which then cannot fall back after it: up to 256 rows of 1792,
+// 2560 or 3584 values one of which does (3584: 14.8 / 18.1; 7.7 where none does).
 template <int ADT, int KIND, bool ADD>
 __global__ __launch_bounds__(kSsThreads) void k_norm8(const uint8_t* __restrict__ a, int a_pitch,
                                                       const float* __restrict__ braw, int b_pitch, float bscale,
                                                       uint8_t* __restrict__ h_out, int h_pitch,
                                                       const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
                                                       uint8_t* __restrict__ out, int out_pitch, int n, int row_cols,
-                                                      float post_scale, const int* __restrict__ dpos)
+                                                      float post_scale, const int* __restrict__ dpos, bool grid_mean)
 {
     constexpr int kSlots = kNormMaxCols / 8 / kSsThreads;
     __shared__ __align__(16) float buf[kNormMaxCols];
@@ -203,14 +207,20 @@ __global__ __launch_bounds__(kSsThreads) void k_norm8(const uint8_t* __restrict_
     __syncthreads();
     float mean = 0.0f;
     if (KIND == kLayerNorm) {
-        float s1;
-        switch (n / kSsThreads) {
+        float s1 = 0.0f;
+        switch (grid_mean ? n / kSsThreads : 0) {
         case 4: s1 = block_seq_sum_grid<4, kSsThreads>(buf, sgh); break;
         case 5: s1 = block_seq_sum_grid<5, kSsThreads>(buf, sgh); break;
         case 6: s1 = block_seq_sum_grid<6, kSsThreads>(buf, sgh); break;
         case 8: s1 = block_seq_sum_grid<8, kSsThreads>(buf, sgh); break;
         case 9: s1 = block_seq_sum_grid<9, kSsThreads>(buf, sgh); break;
-        default: s1 = seq_sum(buf, n); break;
+        default:
+            if (tid < kWave) {
+                s1 = seq_sum(buf, n);
+                if (tid == 0) sgh.result = s1;
+            }
+            __syncthreads();
+            s1 = sgh.result;
         }
         mean = s1 / (float)n;
         __syncthreads();  // the values have been read
@@ -661,6 +671,24 @@ static bool fits8(int rows, int cols) { return (int64_t)rows * cols < ((int64_t)
 // 9.1 / 7.4.
 constexpr int kEw8Min = 1 << 18, kSilu8Min = 1 << 20;
 
+// The widths of k_norm8: at 256 values only a lane quad's worth of threads load,
+// and k_norm's 256 of one value each are 0.2 to 0.8 us faster.
+static bool norm8_takes(int d_norm) { return d_norm % kSsThreads == 0 && d_norm > kSsThreads; }
+
+// Whether k_norm8 takes a layer_norm's mean as the exact grid sum rather than
+// the loop: a pass per step that rounds, so a launch is as slow as its row with
+// the most of them (up to 48 passes and then the loop).  Rows of 2048 always do
+// (their loop's 6 us; k_norm's did as well).  Q8 rows, multiples of a few deltas'
+// grids, round rarely, so they do while they are few: 64 rows of 2304 8-11 us
+// against 13.5, 128 rows 18-24 against 13.6; 64 of 1536 8.6 / 11.4, 256 18-43 / 11.7;
+// of 1024 any number (1500 rows 15.6 / 19.4).
+// fp16 rows round often: one row of 1024 or 1280 7.2-8.9 / 8.4-9.5, 4 rows 9.3-10.2 /
+// 8.4-9.5, one of 2304 10.3-14.9 / 12.3.
+static bool norm8_grid_mean(int adt, int d_norm, int segments)
+{
+    return d_norm == 2048 || (adt == NC_Q8 && d_norm == 1024) || (int64_t)segments * d_norm <= (adt == NC_Q8 ? 150000 : 1280);
+}
+
 // Threads per norm workgroup: the largest multiple of 64 up to 1024 that
 // divides the segment (each thread then owns n / bs values).
 static int norm_block(int n)
@@ -681,13 +709,14 @@ int norm_launch(int kind, int adt, bool add, const uint8_t* a, int a_pitch, cons
     if (adt != NC_Q8 && adt != NC_F16) return fail(NC_ERR_ARG, "norm: activation dtype %d", adt);
     const dim3 grid(row_cols / d_norm, rows);
     // eight values per thread where the widths and every row's alignment allow
-    const bool vec = d_norm % kSsThreads == 0 && act_vec(adt, a, a_pitch) && act_vec(adt, out, out_pitch) &&
+    const bool vec = norm8_takes(d_norm) && act_vec(adt, a, a_pitch) && act_vec(adt, out, out_pitch) &&
                      act_vec(NC_F16, w, 0) && (kind == kRms || act_vec(NC_F16, bias, 0)) &&
                      (!add || (act_vec(NC_F32, braw, b_pitch * 4) && act_vec(adt, h_out, h_pitch)));
     if (vec) {
+        const bool grid_mean = norm8_grid_mean(adt, d_norm, rows * (row_cols / d_norm));
         auto go = [&](auto kern) {
             hipLaunchKernelGGL(kern, grid, dim3(kSsThreads), 0, st, a, a_pitch, braw, b_pitch, bscale, h_out, h_pitch, w,
-                               bias, out, out_pitch, d_norm, row_cols, post_scale, dpos);
+                               bias, out, out_pitch, d_norm, row_cols, post_scale, dpos, grid_mean);
         };
         auto by_kind = [&](auto t) {
             constexpr int ADT = decltype(t)::value;
@@ -1161,4 +1190,14 @@ extern "C" int nc_expf(const float* x, float* y, int64_t n, void* stream)
     if (!n) return NC_OK;
     hipLaunchKernelGGL(k_expf, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream_of(stream), x, y, n);
     return launch_status("k_expf");
+}
+
+// The kernel that nc_rms_norm (layer 0) or nc_layer_norm takes for aligned rows,
+// and where a layer_norm takes its mean from.
+extern "C" const char* nc_debug_norm_route(int layer, int dtype, int d_norm, int rows)
+{
+    if (!nc::norm8_takes(d_norm)) return "k_norm";
+    if (!layer) return "k_norm8";
+    const int c = nc::norm8_grid_mean(dtype, d_norm, rows) ? d_norm / nc::kSsThreads : 0;
+    return c == 4 || c == 5 || c == 6 || c == 8 || c == 9 ? "k_norm8, grid mean" : "k_norm8, loop mean";
 }

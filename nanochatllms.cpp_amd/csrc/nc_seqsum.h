@@ -609,7 +609,7 @@ NC_HD bool sg_on_grid(float x)
 
 // Sum of x[0..n) in index order, n = C * NT, called by threads 0 .. NT-1
 // (NT a multiple of 64, at most 1024), which synchronize through bar; thread
-// t owns x[t C .. t C + C).  Every calling thread returns the sum; *passes
+// t owns x[t C .. t C + C); x is 16-byte aligned.  Every calling thread returns the sum; *passes
 // (thread 0's view) gets the passes made (0: the plain loop ran).
 template <int C, int NT, class Bar>
 __device__ __forceinline__ float block_seq_sum_grid(const float* x, SgShared& sh, int* passes, Bar& bar)
@@ -707,8 +707,7 @@ __device__ __forceinline__ float block_seq_sum_grid(const float* x, SgShared& sh
     if (!done) {
         // off the grid or too many rounding steps: the plain loop
         if (tid < kWave) {
-            float s = 0.0f;
-            for (int i = 0; i < n; i++) s = s + x[i];
+            const float s = seq_sum(x, n);
             if (tid == 0) sh.result = s;
         }
         bar();

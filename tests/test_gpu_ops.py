@@ -317,9 +317,9 @@ def test_rms_norm(gpu, oracle, dt, d, scale):
 @pytest.mark.parametrize("d,shift", [(256, 0), (1024, 0), (1280, 0), (1536, 0), (2304, 0), (3072, 0), (4096, 0),
                                      (2048, 2), (320, 0)])
 def test_norm_widths(gpu, oracle, dt, kind, d, shift):
-    """Every width the eight-value norm takes (one and two slots per thread,
-    means with and without the exact grid sum), a width it leaves to the other
-    kernel, and gains at an address it does not take (shift bytes)."""
+    """Widths of one and two slots per thread, means from the exact grid sum and
+    from the loop, widths the eight-value norm leaves to the other kernel (256,
+    320), and gains at an address it does not take (shift bytes)."""
     rng = np.random.default_rng(d + shift)
     rows, start = 3, 1
     x = rand_act(oracle, rng, dt, rows, d, 3.0)
@@ -339,6 +339,54 @@ def test_norm_widths(gpu, oracle, dt, kind, d, shift):
                              rows, None)
     gpu.check(st, "norm")
     assert_same(out.ref()[start:], want[start:], f"{kind} norm of {d}")
+
+
+def hard_rows(rng, dt, d):
+    """Rows whose mean rounds at many steps, at few, or at none, and rows whose
+    sums hit the largest values: blocks of unequal scales (Q8) or values of
+    unequal exponents (fp16)."""
+    b = np.repeat(2.0 ** rng.integers(-12, 9, (12, d // 32)), 32, axis=1)
+    x = [rng.standard_normal((12, d)) * b]
+    if dt == F16:
+        x.append(rng.standard_normal((12, d)) * 2.0 ** rng.integers(-14, 8, (12, d)))
+    x.append(np.abs(rng.standard_normal((4, d))))  # the running sum only grows
+    absorb = rng.integers(-3, 4, (4, d)).astype(np.float64)
+    absorb[:, 0] = 1024.0
+    absorb[:, 1:11] = 2.0**-14
+    big = np.where(rng.random((4, d)) < 0.1, 60000.0, 0.0) * np.where(rng.random((4, d)) < 0.5, 1, -1)
+    x += [absorb, big, np.zeros((1, d)), np.full((1, d), 0.5)]
+    return np.concatenate(x).astype(np.float32)
+
+
+@pytest.mark.parametrize("dt,d", [(Q8, 1024), (Q8, 1280), (Q8, 1536), (Q8, 2048), (Q8, 2304), (F16, 2048), (F16, 1280),
+                                  (F16, 2304), (Q8, 2816)])
+def test_layer_norm_hard_rows(gpu, oracle, dt, d):
+    """Every instantiation of the exact grid sum that the eight-value norm uses
+    (Q8 rows are few enough here, fp16 rows of 2048 always, of 1280 one by one),
+    on rows that round often, fall back or have no rounding step, and the loop."""
+    rng = np.random.default_rng(d)
+    v = hard_rows(rng, dt, d)
+    rows = len(v)
+    if dt == F16:
+        x = v.astype(np.float16).view(np.uint16)
+    else:
+        x = np.zeros((rows, OL.row_bytes(Q8, d)), np.uint8)
+        for r in range(rows):
+            oracle.q8_quantize_row(OL.ptr(v[r]), OL.ptr(x[r]), d)
+    w = (1 + 0.2 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
+    b = (0.1 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
+    want = np.zeros_like(x)
+    oracle.layer_norm(OL.ptr(x), dt, OL.ptr(w), OL.ptr(b), OL.ptr(want), d, 0, rows)
+    one = dt == F16 and d == 1280  # a call per row
+    mean = "grid" if d != 2816 and (dt == Q8 or d <= 2048) else "loop"
+    L = gpu.lib()
+    assert L.nc_debug_norm_route(1, dt, d, 1 if one else rows).decode() == f"k_norm8, {mean} mean"
+    dx, out = DevAct(x, dt, rows, d), DevAct.empty(dt, rows, d)
+    dw_, db_ = dev_array(w), dev_array(b)
+    for start, end in [(i, i + 1) for i in range(rows)] if one else [(0, rows)]:
+        gpu.check(L.nc_layer_norm(C.byref(dx.t), C.c_void_p(dw_.ptr), C.c_void_p(db_.ptr), C.byref(out.t), start, end,
+                                  None), "layer_norm")
+    assert_same(out.ref(), want, f"layer norm of {d}")
 
 
 @pytest.mark.parametrize("dt", [Q8, F16])

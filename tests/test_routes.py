@@ -81,3 +81,26 @@ ATTN = [
 @pytest.mark.parametrize("dtype,heads,rows,n_ctx,route", ATTN)
 def test_attention_takes_the_faster_route(nc, dtype, heads, rows, n_ctx, route):
     assert nc.lib().nc_debug_attn_route(dtype, heads, rows, n_ctx).decode() == route
+
+
+NORM = [
+    # (layer, dtype, width, rows, kernel)
+    (0, Q8, 256, 64, "k_norm"),  # 5.5, k_norm8 5.9
+    (1, F16, 256, 1500, "k_norm"),  # 12.7, k_norm8 13.4
+    (0, Q8, 2048, 512, "k_norm8"),
+    (1, F16, 2048, 1500, "k_norm8, grid mean"),  # 29.7, k_norm 93.9
+    (1, Q8, 2304, 64, "k_norm8, grid mean"),  # 8-11, loop 13.5
+    (1, Q8, 2304, 128, "k_norm8, loop mean"),  # 13.6, grid 18-24
+    (1, Q8, 1024, 1500, "k_norm8, grid mean"),  # 15.6, loop 19.4
+    (1, Q8, 1536, 256, "k_norm8, loop mean"),  # 11.7, grid 18-43
+    (1, F16, 2304, 1, "k_norm8, loop mean"),  # 12.3, grid 10-15
+    (1, F16, 2304, 256, "k_norm8, loop mean"),  # 13.5, grid 20.8, k_norm 13.9
+    (1, F16, 1280, 1, "k_norm8, grid mean"),  # 7.2-8.9, loop 9.5
+    (1, F16, 1024, 256, "k_norm8, loop mean"),  # 9.2, grid 12.0, k_norm 10.1
+    (1, F16, 3072, 4, "k_norm8, loop mean"),
+]
+
+
+@pytest.mark.parametrize("layer,dtype,d,rows,route", NORM)
+def test_norms_take_the_faster_sums(nc, layer, dtype, d, rows, route):
+    assert nc.lib().nc_debug_norm_route(layer, dtype, d, rows).decode() == route
