@@ -921,6 +921,16 @@ static int f16_row(const uint8_t* x, const nc_tensor* w, void* out, hipStream_t 
     return launch_status("k_matvec_f16_row");
 }
 
+// Whether two fp16 rows go one after the other through the one-row kernel: its
+// launch of few columns is over long before k_mfma_f16's chain of K steps, which
+// two rows hardly fill (us back to back, k_mfma_f16 / this: 2048 x 2048 14.8 / 6.8,
+// 1280 x 1280 10.0 / 8.4, 2304 x 5760 37.5 / 14.7, 4096 x 1536 12.0 / 11.5; 5632 x 2048
+// 15.3, two of 5.9 and a gap).
+static bool f16_two_rows(int n_rows, const nc_tensor* w)
+{
+    return n_rows == 2 && w->rows <= 4096 && f16_shape_ok(w) && w->cols <= 8192;
+}
+
 // out[r, c] = dot(x[r], w[c]) for x rows [0, n_rows) (pointers already at
 // the first row), fp32 out with `out_pitch` floats per row.
 int matvec_raw(const uint8_t* x, int x_dtype, int x_pitch, int n_rows, const nc_tensor* w, float* out, int out_pitch,
@@ -959,6 +969,10 @@ int matvec_raw(const uint8_t* x, int x_dtype, int x_pitch, int n_rows, const nc_
         if (K % 64) return fail(NC_ERR_ARG, "matmul: F16 path needs K %% 64 == 0, K=%d", K);
         if (!f16_shape_ok(w)) return fail(NC_ERR_ARG, "matmul: K=%d too large", K);
         if (n_rows == 1 && K <= 8192) return f16_row<false>(x, w, out, st, ev_start, ev_stop);
+        if (!ev_start && f16_two_rows(n_rows, w)) {
+            const int s = f16_row<false>(x, w, out, st, nullptr, nullptr);
+            return s ? s : f16_row<false>(x + x_pitch, w, out + out_pitch, st, nullptr, nullptr);
+        }
         return mfma_f16<F32>(x, x_pitch, n_rows, w, out, out_pitch, st, ev_start, ev_stop);
     }
     return fail(NC_ERR_ARG, "matmul: weight dtype %d", w->dtype);
@@ -1170,6 +1184,10 @@ int matmul_2d(const char* name, const nc_tensor* x, const nc_tensor* w, nc_tenso
             return rows < kGemmMinRows ? matvec_qa(xr, x->pitch, rows, w, orow, out->pitch, st)
                                        : gemm_q_act(xr, x->pitch, rows, w, orow, out->pitch, st);
         if (rows == 1 && w->cols <= 8192) return f16_row<true>(xr, w, orow, st, nullptr, nullptr);
+        if (f16_two_rows(rows, w)) {
+            s = f16_row<true>(xr, w, orow, st, nullptr, nullptr);
+            return s ? s : f16_row<true>(xr + x->pitch, w, orow + out->pitch, st, nullptr, nullptr);
+        }
         return mfma_f16<F16>(xr, x->pitch, rows, w, orow, out->pitch, st, nullptr, nullptr);
     }
     if ((s = matvec_raw(xr, x->dtype, x->pitch, rows, w, sp, w->rows, st))) return s;
@@ -1213,7 +1231,9 @@ extern "C" const char* nc_debug_matmul_route(int x_dtype, int w_dtype, int out_d
         if (direct) snprintf(name, sizeof name, "k_matvec_qa %dx%d%s", q.term, q.items, tail);
         else snprintf(name, sizeof name, "k_matvec_q%s", tail);
     } else {
-        snprintf(name, sizeof name, "%s%s", w_dtype == NC_F16 ? "fp16" : gemm_route(pitch, rows, &w, direct), tail);
+        const bool one = (rows == 1 && K <= 8192) || f16_two_rows(rows, &w);
+        snprintf(name, sizeof name, "%s%s",
+                 w_dtype != NC_F16 ? gemm_route(pitch, rows, &w, direct) : one ? "one fp16 row" : "k_mfma_f16", tail);
     }
     return name;
 }

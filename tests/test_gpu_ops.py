@@ -179,6 +179,12 @@ F16_CASES = [
     (128, 8, 7, 0),
     (192, 1300, 300, 0),
     (64, 1000, 1281, 0),
+    # two rows through the one-row kernel, built for the width and not, and
+    # where they go to the matrix cores (columns past 4096, K past 8192)
+    (2048, 100, 3, 1),
+    (1280, 4096, 2, 0),
+    (64, 4097, 2, 0),
+    (8256, 40, 2, 0),
 ]
 
 

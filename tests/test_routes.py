@@ -59,6 +59,21 @@ def test_prefill_products_take_the_faster_shape(nc, wdt, odt, rows, N, K, route)
     assert nc.lib().nc_debug_matmul_route(Q8, wdt, odt, rows, N, K).decode() == route
 
 
+FP16 = [
+    # (out dtype, rows, N, K, route)
+    (F32, 1, 2048, 2048, "one fp16 row"),
+    (F32, 2, 1280, 1280, "one fp16 row"),  # 8.4, k_mfma_f16 10.0
+    (F16, 2, 2304, 5760, "one fp16 row, rows"),  # 14.7, k_mfma_f16 37.5
+    (F32, 2, 5632, 2048, "k_mfma_f16"),
+    (F16, 3, 1280, 1280, "k_mfma_f16, rows"),
+]
+
+
+@pytest.mark.parametrize("odt,rows,N,K,route", FP16)
+def test_two_fp16_rows_take_the_faster_route(nc, odt, rows, N, K, route):
+    assert nc.lib().nc_debug_matmul_route(F16, F16, odt, rows, N, K).decode() == route
+
+
 ATTN = [
     # (dtype, heads, rows, n_ctx, kernel)
     (F16, 32, 16, 128, "k_attn_rows"),  # 10.0, k_attn_f16 12.9
