@@ -175,6 +175,9 @@ const char* nc_debug_attn_route(int dtype, int n_heads, int rows, int n_ctx);
 /* Test hook, on the host: the kernel of nc_rms_norm (layer 0) or
  * nc_layer_norm for rows of d_norm values. */
 const char* nc_debug_norm_route(int layer, int dtype, int d_norm, int rows);
+/* Test hook, on the host: the kernel of nc_silu (silu 1) or of nc_multiply,
+ * nc_add, nc_scale and nc_bias_add (0). */
+const char* nc_debug_ew_route(int silu, int dtype, int rows, int cols);
 /* Greedy pick of greedy_sample (src/gten/sampler.cpp:33-41): first index of
  * the maximum. */
 int nc_argmax(const float* x, int n, int32_t* out, void* stream);

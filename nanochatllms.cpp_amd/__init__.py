@@ -156,7 +156,8 @@ def lib():
         "nc_bias_add": (I, [TP, VP, I, I, VP]), "nc_qkv_attn": (I, [TP, TP, TP, TP, I, I, I, I, I, VP]),
         "nc_argmax": (I, [VP, I, VP, VP]), "nc_expf": (I, [VP, VP, C.c_int64, VP]),
         "nc_expf_host": (F, [F]), "nc_debug_spec": (I, [F, VP]),
-        "nc_debug_attn_route": (C.c_char_p, [I] * 4), "nc_debug_norm_route": (C.c_char_p, [I] * 4), "nc_debug_matmul_route": (C.c_char_p, [I] * 6),
+        "nc_debug_attn_route": (C.c_char_p, [I] * 4), "nc_debug_norm_route": (C.c_char_p, [I] * 4),
+        "nc_debug_ew_route": (C.c_char_p, [I] * 4), "nc_debug_matmul_route": (C.c_char_p, [I] * 6),
         "nc_block_seq_sum_grid": (I, [VP, I, I, VP, VP, VP]),
         "nc_seq_sum_grid_host": (F, [VP, I, I, C.POINTER(I)]),
         "nc_model_create": (I, [C.POINTER(ModelConfig), C.POINTER(VP)]), "nc_model_free": (I, [VP]),

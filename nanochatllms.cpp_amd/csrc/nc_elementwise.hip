@@ -666,10 +666,15 @@ static unsigned grid8(int rows, int cols) { return (unsigned)(((int64_t)rows * (
 static bool fits8(int rows, int cols) { return (int64_t)rows * cols < ((int64_t)1 << 31); }
 // Values from which eight per thread win (us, one value per thread against
 // eight, Q8 rows): add 90K values 2.4 / 2.3, 360K 2.7 / 2.4, 1.2M 4.3 / 3.2, 3.1M
-// 8.1 / 4.3; rotary embedding 2.5 / 3.0, 3.6 / 3.1, 7.0 / 4.4, 13.7 / 6.2; with
-// an exponential (eight in turn per thread) 360K 3.0 / 3.8, 1.2M 5.0 / 5.0, 3.1M
-// 9.1 / 7.4.
-constexpr int kEw8Min = 1 << 18, kSilu8Min = 1 << 20;
+// 8.1 / 4.3; rotary embedding 2.5 / 3.0, 3.6 / 3.1, 7.0 / 4.4, 13.7 / 6.2.  With an
+// exponential (eight in turn per thread) later, and the later the less the
+// rows' format costs beside it: silu of Q8 rows 430K 3.5 / 3.6, 1.05M 5.1 / 5.1,
+// 1.4M 6.2 / 5.4; of fp16 rows 1.05M 4.0 / 4.6, 2.3M 6.2 / 6.4, 2.9M 7.1 / 7.0; of fp32
+// rows 1.05M 4.4 / 5.0, 2.9M 8.2 / 8.7, 3.5M 10.4 / 10.0.  SwiGLU, which also reads
+// two fp32 rows: fp16 1.07M 5.0 / 5.2, 1.24M 5.1 / 5.2, 1.4M 5.6 / 5.4.
+constexpr int kEw8Min = 1 << 18;
+static int silu8_min(int dtype) { return dtype == NC_Q8 ? 1 << 20 : dtype == NC_F16 ? 5 << 19 : 3 << 20; }
+static int silu_mul8_min(int dtype) { return dtype == NC_Q8 ? 1 << 20 : 5 << 18; }
 
 // The widths of k_norm8: at 256 values only a lane quad's worth of threads load,
 // and k_norm's 256 of one value each are 0.2 to 0.8 us faster.
@@ -792,7 +797,7 @@ int silu_mul_launch(int adt, const float* raw, int raw_pitch, int f, uint8_t* ou
                     hipStream_t st)
 {
     if (rows <= 0) return NC_OK;
-    if ((adt == NC_Q8 || adt == NC_F16) && rows8(adt, f) && fits8(rows, f) && (int64_t)rows * f >= kSilu8Min &&
+    if ((adt == NC_Q8 || adt == NC_F16) && rows8(adt, f) && fits8(rows, f) && (int64_t)rows * f >= silu_mul8_min(adt) &&
         act_vec(NC_F32, raw, raw_pitch * 4) &&
         act_vec(adt, out, out_pitch)) {
         const dim3 g8(grid8(rows, f));
@@ -843,12 +848,17 @@ int argmax_advance_launch(const float* x, int n, int32_t* tokens, int* dpos, uns
     return launch_status("k_argmax_advance");
 }
 
+static bool ew8_takes(int op, int dtype, int rows, int cols)
+{
+    return rows8(dtype, cols) && fits8(rows, cols) &&
+           (int64_t)rows * cols >= (op == kSilu ? silu8_min(dtype) : kEw8Min);
+}
+
 int ew_launch(int op, int adt, const uint8_t* a, int a_pitch, const uint8_t* b, int b_pitch, const uint16_t* bias,
               float s, uint8_t* out, int out_pitch, int cols, int rows, hipStream_t st)
 {
     if (rows <= 0) return NC_OK;
-    if (rows8(adt, cols) && fits8(rows, cols) && (int64_t)rows * cols >= (op == kSilu ? kSilu8Min : kEw8Min) && act_vec(adt, a, a_pitch) &&
-        act_vec(adt, out, out_pitch) && (!b || act_vec(adt, b, b_pitch)) && (!bias || act_vec(NC_F16, bias, 0))) {
+    if (ew8_takes(op, adt, rows, cols) && act_vec(adt, a, a_pitch) && act_vec(adt, out, out_pitch) && (!b || act_vec(adt, b, b_pitch)) && (!bias || act_vec(NC_F16, bias, 0))) {
         const dim3 g8(grid8(rows, cols));
 #define EW8_CALL(OPV) hipLaunchKernelGGL((k_ew8<ADT, OPV>), g8, dim3(256), 0, st, a, a_pitch, b, b_pitch, bias, s, out, out_pitch, cols, rows)
         NC_ADT_DISPATCH(adt, {
@@ -1200,4 +1210,11 @@ extern "C" const char* nc_debug_norm_route(int layer, int dtype, int d_norm, int
     if (!layer) return "k_norm8";
     const int c = nc::norm8_grid_mean(dtype, d_norm, rows) ? d_norm / nc::kSsThreads : 0;
     return c == 4 || c == 5 || c == 6 || c == 8 || c == 9 ? "k_norm8, grid mean" : "k_norm8, loop mean";
+}
+
+// The kernel that an elementwise operator (silu: nc_silu; else nc_multiply,
+// nc_add, nc_scale, nc_bias_add) takes for aligned rows.
+extern "C" const char* nc_debug_ew_route(int silu, int dtype, int rows, int cols)
+{
+    return nc::ew8_takes(silu ? nc::kSilu : nc::kAdd, dtype, rows, cols) ? "k_ew8" : "k_ew";
 }

@@ -421,6 +421,56 @@ def test_elementwise_many_rows(gpu, oracle, dt, op, d, rows):
     assert_same(out.ref(), want, op)
 
 
+EIGHT_ROWS = {"silu": {Q8: 515, F16: 1283, F32: 1541}}  # past each type's line at 2048 columns
+
+
+@pytest.mark.parametrize("dt", [Q8, F16, F32])
+@pytest.mark.parametrize("op", ["silu", "mul", "add", "scale", "bias"])
+def test_eight_value_operators_in_place(gpu, oracle, dt, op):
+    """Every operator of eight values per thread with the output over its input,
+    rows from a position on, a last workgroup that is not full."""
+    d, start = 2048, 2
+    n = start + EIGHT_ROWS.get(op, {}).get(dt, 131)
+    assert gpu.lib().nc_debug_ew_route(op == "silu", dt, n - start, d).decode() == "k_ew8"
+    rng = np.random.default_rng(n + dt)
+    a, b = rand_act(oracle, rng, dt, n, d, 4.0), rand_act(oracle, rng, dt, n, d, 1.0)
+    bias = (0.1 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
+    want, scale = a.copy(), 0.3
+    da, db_, dbias = DevAct(a, dt, n, d), DevAct(b, dt, n, d), dev_array(bias)
+    L, A = gpu.lib(), C.byref(da.t)
+    if op == "silu":
+        oracle.silu(OL.ptr(want), OL.ptr(want), dt, d, start, n)
+        st = L.nc_silu(A, A, start, n, None)
+    elif op == "scale":
+        oracle.scale(OL.ptr(want), dt, scale, d, start, n)
+        st = L.nc_scale(A, scale, start, n, None)
+    elif op == "bias":
+        oracle.bias_add(OL.ptr(want), dt, OL.ptr(bias), d, start, n)
+        st = L.nc_bias_add(A, C.c_void_p(dbias.ptr), start, n, None)
+    else:
+        (oracle.multiply if op == "mul" else oracle.add)(OL.ptr(want), OL.ptr(b), OL.ptr(want), dt, d, start, n)
+        st = (L.nc_multiply if op == "mul" else L.nc_add)(A, C.byref(db_.t), A, start, n, None)
+    gpu.check(st, op)
+    assert_same(da.ref(), want, op)
+
+
+@pytest.mark.parametrize("dt", [Q8, F16])
+def test_rope_many_rows_from_a_position(gpu, oracle, dt):
+    """The eight-value rotary embedding of whole heads (every lane rotated), its
+    table from a later position on."""
+    d, start, n = 2304, 7, 150
+    rng = np.random.default_rng(dt)
+    a = rand_act(oracle, rng, dt, n, d, 2.0)
+    tab = np.zeros((n, 32, 2), np.float32)
+    gpu.check(gpu.lib().nc_rope_table(n, 64, 1.0, ptr(tab)), "rope_table")
+    dtab, da, out = dev_array(tab), DevAct(a, dt, n, d), DevAct.empty(dt, n, d)
+    want = a.copy()
+    oracle.rotary_emb(OL.ptr(a), OL.ptr(want), dt, d, 64, 1.0, start, n)
+    gpu.check(gpu.lib().nc_rotary_emb(C.byref(da.t), C.byref(out.t), 64, 1.0, C.c_void_p(dtab.ptr), start, n, None),
+              "rope")
+    assert_same(out.ref()[start:], want[start:], "rope")
+
+
 @pytest.mark.parametrize("dt", [Q8, F16])
 def test_rms_norm_per_head(gpu, oracle, dt):
     rng = np.random.default_rng(5)

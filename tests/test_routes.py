@@ -119,3 +119,21 @@ NORM = [
 @pytest.mark.parametrize("layer,dtype,d,rows,route", NORM)
 def test_norms_take_the_faster_sums(nc, layer, dtype, d, rows, route):
     assert nc.lib().nc_debug_norm_route(layer, dtype, d, rows).decode() == route
+
+
+EW = [
+    # (silu, dtype, rows, cols, kernel)
+    (1, Q8, 256, 5632, "k_ew8"),  # 5.4, k_ew 6.2
+    (1, F16, 187, 5632, "k_ew"),  # 4.0, k_ew8 4.6
+    (1, F16, 400, 2304, "k_ew"),  # 3.9, k_ew8 4.7
+    (1, F16, 512, 5632, "k_ew8"),  # 7.0, k_ew 7.1
+    (1, F32, 512, 5632, "k_ew"),  # 8.2, k_ew8 8.7
+    (1, F32, 1500, 5632, "k_ew8"),  # 18.1, k_ew 20.6
+    (0, F32, 400, 2304, "k_ew8"),  # 3.4, k_ew 3.7
+    (0, Q8, 16, 2048, "k_ew"),
+]
+
+
+@pytest.mark.parametrize("silu,dtype,rows,cols,route", EW)
+def test_elementwise_operators_take_the_faster_kernel(nc, silu, dtype, rows, cols, route):
+    assert nc.lib().nc_debug_ew_route(silu, dtype, rows, cols).decode() == route
