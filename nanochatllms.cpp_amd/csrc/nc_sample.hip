@@ -222,6 +222,19 @@ static int sample_grid(int n)
     return g < 1 ? 1 : (g > kSmMaxWg ? kSmMaxWg : g);
 }
 
+// The sampled logits per thread for which the wavefront's largest of them has
+// about the threshold's rank (see k_sample_topk), whether it offers that, and how
+// many of the `loaded` are used.
+__device__ __forceinline__ float sample_large(int k, int n)
+{
+    return 0.69f * (float)n / (kWave * (float)min(3 * k / 2 + 256, n));
+}
+__device__ __forceinline__ bool sample_few(int k, int n) { return k < kWave && sample_large(k, n) >= 0.8f; }
+__device__ __forceinline__ int sample_per(int k, int n, int loaded)
+{
+    return sample_few(k, n) ? min(max((int)sample_large(k, n), 1), loaded) : loaded;
+}
+
 __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
 {
     // cand: candidate (key << 32 | index); later the fallback's logit stage,
@@ -264,7 +277,10 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
     // the threshold sample and the slice requested together
     const bool sampled = n > kSmCap;
     float sx[kSmPer] = {};
-    const int loaded = n > kSmOneMax ? kSmPer : 1;
+    // (a k of the launch's own arguments that uses one logit per thread
+    // requests one: 50304 logits, k = 50, 18.9 -> 18.3 us; a device-held k would
+    // have to arrive first)
+    const int loaded = n <= kSmOneMax ? 1 : A.dset ? kSmPer : sample_per(A.k, n, kSmPer);
     if (sampled) {
         sx[0] = A.logits[(long long)(kSmPer * tid) * n / kSmSample];
         if (loaded > 1) {
@@ -295,20 +311,22 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
     // k < 64, where far more than k are kept anyway, the offer is the largest
     // (no sort: 32000 logits, k = 50, 17 us against 19) of as few logits per
     // thread as keep T (0.8 T at least): fewer candidates in large
-    // vocabularies, 151936 logits, k = 50, 24 -> 20 us.
+    // vocabularies (k = 50, median of 8 draws: 100352 logits 21.2 -> 20.0 us, 151936
+    // 24.7 -> 20.6).
     // One sampled logit per thread leaves at least 3 above the wanted one for
     // the largest k up to kSmOneMax logits; four cost 0.5 us there.  Beyond,
-    // one leaves 0.7 to 3, too few: 3 of 12 draws of k = 850 of 100352 logits
-    // and 4 of 12 of k = 1000 of 122753 kept fewer than k or more than kSmCap
-    // and ran the serial fallback, 10 to 12.6 ms; with four none of 24 draws
-    // of any k from 2 to 1000 of up to 151936 logits did.
+    // one leaves 0.7 to 3, too few for a large k: 3 of 12 draws of k = 850 of
+    // 100352 logits and 4 of 12 of k = 1000 of 122753 kept fewer than k or more than
+    // kSmCap and ran the serial fallback, 10 to 12.6 ms; with four none of 24 draws
+    // of any k from 2 to 1000 of up to 151936 logits did.  That bound on the worst
+    // draw costs the median one up to 4 us where one logit would have done (50304
+    // logits: k = 100 38.8 -> 42.5 us, 300 50.9 -> 54.8).
     uint32_t thr = 0;
     if (sampled) {
         const int T = min(3 * k / 2 + 256, n);
         const float f = (float)T / (float)n;
-        const float large = 0.69f / (kWave * f);  // threads' logits for which lam = 0.69
-        const bool few = k < kWave && large >= 0.8f;
-        const int per = few ? min(max((int)large, 1), loaded) : loaded;
+        const bool few = sample_few(k, n);
+        const int per = sample_per(k, n, loaded);
         uint32_t sk = fkey(sx[0]);
         float none = 1.0f - f;
 #pragma unroll
@@ -320,7 +338,7 @@ __global__ __launch_bounds__(kSmThreads) void k_sample_topk(SampleArgs A)
         }
         const float lam = (float)kWave * (1.0f - none);
         const float want = lam * fmaxf(0.8f, fminf(1.0f, 4.0f * (float)k / (float)T));
-        const int rw = few         ? 0
+        const int rw = few          ? 0
                        : loaded > 1 ? min(max((int)ceilf(want - 0.69f), 0), kWave - 1)
                                     : min((int)((float)kWave * f), kWave - 1);
         if (rw == 0) {
