@@ -3,11 +3,13 @@
 The reference's Q4 block dot product (gten/ops.cpp:387-490) multiplies each
 activation code x by the decoded weight n - 7 (n the stored nibble) and sums
 eight such products per AVX lane.  The prefill matmul (k_gemm_qw) hands
-the fp16 matrix cores the raw weight 1024 + n instead (fp16 bits 0x6400 | n,
-one v_perm_b32 per two codes) and starts each product sum from
--1031 x (sum of the lane's activation codes).  That equals the reference's
-integer lane sum exactly when every value the matrix core can form on the way
-is an integer below 2^24 (exact in fp32 whatever the order of the adds).
+the fp16 matrix cores the raw weight 1024 + n instead for the low nibbles (fp16
+bits 0x6400 | n, one v_perm_b32 per two codes) and adds -1031 x (the sum of the
+activation codes they meet) to the product sum's start; the high nibbles, in
+place as 1024 + 16 n against sixteenths of the codes, add -71 of theirs (the whole
+start: test_gemm_codes).  That equals the reference's integer lane sum exactly
+when every value the matrix core can form on the way is an integer below 2^24
+(exact in fp32 whatever the order of the adds).
 These tests check that bound and the identity on random and extreme codes,
 in several summation orders, and that a wrong offset is caught.
 """

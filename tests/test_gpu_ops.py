@@ -58,10 +58,9 @@ MATMUL_CASES = [
     (Q8, Q8, 8192, 2048, 1, 0),
     (Q8, Q8, 64, 40, 5, 2),
     (Q8, Q4, 1024, 96, 9, 0),
-    # prompt-row shapes: every launch shape of the prefill matmul's table
-    # (fp16 matrix cores: 8- and 4-block chunks, short / medium / long
-    # prompts, tall weights, columns past a 16-multiple; the integer kernel
-    # for long prompts of tall weights and for rows of K % 128 != 0)
+    # prompt rows: short, medium and long prompts, tall weights, columns past a
+    # 16-multiple on the fp16 matrix cores, and rows of K % 128 != 0 on the
+    # integer ones (their shapes by name: WIDE_ROUTES, INTEGER_CASES)
     (Q8, Q4, 2048, 2560, 64, 0),
     (Q8, Q4, 2048, 2048, 40, 3),
     (Q8, Q4, 5632, 2048, 16, 0),
@@ -167,6 +166,46 @@ WIDE_ROUTES = [
 def test_matmul_wide_routes(gpu, oracle, wdt, K, N, rows, odt, route):
     assert gpu.lib().nc_debug_matmul_route(Q8, wdt, odt, rows, N, K).decode() == route
     test_matmul_wide(gpu, oracle, wdt, K, N, rows, 0, odt)
+
+
+INTEGER_CASES = [
+    # (K, N, rows): the integer matrix-core kernel's three shapes (K no multiple
+    # of 128): 256 rows and more of 8192 columns and more; 256 rows of fewer, and
+    # 32 rows of tall weights; the rest.  One, an odd and an even number of
+    # chunks of four blocks, the last one partial
+    (96, 8200, 260),
+    (160, 8192, 257),
+    (160, 300, 259),
+    (96, 8193, 33),
+    (288, 8192, 250),
+    (2080, 70, 30),
+    (224, 8300, 9),
+]
+
+
+@pytest.mark.parametrize("wdt", [Q4, Q8])
+@pytest.mark.parametrize("K,N,rows", INTEGER_CASES)
+def test_matmul_integer_shapes(gpu, oracle, wdt, K, N, rows):
+    assert gpu.lib().nc_debug_matmul_route(Q8, wdt, F32, rows, N, K).decode() == "k_gemm_q"
+    test_matmul_wide(gpu, oracle, wdt, K, N, rows, 0, F32)
+
+
+@pytest.mark.parametrize("wdt", [Q4, Q8])
+def test_matmul_deltas_off_a_dword(gpu, oracle, wdt):
+    """Weight deltas two bytes off a dword: the kernels that load whole dwords do
+    not take them."""
+    K, N, rows = 256, 300, 40
+    rng = np.random.default_rng(wdt)
+    x, w = rand_act(oracle, rng, Q8, rows, K), rand_weight(oracle, rng, wdt, N, K)
+    want = np.zeros((rows, N), np.float32)
+    oracle.matmul(OL.ptr(x), Q8, OL.ptr(w), wdt, OL.ptr(want), F32, K, N, 0, rows, None)
+    dx, dw, out = DevAct(x, Q8, rows, K), DevWeight(w, wdt, N, K), DevAct.empty(F32, rows, N)
+    deltas = np.zeros(N * K // 32, np.uint16)
+    dw.dbuf.download(deltas)
+    moved = dev_array(np.concatenate([np.zeros(1, np.uint16), deltas, np.zeros(1, np.uint16)]))
+    dw.t.deltas = moved.ptr + 2
+    gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), 0, rows, None), "matmul")
+    assert_same(out.ref().view(np.float32), want, "matmul, deltas off a dword")
 
 
 F16_CASES = [
@@ -469,6 +508,93 @@ def test_rope_many_rows_from_a_position(gpu, oracle, dt):
     gpu.check(gpu.lib().nc_rotary_emb(C.byref(da.t), C.byref(out.t), 64, 1.0, C.c_void_p(dtab.ptr), start, n, None),
               "rope")
     assert_same(out.ref()[start:], want[start:], "rope")
+
+
+def assert_same_f16(got, want, what):
+    """Equal bits, any NaN for a NaN."""
+    g = np.ascontiguousarray(got).view(np.uint8).reshape(-1).view(np.float16)
+    w = np.ascontiguousarray(want).view(np.uint8).reshape(-1).view(np.float16)
+    nan = np.isnan(w)
+    assert np.array_equal(np.isnan(g), nan), f"{what}: NaN at other places"
+    assert nan.any() and not nan.all(), what
+    assert_same(g[~nan], w[~nan], what)
+
+
+def with_specials(rng, a, share=0.002):
+    a = a.copy().view(np.float16)
+    at = rng.random(a.shape) < share
+    a[at] = rng.choice(np.array([np.inf, -np.inf, np.nan, 65504.0, -65504.0], np.float16), int(at.sum()))
+    return a.view(np.uint16)
+
+
+@pytest.mark.parametrize("K,N,rows", [(192, 130, 18), (128, 70, 5)])
+def test_matmul_f16_non_finite(gpu, oracle, K, N, rows):
+    """Infinities and NaN of one row or column reach no other one on the matrix
+    cores."""
+    rng = np.random.default_rng(K)
+    x, w = rand_act(oracle, rng, F16, rows, K), rand_weight(oracle, rng, F16, N, K)
+    x[rows // 2 :] = with_specials(rng, x[rows // 2 :], 0.01)
+    w[: N // 2] = with_specials(rng, w[: N // 2], 0.002)
+    want = np.zeros((rows, OL.row_bytes(F16, N)), np.uint8)
+    oracle.matmul(OL.ptr(x), F16, OL.ptr(w), F16, OL.ptr(want), F16, K, N, 0, rows, None)
+    assert gpu.lib().nc_debug_matmul_route(F16, F16, F16, rows, N, K).decode() == "k_mfma_f16, rows"
+    dx, dw, out = DevAct(x, F16, rows, K), DevWeight(w, F16, N, K), DevAct.empty(F16, rows, N)
+    gpu.check(gpu.lib().nc_matmul_2d(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), 0, rows, None), "matmul")
+    assert_same_f16(out.ref(), want, "matmul of non-finite values")
+
+
+@pytest.mark.parametrize("where", ["k", "v"])
+def test_qkv_attn_f16_non_finite_later_rows(gpu, oracle, where):
+    """Infinities and NaN in K or V rows reach only the query rows that attend
+    them, also within one tile of sixteen: rows before them are those of finite
+    values, the last row is the oracle's."""
+    hq, hkv, n, start, first = 3, 1, 660, 625, 641
+    rng = np.random.default_rng(ord(where))
+    q, k, v = (rand_act(oracle, rng, F16, n, h * 64) for h in (hq, hkv, hkv))
+
+    def attn(k, v):
+        want = np.zeros((n, OL.row_bytes(F16, hq * 64)), np.uint8)
+        oracle.qkv_attn(OL.ptr(q), OL.ptr(k), OL.ptr(v), OL.ptr(want), F16, hq, hkv, 64, start, n)
+        return want
+
+    finite = attn(k, v)
+    if where == "k":
+        k[first:] = with_specials(rng, k[first:], 0.05)
+    else:
+        v[first:] = with_specials(rng, v[first:], 0.05)
+    want = attn(k, v)
+    assert gpu.lib().nc_debug_attn_route(F16, hq, n - start, n).decode() == "k_attn_f16"
+    dq, dk, dv = DevAct(q, F16, n, hq * 64), DevAct(k, F16, n, hkv * 64), DevAct(v, F16, n, hkv * 64)
+    out = DevAct.empty(F16, n, hq * 64)
+    gpu.check(gpu.lib().nc_qkv_attn(C.byref(dq.t), C.byref(dk.t), C.byref(dv.t), C.byref(out.t), hq, hkv, 64, start,
+                                    n, None), "qkv_attn")
+    got = out.ref()
+    assert_same(got[start:first], finite[start:first], "rows before the non-finite ones")
+    last, ref = (a[n - 1].view(np.float16) for a in (got, want))
+    assert np.isnan(ref).any() and np.array_equal(np.isnan(last), np.isnan(ref))
+    assert_same(last[~np.isnan(ref)], ref[~np.isnan(ref)], "the last row")
+
+
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+@pytest.mark.parametrize("d", [2048, 2304])
+def test_norm_non_finite(gpu, oracle, kind, d):
+    rng = np.random.default_rng(d)
+    rows = 9
+    x = rand_act(oracle, rng, F16, rows, d)
+    x[1::2] = with_specials(rng, x[1::2], 0.001)
+    w = (1 + 0.2 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
+    b = (0.1 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
+    want = np.zeros_like(x)
+    dx, out, dw_, db_ = DevAct(x, F16, rows, d), DevAct.empty(F16, rows, d), dev_array(w), dev_array(b)
+    L = gpu.lib()
+    if kind == "rms":
+        oracle.rms_norm(OL.ptr(x), F16, OL.ptr(w), OL.ptr(want), d, 0, rows)
+        st = L.nc_rms_norm(C.byref(dx.t), C.c_void_p(dw_.ptr), C.byref(out.t), d, 0, rows, None)
+    else:
+        oracle.layer_norm(OL.ptr(x), F16, OL.ptr(w), OL.ptr(b), OL.ptr(want), d, 0, rows)
+        st = L.nc_layer_norm(C.byref(dx.t), C.c_void_p(dw_.ptr), C.c_void_p(db_.ptr), C.byref(out.t), 0, rows, None)
+    gpu.check(st, "norm")
+    assert_same_f16(out.ref(), want, f"{kind} norm of non-finite values")
 
 
 @pytest.mark.parametrize("dt", [Q8, F16])

@@ -1,9 +1,11 @@
 """nc_matmul_2d_noalloc (the allocation-free matmul_2d) against nc_matmul_2d.
 
-Two calls in a row through the C-ABI, the second with a smaller input (the
-staging array keeps the first call's contents), for Q8 and fp16 activation
-outputs: every output byte must equal the allocating entry point's and the
-oracle's.  A call whose staging would not fit the array is refused.
+Two calls in a row through the C-ABI, the second with a smaller input, for Q8
+and fp16 activation outputs: every output byte must equal the allocating entry
+point's and the oracle's.  The staged pairs go through the staging array in both
+calls, so the second finds the first one's contents there; the others' launches
+store their rows themselves.  A call whose staging would not fit the array is
+refused.
 """
 import ctypes as C
 
@@ -39,7 +41,7 @@ def rand_weight(oracle, rng, dtype, rows, cols):
 
 
 # (activation dtype, weight dtype, K, N, rows, start): each pair's second
-# call is smaller than its first
+# call is smaller than its first; one or both of these store rows directly
 CALLS = {
     "q8": [(Q8, Q4, 2048, 5632, 64, 0), (Q8, Q4, 2048, 2048, 3, 1)],
     "f16": [(F16, F16, 2048, 2048, 24, 0), (F16, F16, 256, 1000, 1, 0)],
@@ -65,6 +67,39 @@ def test_matmul_noalloc_matches_matmul(gpu, oracle, kind):
         got_a, got_b = a.ref()[start:], b.ref()[start:]
         assert np.array_equal(got_b, got_a), f"{kind} K={K} N={N}: noalloc differs from matmul_2d"
         assert np.array_equal(got_b, want[start:]), f"{kind} K={K} N={N}: noalloc differs from the oracle"
+
+
+# pairs staged in both calls: products whose launch does not store Q8 rows, and
+# fp16 products with the output over the input (K = N), which must be read whole
+STAGED = {
+    "q8": [(Q8, Q4, 2048, 2048, 64, 0), (Q8, Q4, 2048, 1000, 9, 1)],
+    "q8 few rows": [(Q8, Q8, 4096, 2048, 7, 0), (Q8, Q8, 4096, 300, 3, 1)],
+    "f16 in place": [(F16, F16, 1024, 1024, 24, 0), (F16, F16, 192, 192, 5, 1)],
+}
+
+
+@pytest.mark.parametrize("kind", list(STAGED))
+def test_matmul_noalloc_staged_twice(gpu, oracle, kind):
+    L = gpu.lib()
+    fn = L.nc_matmul_2d_noalloc
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p] * 3 + [C.c_int, C.c_int, C.c_void_p]
+    rng = np.random.default_rng(len(kind))
+    for adt, wdt, K, N, rows, start in STAGED[kind]:
+        x = rand_act(oracle, rng, adt, rows, K)
+        w = rand_weight(oracle, rng, wdt, N, K)
+        dw, got = DevWeight(w, wdt, N, K), []
+        if adt == Q8:
+            assert L.nc_debug_matmul_route(adt, wdt, adt, rows - start, N, K).endswith(b" + k_write_rows")
+        for f in (L.nc_matmul_2d, fn):
+            dx = DevAct(x, adt, rows, K)
+            out = dx if adt == F16 else DevAct.empty(adt, rows, N)
+            gpu.check(f(C.byref(dx.t), C.byref(dw.t), C.byref(out.t), start, rows, None), "matmul_2d")
+            sync()
+            got.append(out.ref()[start:])
+        want = np.zeros((rows, OL.row_bytes(adt, N)), np.uint8)
+        oracle.matmul(OL.ptr(x), adt, OL.ptr(w), wdt, OL.ptr(want), adt, K, N, start, rows, None)
+        assert np.array_equal(got[1], got[0]), f"{kind} K={K} N={N}: noalloc differs from matmul_2d"
+        assert np.array_equal(got[1], want[start:]), f"{kind} K={K} N={N}: noalloc differs from the oracle"
 
 
 def test_matmul_noalloc_refuses_oversize(gpu, oracle):
