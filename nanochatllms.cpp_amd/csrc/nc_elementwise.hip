@@ -681,17 +681,19 @@ static int silu_mul8_min(int dtype) { return dtype == NC_Q8 ? 1 << 20 : 5 << 18;
 static bool norm8_takes(int d_norm) { return d_norm % kSsThreads == 0 && d_norm > kSsThreads; }
 
 // Whether k_norm8 takes a layer_norm's mean as the exact grid sum rather than
-// the loop: a pass per step that rounds, so a launch is as slow as its row with
-// the most of them (up to 48 passes and then the loop).  Rows of 2048 always do
-// (their loop's 6 us; k_norm's did as well).  Q8 rows, multiples of a few deltas'
-// grids, round rarely, so they do while they are few: 64 rows of 2304 8-11 us
-// against 13.5, 128 rows 18-24 against 13.6; 64 of 1536 8.6 / 11.4, 256 18-43 / 11.7;
-// of 1024 any number (1500 rows 15.6 / 19.4).
-// fp16 rows round often: one row of 1024 or 1280 7.2-8.9 / 8.4-9.5, 4 rows 9.3-10.2 /
-// 8.4-9.5, one of 2304 10.3-14.9 / 12.3.
+// the loop.  The grid takes a pass per step that rounds and after 48 of them the
+// loop, so a launch is as slow as its row with the most.  Q8 rows, multiples of
+// a few deltas' grids, round rarely, but one of some hundred or thousand, the
+// more the wider (of 1024 values none seen), does all the way.  Means over ten
+// draws, grid / loop, us: 2304 values, 4 rows 8.2 / 13.4, 64 rows 18 / 14.9; 2048, 64
+// rows 10.8 / 12.6, 128 16.1 / 13.6; 1536, 64 rows 8.5 / 11.6, 256 15.9 / 11.7; 1280, 64
+// rows 8.0 / 10.4; 1024, 1500 rows 16 / 19.  fp16 rows round often: one row of 2048
+// 10.6 / 12, 16 rows 15.3 / 11.6; one of 1280 8.8 / 9.6, 4 rows 9.8 / 9.6.
 static bool norm8_grid_mean(int adt, int d_norm, int segments)
 {
-    return d_norm == 2048 || (adt == NC_Q8 && d_norm == 1024) || (int64_t)segments * d_norm <= (adt == NC_Q8 ? 150000 : 1280);
+    const int64_t values = (int64_t)segments * d_norm;
+    if (adt != NC_Q8) return values <= 2048;
+    return d_norm == 1024 || values <= (d_norm <= 2048 ? 131072 : 10000);
 }
 
 // Threads per norm workgroup: the largest multiple of 64 up to 1024 that

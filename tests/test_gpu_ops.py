@@ -403,12 +403,13 @@ def hard_rows(rng, dt, d):
     return np.concatenate(x).astype(np.float32)
 
 
-@pytest.mark.parametrize("dt,d", [(Q8, 1024), (Q8, 1280), (Q8, 1536), (Q8, 2048), (Q8, 2304), (F16, 2048), (F16, 1280),
-                                  (F16, 2304), (Q8, 2816)])
-def test_layer_norm_hard_rows(gpu, oracle, dt, d):
-    """Every instantiation of the exact grid sum that the eight-value norm uses
-    (Q8 rows are few enough here, fp16 rows of 2048 always, of 1280 one by one),
-    on rows that round often, fall back or have no rounding step, and the loop."""
+@pytest.mark.parametrize("dt,d,each", [(Q8, 1024, 0), (Q8, 1280, 0), (Q8, 1536, 0), (Q8, 2048, 0), (Q8, 2304, 4),
+                                       (F16, 2048, 1), (F16, 1280, 1), (F16, 2048, 0), (Q8, 2304, 0), (F16, 2304, 0),
+                                       (Q8, 2816, 0)])
+def test_layer_norm_hard_rows(gpu, oracle, dt, d, each):
+    """Rows that round often, fall back or have no rounding step, in one call or
+    `each` rows per call: few enough for every instantiation of the exact grid
+    sum that the eight-value norm uses, and many, for the loop."""
     rng = np.random.default_rng(d)
     v = hard_rows(rng, dt, d)
     rows = len(v)
@@ -422,13 +423,14 @@ def test_layer_norm_hard_rows(gpu, oracle, dt, d):
     b = (0.1 * rng.standard_normal(d)).astype(np.float16).view(np.uint16)
     want = np.zeros_like(x)
     oracle.layer_norm(OL.ptr(x), dt, OL.ptr(w), OL.ptr(b), OL.ptr(want), d, 0, rows)
-    one = dt == F16 and d == 1280  # a call per row
-    mean = "grid" if d != 2816 and (dt == Q8 or d <= 2048) else "loop"
+    grid = each or (dt == Q8 and d <= 2048)
     L = gpu.lib()
-    assert L.nc_debug_norm_route(1, dt, d, 1 if one else rows).decode() == f"k_norm8, {mean} mean"
+    route = L.nc_debug_norm_route(1, dt, d, each or rows).decode()
+    assert route == ("k_norm8, grid mean" if grid else "k_norm8, loop mean")
     dx, out = DevAct(x, dt, rows, d), DevAct.empty(dt, rows, d)
     dw_, db_ = dev_array(w), dev_array(b)
-    for start, end in [(i, i + 1) for i in range(rows)] if one else [(0, rows)]:
+    for start in range(0, rows, each or rows):
+        end = min(rows, start + (each or rows))
         gpu.check(L.nc_layer_norm(C.byref(dx.t), C.c_void_p(dw_.ptr), C.c_void_p(db_.ptr), C.byref(out.t), start, end,
                                   None), "layer_norm")
     assert_same(out.ref(), want, f"layer norm of {d}")

@@ -103,14 +103,18 @@ NORM = [
     (0, Q8, 256, 64, "k_norm"),  # 5.5, k_norm8 5.9
     (1, F16, 256, 1500, "k_norm"),  # 12.7, k_norm8 13.4
     (0, Q8, 2048, 512, "k_norm8"),
-    (1, F16, 2048, 1500, "k_norm8, grid mean"),  # 29.7, k_norm 93.9
-    (1, Q8, 2304, 64, "k_norm8, grid mean"),  # 8-11, loop 13.5
-    (1, Q8, 2304, 128, "k_norm8, loop mean"),  # 13.6, grid 18-24
-    (1, Q8, 1024, 1500, "k_norm8, grid mean"),  # 15.6, loop 19.4
-    (1, Q8, 1536, 256, "k_norm8, loop mean"),  # 11.7, grid 18-43
-    (1, F16, 2304, 1, "k_norm8, loop mean"),  # 12.3, grid 10-15
+    (1, F16, 2048, 1500, "k_norm8, loop mean"),  # 26.9, grid 29.7, k_norm 92
+    (1, F16, 2048, 16, "k_norm8, loop mean"),  # 11.6, grid 15
+    (1, F16, 2048, 1, "k_norm8, grid mean"),  # 10.7, loop 12
+    (1, Q8, 2048, 64, "k_norm8, grid mean"),  # 10.8 in the mean, loop 12.6, k_norm 14.2
+    (1, Q8, 2048, 128, "k_norm8, loop mean"),  # 13.6, grid 16 in the mean, k_norm 22
+    (1, Q8, 1024, 1500, "k_norm8, grid mean"),  # 16.1, loop 19.4
+    (1, Q8, 2304, 4, "k_norm8, grid mean"),  # 8.2, loop 13.4
+    (1, Q8, 2304, 48, "k_norm8, loop mean"),  # 13.6, grid 8-22
+    (1, Q8, 1536, 64, "k_norm8, grid mean"),  # 8.5, loop 11.6
+    (1, Q8, 1536, 256, "k_norm8, loop mean"),  # 11.7, grid 16 in the mean
     (1, F16, 2304, 256, "k_norm8, loop mean"),  # 13.5, grid 20.8, k_norm 13.9
-    (1, F16, 1280, 1, "k_norm8, grid mean"),  # 7.2-8.9, loop 9.5
+    (1, F16, 1280, 1, "k_norm8, grid mean"),  # 8.7, loop 9.6
     (1, F16, 1024, 256, "k_norm8, loop mean"),  # 9.2, grid 12.0, k_norm 10.1
     (1, F16, 3072, 4, "k_norm8, loop mean"),
 ]
